@@ -111,7 +111,7 @@ constexpr int kFusedDepth = 4;
 // Share of each fused workgroup's suffix windows that its streaming waves take
 // (in 1/256); the stage-1 waves take the rest after their stage-1 unit.
 constexpr int kFusedSplit = 208;
-static_assert(kFusedSplit >= 128 && kFusedSplit < 256, "ChunkMap::none_empty assumes a share in [1/2, 1)");
+static_assert(kFusedSplit >= 128 && kFusedSplit < 256, "ChunkMap assumes a share in [1/2, 1)");
 
 // LDS layout (bytes) of the stream body for G query heads per group and NW waves;
 // TOK (the token-major body) adds the merged results of a phase's segments,
@@ -193,11 +193,26 @@ __device__ __forceinline__ int64_t div_nonneg(int64_t x, int64_t d) {
     return (int64_t)((double)x / (double)d);
 }
 
+// With fewer windows than chunks the first chunks take one window each (split > 0:
+// the first pairs two, one per chunk; an odd last window joins the last pair, and
+// a single window is the first pair's second chunk's), in closed form without a
+// division. So no chunk between two that hold windows is ever empty, and folding a
+// cut sequence's partials tests nothing (ranges spread over all P chunks left
+// empty ones inside a sequence there, and testing them, two chunk bounds per chunk
+// of dependent double divisions, cost the cascade epilogue half of its 13.3 us at 8
+// sequences on a 2048-token prefix).
 struct ChunkMap {
     int64_t W;
     int P;
     int split;
     __device__ __forceinline__ int64_t lo(int c) const {
+        if (W < P) {
+            if (split == 0) return min((int64_t)c, W);
+            const int h = max((int)W >> 1, 1);  // pairs that hold windows
+            if (c >= 2 * h) return W;
+            const int a = c & ~1;
+            return (c & 1) == 0 ? a : a + (((a == 2 * h - 2 ? (int)W - a : 2) * split) >> 8);
+        }
         if (split == 0) return div_nonneg((int64_t)c * W, P);
         const int h = P >> 1, j = c >> 1;
         const int64_t a = div_nonneg((int64_t)j * W, h);
@@ -206,16 +221,16 @@ struct ChunkMap {
     }
     // the chunk that owns window p < W
     __device__ __forceinline__ int owner(int64_t p) const {
-        if (split == 0) return (int)div_nonneg((p + 1) * P - 1, W);
-        const int j = (int)div_nonneg((p + 1) * (P >> 1) - 1, W);
+        int j;
+        if (W < P) {
+            if (split == 0) return (int)p;
+            j = min((int)p >> 1, max((int)W >> 1, 1) - 1);
+        } else {
+            if (split == 0) return (int)div_nonneg((p + 1) * P - 1, W);
+            j = (int)div_nonneg((p + 1) * (P >> 1) - 1, W);
+        }
         return 2 * j + (p >= lo(2 * j + 1) ? 1 : 0);
     }
-    __device__ __forceinline__ bool empty(int c) const { return lo(c) == lo(c + 1); }
-    // No chunk is empty once there are at least as many windows as chunks: equal
-    // chunks then hold >= 1 window each, and each pair's range holds >= 2, of which
-    // a share split / 256 in [1/2, 1) leaves >= 1 to either chunk. (Saves the
-    // divisions of empty(), which dominated the fix-up's and epilogue's time.)
-    __device__ __forceinline__ bool none_empty() const { return W >= P; }
 };
 
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -410,7 +425,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         if (spin == (1 << 22)) count_giveup(&g_wait_giveups);
     }
 
-    const int W = cw[a.batch];
+    const int W = __builtin_amdgcn_readfirstlane(cw[a.batch]);  // scalar: ChunkMap branches on it
     const ChunkMap cm{W, a.chunks, a.split};
     const int w0 = (int)cm.lo(chunk);
     const int w1 = (int)cm.lo(chunk + 1);
@@ -1056,7 +1071,7 @@ static_assert(SfxLds<kMaxGroup, 4, true>::kBytes <= 160 * 1024, "one above");
 
 // Folds the partials of one query head of a sequence cut by chunk boundaries
 // (chunks ca < cb): the tail slot (1) of chunk ca and the head slot (0) of every
-// later chunk that holds windows, weighted by exp(lse - max). Online over batches
+// later chunk, weighted by exp(lse - max). Online over batches
 // of kB chunks whose loads all go out before any is used: one memory round trip
 // per batch, not one per chunk (a long sequence spans many chunks, and the
 // slowest sequence sets the kernel's time).
@@ -1070,28 +1085,23 @@ __device__ __forceinline__ void fold_cut(const float *part_o, const float *part_
     for (int c0 = ca; c0 <= cb; c0 += kB) {
         float pl[kB];
         float4 po[kB];
-        bool ok[kB];
-        // a chunk with no windows wrote nothing (chunk ca holds the sequence's
-        // start); empty chunks exist only below one window per chunk, and their
-        // test runs as a rolled loop off the common path
-        uint32_t okm = cb - c0 + 1 >= kB ? (1u << kB) - 1 : (1u << (cb - c0 + 1)) - 1;
-        if (!cm.none_empty()) {
-#pragma unroll 1
-            for (int j = 0; j < kB; ++j)
-                if (c0 + j <= cb && c0 + j != ca && cm.empty(c0 + j)) okm &= ~(1u << j);
-        }
+        // every chunk from ca to cb holds windows (ChunkMap); past cb, an in-bounds
+        // index, dropped below
 #pragma unroll
         for (int j = 0; j < kB; ++j) {
-            const int ch = min(c0 + j, cb);  // clamped: every load is in bounds
-            ok[j] = (okm >> j) & 1;
-            const int64_t p = pidx(ch, c0 + j == ca ? 1 : 0);
+            const int64_t p = pidx(min(c0 + j, cb), c0 + j == ca ? 1 : 0);
             pl[j] = part_lse[p];
             po[j] = *reinterpret_cast<const float4 *>(part_o + p * kD + 4 * d4);
         }
         float mb = m;
 #pragma unroll
-        for (int j = 0; j < kB; ++j)
-            if (ok[j]) mb = fmaxf(mb, pl[j]);
+        for (int j = 0; j < kB; ++j) {
+            if (c0 + j > cb) {  // weight 0, and 0 * 0 (the clamped partial may be infinite)
+                pl[j] = -INFINITY;
+                po[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            mb = fmaxf(mb, pl[j]);
+        }
         const float mu = mb == -INFINITY ? 0.f : mb;
         const float r = exp2_fast((m - mu) * kLog2e);  // 0 from m = -inf
         acc.x *= r;
@@ -1101,7 +1111,6 @@ __device__ __forceinline__ void fold_cut(const float *part_o, const float *part_
         wsum *= r;
 #pragma unroll
         for (int j = 0; j < kB; ++j) {
-            if (!ok[j]) continue;
             const float wgt = exp2_fast((pl[j] - mu) * kLog2e);
             acc.x = fmaf(wgt, po[j].x, acc.x);
             acc.y = fmaf(wgt, po[j].y, acc.y);
