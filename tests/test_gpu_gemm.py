@@ -312,3 +312,27 @@ def test_rejections_and_abi():
                                          None, None, 1)
     assert abi.lib().ck_f3_gateup_epilogue(a.data_ptr(), a.data_ptr(), None, a.data_ptr(), 16, 128, 128, 6, 128,
                                            None) == -1
+
+
+# The decode-sized kernel (M <= 128, K % 128 == 0): 16-row activation blocks 2 / 4 / 6 /
+# 8 and their edges, 1 to 9 steps of 128 K per K group (rings of 3 and 2 that never
+# fill, wrap and end on every slot), and 4 / 2 / 1 K groups (I <= 4096, <= 8192,
+# above; K must be a multiple of 512 / 256 / 128). M = 129 takes the DMA ring.
+@pytest.mark.parametrize("M,K,I", [
+    (1, 128, 128), (32, 512, 256), (33, 512, 128), (64, 1024, 4096), (64, 1536, 128), (65, 512, 256),
+    (17, 256, 128), (64, 768, 128), (96, 256, 128), (97, 1280, 256), (128, 2304, 128),
+    (33, 1024, 8192), (128, 512, 8192), (32, 256, 8320), (64, 384, 8320), (65, 512, 8320), (96, 640, 8320),
+    (97, 896, 8320), (128, 1152, 8320), (129, 384, 128), (100, 128, 128)])
+@pytest.mark.parametrize("mode", [1, 0])
+def test_decode_sized_tiles(M, K, I, mode):
+    a16, b16 = _inputs(M, K, I, seed=M + K)
+    a, b = bits_to_f32(a16), bits_to_f32(b16)
+    d, ws = torch.ops.npu.f3_gateup_epilogue(torch_bf16(a16, DEV), torch_bf16(b16, DEV), None, None, mode)
+    rows = None if M * K * I <= 1 << 26 else np.unique(np.r_[0, M - 1, np.random.default_rng(K).choice(M, 6)])
+    if mode == 1:
+        _swiglu_check(bf16_to_np(d), a, b, rows)
+    else:
+        c = bf16_to_np(ws)
+        assert np.array_equal(bf16_to_np(d), c[:, :I])
+        rows = np.arange(M) if rows is None else rows
+        _c_check(c[rows], a[rows], b)

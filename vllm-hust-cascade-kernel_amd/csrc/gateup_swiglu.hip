@@ -40,16 +40,16 @@
 //   64 up rows, three 48-KB stages) runs when the full-width grid would leave
 //   CUs idle (a few m-tiles, e.g. M = 256 at I = 14336: 224 workgroups instead
 //   of 112). K = 32 mod 64 runs the same kernel on 32-deep stages (4-stage ring).
-// * Decode-sized kernel (M <= 32, K % 256 == 0): the weight stream bounds the
-//   op, so a workgroup takes 32 gate + 32 up rows (I / 32 workgroups, two per
-//   CU) and its 4 waves each stream a quarter of K from global memory straight
-//   into MFMA operand registers, several 64-deep steps ahead; the partial sums
-//   meet in LDS once. It runs on 16x16x32 MFMA, whose operand layout (four lanes
-//   per row) needs half the address lines per weight byte of the 32x32 one.
+// * Decode-sized kernel (M <= 128, K % 128 == 0): the weight stream bounds the op, so
+//   weights go straight from global memory into MFMA operand registers, several
+//   steps ahead, the activations through LDS, and K is split over wave groups
+//   where the columns alone would leave CUs idle.
 // * General kernel (any K % 16 == 0): 8 waves of 128 x (32 + 32), operands
 //   staged global -> registers -> LDS.
 // * Tiles are ordered M-fastest and XCD-aware so the workgroups sharing a
 //   weight slice run on the same XCD and hit its L2.
+#include <type_traits>
+
 #include "ck_common.h"
 
 namespace ck {
@@ -64,6 +64,18 @@ constexpr int kRowBytes = kBK * 2;                // 128 B per staged row
 constexpr int kTileBytes = (kBM + kBW) * kRowBytes;  // 64 KB per stage
 constexpr int kChunksPerThread = (kBM + kBW) * (kBK / 8) / kThreads;  // 8
 
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for_from(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for_from<I + 1, N>(f);
+    }
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+    static_for_from<0, N>(f);
+}
+
 struct GemmArgs {
     const uint16_t *a;
     const uint16_t *b;
@@ -75,6 +87,7 @@ struct GemmArgs {
     int64_t d_stride;
     int mtiles;
     int ntiles;
+    int mode;  // the decode-sized kernel's C / D windows (modes other than 1)
 };
 
 __device__ __forceinline__ int sw_off(int row, int c) { return row * kRowBytes + ((c ^ (row & 7)) << 4); }
@@ -526,135 +539,193 @@ __global__ __launch_bounds__(kDThreads, 1) void gateup_dma_kernel(GemmArgs p) {
     }
 }
 
-// ---- decode-sized activations (M <= 32) --------------------------------------
+// ---- decode-sized activations (M <= 128) -----------------------------------------
 // With few activation rows the op is bound by the weight stream (2I x K bf16),
-// not by MFMA: the 256-row tile above would run I / 128 workgroups (112 at
-// I = 14336) with half their DMAs fetching padding, and the bytes they keep in
-// flight cap the stream near 2.8 TB/s. Here a workgroup takes 32 gate + 32 up
-// weight rows against all activation rows (I / 32 workgroups, two per CU), and
-// each of its 4 waves streams a quarter of K straight from global memory into
-// MFMA operand registers, several steps ahead; the four partial accumulators
-// meet in LDS once at the end.
-//   On v_mfma_f32_16x16x32_bf16 four lanes share a row (K groups of 8), so a
-//   16-byte-per-lane load covers 16 rows x 64 B: 16 address lines per
-//   instruction, half what the 32x32 layout (two lanes per row) needs per weight
-//   byte. Per 64-deep K step, lane (row r, group q) loads 32 contiguous bytes of
-//   its row, K [64 s + 16 q, +16); MFMA j (of 2) takes the j-th 16 bytes of both
-//   operands, i.e. K {64 s + 16 q + 8 j + t}, the same permutation on both sides,
-//   hence the exact product. Each wave holds 4 weight tiles (gate/up x 2 blocks of
-//   16 rows) per 16-row activation block (NB = 1 up to M = 16, 2 up to M = 32).
-//   Activation rows past M load row M - 1: they feed only output rows that are
-//   not stored.
-constexpr int kSThreads = 256;  // 4 waves, wave w reduces K quarter w
-constexpr int kSN = 32;         // gate rows (and as many up rows) per workgroup
-constexpr int kSStep = 64;      // K per pipeline step
-constexpr int kSDepth = 4;      // steps whose loads are in flight per wave (NB = 1)
-constexpr int kSMaxM = 32;
+// not by MFMA; the 256-row tile above spends most of its LDS and DMAs on padding
+// rows there (M = 64, K = 4096, I = 14336: 59 us, 4.0 TB/s of weights). Here
+// weights go from global memory straight into MFMA operand registers, kMDepth
+// steps of 128 K ahead, and the activations, shared by the waves, through LDS
+// (two buffers, one barrier per step, their loads two steps ahead in registers).
+// * 16x16x32 MFMA: four lanes share a weight row, so a 16-byte-per-lane load covers
+//   16 rows x 64 B. A wave's 16-row weight tile holds 8 gate and 8 up rows in the
+//   order g g u u, so a lane's accumulator has two gate columns and their two up
+//   columns of one activation row: SwiGLU in registers, and the result tile goes
+//   out through LDS in whole row pieces.
+// * NR waves side by side take 8 NR gate (and up) columns; KS such groups each take
+//   a K slice with activation buffers of their own, their sums meet in LDS.
+// * Workgroups start at different K steps and wrap around. Operand rows are a
+//   power of two apart at the usual K, so workgroups in step with each other ask
+//   a few L2 and memory channels for everything (28 workgroups of an XCD, the
+//   same 256 bytes of 64 activation rows): M = 64 at the size above 57 us from
+//   the same step, 70 / 50 us with the start at 1 x / 5 x blockIdx (4 distinct
+//   starts per XCD), 47.0 us with 3 (blockIdx / 8) + blockIdx % 8, which spreads
+//   the workgroups of every XCD (blockIdx % 8) over all steps.
+// * Depth: 2 / 3 / 4 steps of weights 54 / 50 / 51 us (same start); non-temporal
+//   weight loads 59.
+// Against the kernel with a K quarter per wave and no LDS copy of the activations
+// that ran up to M = 32: M = 1 41.0 -> 40.7 us, M = 16 45.7 -> 41.8, M = 32
+// 52.6 -> 42.4 us, M = 64 59.9 -> 46.4; K = 8192, I = 3584: M = 1 35.1 -> 25.0 us.
+constexpr int kMStep = 128;  // K per step
+constexpr int kMDepth = 3;   // steps of weights in flight per wave
+constexpr int kMMaxM = 128;
 
-template <int MODE, int NB>  // NB = 16-row activation blocks (M <= 16 NB)
-__global__ __launch_bounds__(kSThreads) void gateup_skinny16_kernel(GemmArgs p) {
+template <int NB, int NR, int KS>  // NB = 16-row activation blocks (M <= 16 NB)
+struct MidTile {
+    static constexpr int kThr = NR * 64;                         // threads of a K group
+    static constexpr int kNX = 4 * NB / NR;                      // activation chunks per thread and step
+    static constexpr int kRows = 16 * NB;
+    static constexpr int kCols = 8 * NR;                         // gate (and up) columns per workgroup
+    static constexpr int kBuf = kRows * kMStep * 2;              // one activation buffer of a K group
+    static constexpr int kPitch = kCols * 2 + 8;                 // bytes per staged output row
+    static constexpr int kLds = 2 * KS * kBuf;
+    static_assert(kNX * NR == 4 * NB, "the group's threads split the activation rows evenly");
+    static_assert((KS - 1) * kThr * NB * 16 <= kLds && 2 * kRows * kPitch <= kLds, "the sums and output tiles fit");
+    static_assert(kLds <= 160 * 1024, "LDS");
+};
+
+template <bool SWIGLU, int NB, int NR, int KS>
+__global__ __launch_bounds__(KS * NR * 64) __attribute__((amdgpu_waves_per_eu(2))) void gateup_mid_kernel(GemmArgs p) {
     typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
-    // [wave][weight tile: gate b0, gate b1, up b0, up b1][activation block][register][lane]
-    __shared__ float red[4][4][NB][4][64];
-    const int tid = threadIdx.x;
-    const int wid = tid >> 6;
+    using T = MidTile<NB, NR, KS>;
+    constexpr int D = kMDepth;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tid = threadIdx.x % T::kThr;  // within the K group
+    const int grp = wid / NR, wr = wid % NR;
     const int lane = tid & 63;
     const int r16 = lane & 15;
     const int q4 = lane >> 4;
-    const int64_t n0 = (int64_t)blockIdx.x * kSN;
-    const int64_t kq = p.k / 4;
-    const int steps = (int)(kq / kSStep);
-    const int64_t koff = wid * kq + 16 * q4;
-    const uint4 *wp[4];  // gate rows n0 + 16 b + r16, up rows n_half + n0 + 16 b + r16
+    const int64_t n0 = (int64_t)blockIdx.x * T::kCols;
+    const int steps = (int)(p.k / (kMStep * KS));  // of this K group
+    const int64_t k0 = (int64_t)grp * steps * kMStep;
+    const int rot = (int)((3 * (blockIdx.x >> 3) + (blockIdx.x & 7) + grp) % (unsigned)steps);
+    // tile row r16: up if bit 1 is set, column 8 wr + 2 (r16 / 4) + r16 % 2
+    const uint16_t *wp =
+        p.b + (((r16 & 2) ? p.n_half : 0) + n0 + 8 * wr + 2 * (r16 >> 2) + (r16 & 1)) * p.k + k0 + 8 * q4;
+    // activations: thread -> chunk tid % 16 of rows tid / 16 + 4 NR u, at chunk ^ (row % 16)
+    const int xr = tid >> 4, xc = tid & 15;
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(p.a), (short)0, (int)(p.m * p.k * 2), 0x00020000);
+    int xo[T::kNX];  // byte offsets; a row past m lies out of range: zeros, no bytes moved
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-        wp[t] = reinterpret_cast<const uint4 *>(p.b + ((t < 2 ? 0 : p.n_half) + n0 + 16 * (t & 1) + r16) * p.k + koff);
-    const uint4 *xp[NB];
-#pragma unroll
-    for (int ab = 0; ab < NB; ++ab) {
-        const int64_t arow = 16 * ab + r16 < p.m ? 16 * ab + r16 : p.m - 1;
-        xp[ab] = reinterpret_cast<const uint4 *>(p.a + arow * p.k + koff);
+    for (int u = 0; u < T::kNX; ++u) {
+        const int r = xr + 4 * NR * u;
+        xo[u] = r < p.m ? (int)((r * p.k + xc * 8) * 2) : (int)0x80000000;
     }
-    constexpr int kStepVec = kSStep * 2 / 16;  // uint4 per row per step (8)
-    constexpr int kDepth = NB == 1 ? kSDepth : 3;  // registers: 48 per step at NB = 2
+    char *const xbuf = smem + grp * 2 * T::kBuf;
+    const char *xsrc[4];  // fragment f: 16-byte chunk 4 f + q4 of row r16
+#pragma unroll
+    for (int f = 0; f < 4; ++f) xsrc[f] = xbuf + r16 * (kMStep * 2) + (((4 * f + q4) ^ r16) << 4);
 
-    uint4 W[kDepth][4][2], X[kDepth][NB][2];
-    f32x4_t acc[4][NB];
+    u32x4 W[D][4], X[2][T::kNX];
+    f32x4_t acc[NB];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int ab = 0; ab < NB; ++ab) acc[ab] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // a step past the last loads the weights' first line in every lane, and no activations
+    // (nothing reads those registers; repeating the last step there cost 2% at M = 1)
+    auto kstep = [&](int st) __attribute__((always_inline)) {
+        const int x = st + rot;
+        return (int64_t)(x < steps ? x : x - steps) * kMStep;
+    };
+    auto load_w = [&](int slot, int st) __attribute__((always_inline)) {
+        const uint16_t *w = st < steps ? wp + kstep(st) : p.b;
 #pragma unroll
-        for (int ab = 0; ab < NB; ++ab)
+        for (int f = 0; f < 4; ++f) W[slot][f] = *reinterpret_cast<const u32x4 *>(w + 32 * f);
+    };
+    auto load_x = [&](int slot, int st) __attribute__((always_inline)) {
+        const int o = (int)(k0 + kstep(st)) * 2, past = st < steps ? 0 : (int)0x80000000;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[t][ab][e] = 0.f;
-#define CK_SKINNY16_LOAD(slot, st)                                          \
-    do {                                                                    \
-        const int64_t o_ = (int64_t)(st) * kStepVec;                        \
-        _Pragma("unroll") for (int j_ = 0; j_ < 2; ++j_) {                  \
-            _Pragma("unroll") for (int t_ = 0; t_ < 4; ++t_) W[slot][t_][j_] = wp[t_][o_ + j_]; \
-            _Pragma("unroll") for (int b_ = 0; b_ < NB; ++b_) X[slot][b_][j_] = xp[b_][o_ + j_]; \
-        }                                                                   \
-    } while (0)
+        for (int u = 0; u < T::kNX; ++u)
+            X[slot][u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, xo[u] | past, o, 0));
+    };
+    auto store_x = [&](int slot, int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int d = 0; d < kDepth; ++d)
-        if (d < steps) CK_SKINNY16_LOAD(d, d);
-    for (int s = 0; s < steps; s += kDepth) {
+        for (int u = 0; u < T::kNX; ++u) {
+            const int r = xr + 4 * NR * u;
+            *reinterpret_cast<u32x4 *>(xbuf + buf * T::kBuf + r * (kMStep * 2) + ((xc ^ (r & 15)) << 4)) = X[slot][u];
+        }
+    };
+    // step st in ring slots st % D (weights) and st % 2 (activations): the barrier
+    // puts X(st) in its buffer and frees the other, which takes X(st + 1)
+    auto step = [&](auto jc, int st) __attribute__((always_inline)) {
+        constexpr int d = decltype(jc)::value % D, h = decltype(jc)::value & 1;
+        __syncthreads();
+        store_x(h ^ 1, h ^ 1);
+        load_x(h ^ 1, st + 3);
 #pragma unroll
-        for (int d = 0; d < kDepth; ++d) {
-            if (s + d < steps) {
+        for (int f = 0; f < 4; ++f)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+            for (int ab = 0; ab < NB; ++ab)
+                acc[ab] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    __builtin_bit_cast(bf16x8, W[d][f]),
+                    *reinterpret_cast<const bf16x8 *>(xsrc[f] + h * T::kBuf + ab * (16 * kMStep * 2)), acc[ab], 0, 0, 0);
+        load_w(d, st + D);
+    };
+    load_x(0, 0);
+    load_x(1, 1);
 #pragma unroll
-                    for (int ab = 0; ab < NB; ++ab) {
-                        const bf16x8 xf = __builtin_bit_cast(bf16x8, X[d][ab][j]);
+    for (int d = 0; d < D; ++d) load_w(d, d);
+    store_x(0, 0);
+    load_x(0, 2);
+    constexpr int kRound = D % 2 ? 2 * D : D;  // steps after which both rings are back at slot 0
+    int st = 0;
+    for (; st + kRound <= steps; st += kRound)
+        static_for<kRound>([&](auto jc) __attribute__((always_inline)) { step(jc, st + decltype(jc)::value); });
+    const int rem = steps - st;
+    static_for<kRound - 1>([&](auto jc) __attribute__((always_inline)) {
+        if (decltype(jc)::value < rem) step(jc, st + decltype(jc)::value);
+    });
+    __syncthreads();  // every wave is done with the activation buffers
+
+    // ---- the K groups' sums meet in the first group -----------------------------------
+    if constexpr (KS > 1) {
+        f32x4_t *const red = reinterpret_cast<f32x4_t *>(smem);
+        if (grp > 0) {
 #pragma unroll
-                        for (int t = 0; t < 4; ++t)
-                            acc[t][ab] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                __builtin_bit_cast(bf16x8, W[d][t][j]), xf, acc[t][ab], 0, 0, 0);
-                    }
-                if (s + d + kDepth < steps) CK_SKINNY16_LOAD(d, s + d + kDepth);
+            for (int ab = 0; ab < NB; ++ab) red[((grp - 1) * NB + ab) * T::kThr + tid] = acc[ab];
+        }
+        __syncthreads();
+        if (grp == 0) {
+#pragma unroll
+            for (int o = 0; o < KS - 1; ++o)
+#pragma unroll
+                for (int ab = 0; ab < NB; ++ab) acc[ab] += red[(o * NB + ab) * T::kThr + tid];
+        }
+        __syncthreads();
+    }
+    // ---- epilogue: lane (q4, r16) holds columns 8 wr + 2 q4 + {0, 1} of activation row
+    // 16 ab + r16 (registers 0, 1 gate; 2, 3 up) ------------------------------------
+    char *const tg = smem, *const tu = smem + T::kRows * T::kPitch;
+    if (grp == 0) {
+#pragma unroll
+        for (int ab = 0; ab < NB; ++ab) {
+            const int o = (16 * ab + r16) * T::kPitch + (8 * wr + 2 * q4) * 2;
+            const f32x4_t v = acc[ab];
+            if constexpr (SWIGLU) {
+                *reinterpret_cast<uint32_t *>(tg + o) = pack_bf16x2(silu_mul(v[0], v[2]), silu_mul(v[1], v[3]));
+            } else {
+                *reinterpret_cast<uint32_t *>(tg + o) = pack_bf16x2(v[0], v[1]);
+                *reinterpret_cast<uint32_t *>(tu + o) = pack_bf16x2(v[2], v[3]);
             }
         }
     }
-#undef CK_SKINNY16_LOAD
-
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int ab = 0; ab < NB; ++ab)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) red[wid][t][ab][e][lane] = acc[t][ab][e];
     __syncthreads();
-    // thread -> (weight tile pair b: gate b and up b, activation block ab, accumulator
-    // lane l): output row 16 ab + l % 16, columns n0 + 16 b + 4 (l / 16) + 0..3
-    if (tid >= 2 * NB * 64) return;
-    const int b = tid / (NB * 64);
-    const int ab = (tid / 64) % NB;
-    const int l = tid & 63;
-    const int64_t gm = 16 * ab + (l & 15);
-    if (gm >= p.m) return;
-    float g[4], u[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        g[i] = red[0][b][ab][i][l] + red[1][b][ab][i][l] + red[2][b][ab][i][l] + red[3][b][ab][i][l];
-        u[i] = red[0][2 + b][ab][i][l] + red[1][2 + b][ab][i][l] + red[2][2 + b][ab][i][l] + red[3][2 + b][ab][i][l];
-    }
-    const int64_t col = n0 + 16 * b + 4 * (l >> 4);
-    if (MODE == 1) {
-        *reinterpret_cast<uint2 *>(p.d + gm * p.d_stride + col) =
-            make_uint2(pack_bf16x2(silu_mul(g[0], u[0]), silu_mul(g[1], u[1])),
-                       pack_bf16x2(silu_mul(g[2], u[2]), silu_mul(g[3], u[3])));
-    } else {
-        const uint2 gv = make_uint2(pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3]));
-        const uint2 uv = make_uint2(pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]));
-        uint16_t *crow = p.c + gm * (2 * p.n_half);
-        *reinterpret_cast<uint2 *>(crow + col) = gv;
-        *reinterpret_cast<uint2 *>(crow + p.n_half + col) = uv;
-        if (MODE == 0 || MODE == 5)
-            *reinterpret_cast<uint2 *>(p.d + gm * p.d_stride + col) = gv;
-        else if (MODE == 4)
-            *reinterpret_cast<uint2 *>(p.d + gm * p.d_stride + col) = uv;
-        else if (MODE == 8)
-            *reinterpret_cast<uint2 *>(p.d + gm * p.d_stride + col) = make_uint2(0, 0);
+    constexpr int kPc = T::kCols / 4;  // 8-byte pieces of an output row
+    const int c8 = threadIdx.x % kPc;
+    for (int r = threadIdx.x / kPc; r < p.m; r += KS * T::kThr / kPc) {
+        const uint2 gv = *reinterpret_cast<const uint2 *>(tg + r * T::kPitch + c8 * 8);
+        uint16_t *const drow = p.d + r * p.d_stride + n0 + c8 * 4;
+        if constexpr (SWIGLU) {
+            *reinterpret_cast<uint2 *>(drow) = gv;
+        } else {
+            const uint2 uv = *reinterpret_cast<const uint2 *>(tu + r * T::kPitch + c8 * 8);
+            uint16_t *const crow = p.c + (int64_t)r * (2 * p.n_half) + n0 + c8 * 4;
+            *reinterpret_cast<uint2 *>(crow) = gv;
+            *reinterpret_cast<uint2 *>(crow + p.n_half) = uv;
+            if (p.mode == 0 || p.mode == 5) *reinterpret_cast<uint2 *>(drow) = gv;
+            else if (p.mode == 4) *reinterpret_cast<uint2 *>(drow) = uv;
+            else if (p.mode == 8) *reinterpret_cast<uint2 *>(drow) = make_uint2(0, 0);
+        }
     }
 }
 
@@ -692,16 +763,47 @@ int launch_dma(GemmArgs p, hipStream_t s) {
     CK_RETURN_LAUNCH();
 }
 
+template <bool SWIGLU, int NB, int NR, int KS>
+int launch_mid_tile(const GemmArgs &p, hipStream_t s) {
+    using T = MidTile<NB, NR, KS>;
+    static std::atomic<uint64_t> lds_set{0};
+    int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(&gateup_mid_kernel<SWIGLU, NB, NR, KS>), T::kLds, lds_set);
+    if (rc != CK_OK) return rc;
+    hipLaunchKernelGGL((gateup_mid_kernel<SWIGLU, NB, NR, KS>), dim3((unsigned)(p.n_half / T::kCols)),
+                       dim3(KS * T::kThr), T::kLds, s, p);
+    CK_RETURN_LAUNCH();
+}
+
+// A workgroup's time hardly depends on its columns (it is the latency of its K
+// steps: 39 / 25 / 20 us for K = 4096 over 1 / 2 / 4 K groups at M = 64 and up to
+// one workgroup per CU), so K is split as far as all workgroups still run at
+// once. M = 64, K = 4096, 4 / 2 / 1 groups: I = 3584 21.7 / 27.0 / 40.1 us,
+// I = 7168 40.7 / 30.9 / 41.3, I = 10240 58.8 / 54.4 / 43.2. Above 64 rows four
+// groups' activation buffers do not fit the LDS.
+template <int MODE>
+int launch_mid(GemmArgs p, hipStream_t s) {
+    constexpr bool kSw = MODE == 1;
+    p.mode = MODE;
+    if (p.n_half <= 16 * kNumCus && p.m <= 64 && p.k % (4 * kMStep) == 0)
+        return p.m <= 32 ? launch_mid_tile<kSw, 2, 2, 4>(p, s) : launch_mid_tile<kSw, 4, 2, 4>(p, s);
+    if (p.n_half <= 32 * kNumCus && p.k % (2 * kMStep) == 0)
+        return p.m <= 32   ? launch_mid_tile<kSw, 2, 4, 2>(p, s)
+               : p.m <= 64 ? launch_mid_tile<kSw, 4, 4, 2>(p, s)
+                           : launch_mid_tile<kSw, 8, 4, 2>(p, s);
+    return p.m <= 32   ? launch_mid_tile<kSw, 2, 8, 1>(p, s)
+           : p.m <= 64 ? launch_mid_tile<kSw, 4, 8, 1>(p, s)
+           : p.m <= 96 ? launch_mid_tile<kSw, 6, 8, 1>(p, s)
+                       : launch_mid_tile<kSw, 8, 8, 1>(p, s);
+}
+
 template <int MODE>
 int launch_gemm(const GemmArgs &p, hipStream_t s) {
-    if (p.m <= kSMaxM && p.k % (4 * kSStep) == 0) {
-        if (p.m <= 16)
-            hipLaunchKernelGGL((gateup_skinny16_kernel<MODE, 1>), dim3((unsigned)(p.n_half / kSN)), dim3(kSThreads),
-                               0, s, p);
-        else
-            hipLaunchKernelGGL((gateup_skinny16_kernel<MODE, 2>), dim3((unsigned)(p.n_half / kSN)), dim3(kSThreads),
-                               0, s, p);
-        CK_RETURN_LAUNCH();
+    if (p.m <= kMMaxM && p.k % kMStep == 0 && p.k <= kMaxDmaK) {
+        // above 96 rows the activations' share of the L2 and LDS traffic costs what the
+        // padding rows of the 256-row tile do: ahead only in one round of workgroups
+        // (M = 128, K = 8192, I = 28672: 218 us against 208; K = 4096, I = 14336: 57.2
+        // against 58.3)
+        if (p.m <= 96 || p.n_half <= 64 * kNumCus) return launch_mid<MODE>(p, s);
     }
     const int64_t grid = (int64_t)p.mtiles * p.ntiles;
     if (p.k % 32 == 0 && p.k <= kMaxDmaK) {
