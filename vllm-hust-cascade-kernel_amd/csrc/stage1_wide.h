@@ -60,7 +60,7 @@ constexpr int kTBytes = kTTok * kD * 2;              // 16 KB of K (or V) per ti
 // of them. Each 64-token K/V tile in LDS feeds 256 rows (twice the MFMA work
 // per DMA byte and per barrier of the 128-row kernel), and while one wave of a
 // SIMD waits on a fragment read, a DMA issue or its softmax, the other issues
-// MFMAs. Per tile: QK (16 MFMAs, K fragments read four ahead), softmax with
+// MFMAs. Per tile: QK (16 MFMAs, K fragments read six ahead), softmax with
 // the running max moved once per tile, PV (16 MFMAs, V^T fragments read one
 // 16-token group ahead). A 4-slot ring of K+V tiles, three tiles of DMA lead.
 // The body is shared with the fused cascade kernel, where 4 waves run it (128
@@ -221,21 +221,28 @@ __device__ __forceinline__ void stage1_wide_body(const Stage1Args &a, CK_LDS cha
         slot = slot == SLOTS - 1 ? 0 : slot + 1;
         if (!wave_active) continue;
 
-        // S^T of the two 32-token blocks, K fragments read four ahead
+        // S^T of the two 32-token blocks, K fragments read six ahead. The fences hold
+        // that order: without them the compiler reads each pair of fragments right
+        // before its MFMAs and waits out the LDS round trip eight times per tile
+        // (64 queries on 8192 tokens 23.0 -> 22.3 us, 256 x 64 heads on 32768 384 -> 378;
+        // four or eight ahead measure the same).
         f32x16 sb[2];
         {
             const f32x16 zero16 = {};
             auto kfrag = [&](int f) {
                 return *reinterpret_cast<const CK_LDS bf16x8 *>(kb + tile_off(32 * (f & 1) + ktok, 2 * (f >> 1) + hh));
             };
-            bf16x8 kfr[4];
+            constexpr int kAhead = 6;
+            bf16x8 kfr[kAhead];
 #pragma unroll
-            for (int f = 0; f < 4; ++f) kfr[f] = kfrag(f);
+            for (int f = 0; f < kAhead; ++f) kfr[f] = kfrag(f);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int f = 0; f < 16; ++f) {
-                sb[f & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr[f & 3], qf[f >> 1], f < 2 ? zero16 : sb[f & 1],
+                sb[f & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr[f % kAhead], qf[f >> 1], f < 2 ? zero16 : sb[f & 1],
                                                                     0, 0, 0);
-                if (f + 4 < 16) kfr[f & 3] = kfrag(f + 4);
+                if (f + kAhead < 16) kfr[f % kAhead] = kfrag(f + kAhead);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         if (nv < kTTok) {
