@@ -115,6 +115,9 @@ int ck_lse_merge(const void *o1, int o1_dtype, const void *o2, int o2_dtype,
  * P = exp(S - rowmax) is rounded to bf16 (RNE) before the PV product and the
  * row sums use the unrounded fp32 values, as
  * third_party/catlass/.../block_epilogue_online_softmax_no_mask.hpp:487-594 does.
+ * With one query token per request (q_len_uniform == 1), kv_cap >= 1024, the
+ * plan's split count and its workspace, the requests are streamed as
+ * ck_suffix_decode does, with P at fp32 precision.
  * Replaces OPS/fa_fp32_stage1/op_kernel/kernel_fa_fp32_stage1.cpp:848-863.
  * ========================================================================== */
 int ck_fa_fp32_stage1_plan(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_heads,
@@ -266,7 +269,8 @@ int ck_add_rms_norm_stats(const void *x1, const void *x2, const void *gamma, con
 
 /* ============================================================================
  * Health counter of the bounded waits inside the suffix and fused cascade
- * kernels (ck_suffix_decode, ck_cascade_decode, ck_cascade_decode_noalloc).
+ * kernels (ck_suffix_decode, ck_cascade_decode, ck_cascade_decode_noalloc, and
+ * ck_fa_fp32_stage1 with one query token per request).
  * Their waves wait on each other only through LDS counters whose waits are
  * bounded (a hang is never possible); a wait that runs out means a broken
  * invariant and wrong results, and is counted on the device. *count receives

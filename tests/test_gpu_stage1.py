@@ -351,3 +351,47 @@ def test_negative_checks():
         torch.ops.npu.fa_fp32_stage1(q, k, v, bt, qs, kvs, 2)               # T != 2B
     o, l = torch.ops.npu.fa_fp32_stage1(q[:0], k, v, bt, qs[:0], kvs[:0])
     assert o.shape == (0, 40, 128) and l.shape == (0,)
+
+
+# One query token per request from a kv bound of 1024 on: the requests are streamed as
+# suffix windows. Ragged lengths (one token, a page edge, the bound itself), few and
+# many requests per chunk, 1 to 8 and (two groups) 12 query heads per kv head.
+DECODE = [("b1_kv1024", [1024], 8, 8), ("b1_kv20000", [20000], 8, 1), ("b3_edges", [1, 1024, 897], 40, 8),
+          ("b5_h64", [1500, 31, 32, 33, 2047], 64, 8), ("b4_gqa12", [1100, 640, 64, 1], 48, 4),
+          ("b70_h10", [1 + (37 * i) % 1400 for i in range(70)], 10, 2)]
+
+
+@pytest.mark.parametrize("case", DECODE, ids=[c[0] for c in DECODE])
+def test_decode_form(case):
+    from cascade_amd import abi
+    name, kvs, H, KVH = case
+    B = len(kvs)
+    inp = paged_inputs(B, kvs, H, KVH, seed=17, q_len=1, permute=True, block_cols=max(8, (max(kvs) + 127) // 128))
+    out, lse = _run(inp, 1)
+    # P enters as two bf16 terms within 2^-16 of fp32 P, so O is within 2^-16 max|V| (about
+    # 8e-5) of exact attention plus the fp32 sums' rounding. (The bf16-P oracle itself is
+    # up to 2^-9 max|V| from exact on the shortest requests.)
+    o_ref, l_ref = A.stage1(inp["q"], inp["k"], inp["v"], inp["block_table"], np.ones(B, dtype=np.int64),
+                            inp["kv_seqlens"], quantize_p=False)
+    assert np.abs(out - o_ref).max() <= 2.0 ** -16 * np.abs(inp["v"]).max() + 2e-5
+    l8 = lse.reshape(-1, 8)
+    assert (l8 == l8[:, :1]).all()
+    assert np.abs(l8[:, 0].reshape(B, H) - l_ref).max() <= 1e-4
+    out2, lse2 = _run(inp, 0)  # lengths through the host: the same bits
+    assert np.array_equal(out.view(np.uint32), out2.view(np.uint32))
+    assert np.array_equal(lse.view(np.uint32), lse2.view(np.uint32))
+    # a split count of the caller's runs the tiles, within the same bound
+    q, k, v, bt, qs, kl = _dev(inp)
+    cap = bt.shape[1] * 128
+    splits, ws_bytes = abi.stage1_plan(B, 1, H, KVH, 128, cap)
+    forced = splits + 1 if splits + 1 <= bt.shape[1] else max(1, splits - 1)
+    need = max(ws_bytes, forced * B * H * 129 * 4)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    o3 = torch.empty(B, H, 128, dtype=torch.float32, device=DEV)
+    l3 = torch.empty(B * H * 8, dtype=torch.float32, device=DEV)
+    abi.check(abi.lib().ck_fa_fp32_stage1(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), bt.data_ptr(), bt.shape[1], qs.data_ptr(), kl.data_ptr(), None, B, 1,
+        1, B, H, KVH, 128, k.shape[0], 128, float(np.float32(1 / np.sqrt(128))), cap, forced, o3.data_ptr(),
+        l3.data_ptr(), ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
+    assert abi.wait_giveups() == 0
+    _check(inp, o3.cpu().numpy(), l3.cpu().numpy(), H, name + " tiles")

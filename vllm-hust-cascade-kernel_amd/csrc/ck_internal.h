@@ -38,7 +38,7 @@ int stage1_fused_args(const void *q, const void *k, const void *v, const int32_t
 // suffix_decode.hip: sequences per launch of the suffix stream kernel, its
 // chunk count and the workspace one launch group needs.
 int64_t suffix_group_batch(int64_t kv_cap);
-int64_t suffix_default_chunks(int64_t num_heads, int64_t kv_heads);
+int64_t suffix_default_chunks(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap);
 int64_t suffix_group_ws_bytes(int64_t nb, int64_t num_heads, int64_t kv_heads, int64_t chunks);
 
 // Stage-1 result the cascade epilogue folds in, for query token b (row b * H + h).
@@ -60,11 +60,13 @@ int64_t suffix_fused_chunks(int64_t num_heads, int64_t kv_heads);
 // result of every sequence of the group to final_out/final_lse. With `fused`
 // (stage-1 arguments from stage1_fused_args, fused_units units) one fused
 // kernel runs the stage-1 units and the suffix chunks side by side instead.
+// With f32_out (stage-1's decode form, no stage-1 result) out/lse receive fp32
+// rows and 8 copies of each LSE.
 int suffix_launch_group(const void *q, const void *k, const void *v, const int32_t *block_table, int64_t bt_cols,
                         const int64_t *kv_seqlens, int64_t b0, int64_t nb, int64_t num_heads, int64_t kv_heads,
                         int64_t num_blocks, int64_t kv_layout, float scale, int64_t kv_cap, int64_t chunks,
                         void *out, float *lse, void *group_ws, const Stage1Result *cascade, void *final_out,
                         float *final_lse, hipStream_t stream, const s1::Stage1Args *fused = nullptr,
-                        int64_t fused_units = 0);
+                        int64_t fused_units = 0, bool f32_out = false);
 
 }  // namespace ck

@@ -55,6 +55,7 @@
 //   (O, LSE) pairs are folded by an N-way LSE merge (stage1_combine_kernel).
 // * Block order is XCD-aware: the m-tiles that read the same kv pages are
 //   placed on the same XCD so the later reads hit that XCD's L2.
+#include <algorithm>
 #include <cmath>
 
 #include "ck_common.h"
@@ -186,6 +187,25 @@ int make_plan(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_he
     return CK_OK;
 }
 
+// Decode form (one query token per request): a request has H / KVH query rows per
+// kv head of the 128-row tile, so one of its 4 waves computes, in a chain of
+// 64-token tiles, and every tile's MFMAs run for mostly padding. The suffix
+// kernels stream the same pages instead (16-column MFMA tiles, all requests'
+// windows balanced over the chip), with P at fp32 precision: 40 / 8 heads, 7 requests
+// of 1024-4096 tokens 28.4 -> 22.5 us, of 4096-16384 97 -> 58, 24 of 4096 95 -> 75.
+// From a kv bound of 1024: below, the tiles' chain is short and the fix-up kernel
+// costs more than it saves (24 requests of 512: 16.6 us tiles, 18.8 streamed; of
+// 1024 33.4 and 26.0). A kv bound of one 128-token page, where the reference's
+// rounding of P is checked, stays on the tiles.
+constexpr int64_t kDecodeMinCap = 1024;
+bool decode_form(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_heads, int64_t kv_cap) {
+    return max_q_len == 1 && batch > 0 && kv_cap >= kDecodeMinCap && num_heads <= (1 << 16) &&
+           batch <= suffix_group_batch(kv_cap);
+}
+int64_t decode_ws_bytes(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap) {
+    return suffix_group_ws_bytes(batch, num_heads, kv_heads, suffix_default_chunks(batch, num_heads, kv_heads, kv_cap));
+}
+
 int check_dims(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_heads, int64_t head_dim,
                int64_t kv_cap) {
     if (batch < 0 || max_q_len < 0 || kv_cap < 0) return CK_E_INVALID_ARG;
@@ -211,6 +231,8 @@ extern "C" int ck_fa_fp32_stage1_plan(int64_t batch, int64_t max_q_len, int64_t 
     make_plan(batch, max_q_len, num_heads, kv_heads, kv_cap, 0, &p);
     *num_splits = p.splits;
     *workspace_bytes = p.ws_bytes;
+    if (decode_form(batch, max_q_len, num_heads, kv_heads, kv_cap))
+        *workspace_bytes = std::max(p.ws_bytes, decode_ws_bytes(batch, num_heads, kv_heads, kv_cap));
     return CK_OK;
 }
 
@@ -240,7 +262,16 @@ int ck::stage1_launch(const void *q, const void *k, const void *v, const int32_t
     if (num_tokens * num_heads > ((int64_t)1 << 31)) return CK_E_INVALID_ARG;
 
     Plan p;
-    make_plan(batch, max_q_len, num_heads, kv_heads, kv_cap, num_splits, &p);
+    make_plan(batch, max_q_len, num_heads, kv_heads, kv_cap, 0, &p);
+    // the decode form with the plan's split count and workspace; a caller's own split
+    // count, or a workspace sized for the splits alone, runs the tiles
+    if (combine && q_len_uniform == 1 && decode_form(batch, max_q_len, num_heads, kv_heads, kv_cap) &&
+        (num_splits <= 0 || num_splits == p.splits) && workspace != nullptr &&
+        workspace_bytes >= decode_ws_bytes(batch, num_heads, kv_heads, kv_cap))
+        return suffix_launch_group(q, k, v, block_table, bt_cols, kv_seqlens, 0, batch, num_heads, kv_heads,
+                                   num_blocks, CK_KV_NHD, scale, kv_cap,
+                                   suffix_default_chunks(batch, num_heads, kv_heads, kv_cap), out, lse, workspace, nullptr, nullptr, nullptr, s, nullptr, 0, true);
+    if (num_splits > 0) make_plan(batch, max_q_len, num_heads, kv_heads, kv_cap, num_splits, &p);
     if (splits_used) *splits_used = p.splits;
     const int64_t need = p.splits > 1 ? p.splits * num_tokens * num_heads * (kD + 1) * (int64_t)sizeof(float) : 0;
     if (need > 0 && (workspace == nullptr || workspace_bytes < need)) return CK_E_WORKSPACE;

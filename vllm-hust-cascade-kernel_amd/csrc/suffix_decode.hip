@@ -66,6 +66,8 @@
 // * A segment that is a whole sequence writes bf16 O and the LSE directly; a
 //   sequence cut by a chunk boundary leaves fp32 partials that a small fix-up
 //   kernel folds (it also writes O = 0, LSE = -inf for empty suffixes).
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "ck_common.h"
@@ -104,8 +106,7 @@ constexpr int kRsrcFlags = 0x00020000;  // buffer descriptor word 3 for gfx9 raw
 
 // windows of loads in flight per streaming wave: token-major, 2 (24 registers
 // per window and lane; 3 and 4 measured slower in the fused kernel), 1 in the
-// stand-alone kernel above 4 heads (one workgroup per CU there: 1 measured
-// faster than 2 and 3); dims-major (the fused kernel above 4 heads), 4.
+// stand-alone kernel above 4 heads (1 measured faster than 2 and 3); dims-major (the fused kernel above 4 heads), 4.
 constexpr int kTokDepth = 2;
 constexpr int kFusedDepth = 4;
 // Share of each fused workgroup's suffix windows that its streaming waves take
@@ -302,6 +303,13 @@ __device__ __forceinline__ int64_t clamp_len(const SuffixArgs &a, int64_t kvl) {
     return kvl < 0 ? 0 : kvl;
 }
 
+// The result row of stage-1's decode form: fp32 O and 8 copies of the LSE (a.out
+// and a.lse then hold fp32 rows and padded LSEs).
+__device__ __forceinline__ void write_f32_row(const SuffixArgs &a, int64_t row, int d4, f32x4 o, float lse_v) {
+    *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(a.out) + row * kD + 4 * d4) = o;
+    if (d4 < 2) *reinterpret_cast<f32x4 *>(a.lse + row * 8 + 4 * d4) = f32x4{lse_v, lse_v, lse_v, lse_v};
+}
+
 // The stream body on NW waves (thread tid of the group's NW * 64) as workgroup lb
 // of a grid of a.kv_heads * a.chunks, with the group's LDS at smem and its own
 // barrier. Windows hold 8 NW tokens.
@@ -337,7 +345,7 @@ __device__ __forceinline__ int64_t clamp_len(const SuffixArgs &a, int64_t kvl) {
 // body's LDS) skips its own, waits until scan_flag is set and reads the other's
 // lengths and window prefix sums; the body given only scan_flag sets it once its
 // scan is complete.
-template <int G, int NW, int D, bool TOK, class Bar>
+template <int G, int NW, int D, bool TOK, bool F32 = false, class Bar>
 __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS char *smem, int lb, int tid,
                                                    const Bar &bar, CK_LDS int *scan_flag = nullptr,
                                                    const CK_LDS char *scan_src = nullptr) {
@@ -554,9 +562,13 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         const bool tail_part = cw[b + 1] > w1;
         if (!head_part && !tail_part) {
             const int64_t row = (int64_t)b * a.num_heads + g * G + h;
-            *reinterpret_cast<uint2 *>(a.out + row * kD + 4 * d4) =
-                make_uint2(pack_bf16x2(on[0], on[1]), pack_bf16x2(on[2], on[3]));
-            if (d4 == 0) a.lse[row] = lse_v;
+            if constexpr (F32) {
+                write_f32_row(a, row, d4, on, lse_v);
+            } else {
+                *reinterpret_cast<uint2 *>(a.out + row * kD + 4 * d4) =
+                    make_uint2(pack_bf16x2(on[0], on[1]), pack_bf16x2(on[2], on[3]));
+                if (d4 == 0) a.lse[row] = lse_v;
+            }
         } else {
             const int64_t pidx = (((int64_t)g * a.chunks + chunk) * 2 + (head_part ? 0 : 1)) * G + h;
             // non-temporal: read once, by the fix-up or cascade epilogue kernel
@@ -1057,16 +1069,15 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
 
 // The stand-alone stream kernel: the token-major body on the matrix cores (the
 // fused kernel's streaming body) on 4 waves and at most 256 registers; two
-// workgroups per CU up to 4 query heads per group (64 KB of LDS each), one above
-// (103 KB at 8 heads: the grid's second half runs as the first half's
-// workgroups finish; a 4-segment layout that fits two per CU measured no faster).
-template <int G>
+// workgroups fit a CU up to 5 query heads per group (64 KB of LDS each at 4, 74 KB at
+// 5), one above (103 KB at 8 heads).
+template <int G, bool F32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void suffix_stream_kernel(SuffixArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    suffix_stream_body<G, 4, (G > 4 ? 1 : kTokDepth), true>(a, (CK_LDS char *)smem_raw, blockIdx.x, threadIdx.x,
+    suffix_stream_body<G, 4, (G > 4 ? 1 : kTokDepth), true, F32>(a, (CK_LDS char *)smem_raw, blockIdx.x, threadIdx.x,
                                                            WgBarrier{});
 }
-static_assert(SfxLds<4, 4, true>::kBytes <= 80 * 1024, "two stand-alone workgroups per CU up to 4 heads");
+static_assert(SfxLds<5, 4, true>::kBytes <= 80 * 1024, "two stand-alone workgroups per CU up to 5 heads");
 static_assert(SfxLds<kMaxGroup, 4, true>::kBytes <= 160 * 1024, "one above");
 
 // Folds the partials of one query head of a sequence cut by chunk boundaries
@@ -1130,7 +1141,7 @@ __device__ __forceinline__ void fold_cut(const float *part_o, const float *part_
 // folded; others return. The window prefix sums and the grid arithmetic come as
 // leading scalar parameters (preloaded into SGPRs at wave launch, as for the
 // cascade epilogue), so the first load waits for no kernel-argument load.
-template <int G>
+template <int G, bool F32>
 __global__ __launch_bounds__(kMaxGroup * 32) void suffix_fixup_kernel(const int32_t *cw, int kv_heads, int batch,
                                                                       SuffixArgs a) {
     const int b = blockIdx.x / kv_heads;
@@ -1140,8 +1151,12 @@ __global__ __launch_bounds__(kMaxGroup * 32) void suffix_fixup_kernel(const int3
     const int64_t beg = cw[b], end = cw[b + 1], W = cw[batch];
     const int64_t row = (int64_t)b * a.num_heads + g * G + hq;
     if (end == beg) {
-        *reinterpret_cast<uint2 *>(a.out + row * kD + 4 * d4) = make_uint2(0, 0);
-        if (d4 == 0) a.lse[row] = -INFINITY;
+        if constexpr (F32) {
+            write_f32_row(a, row, d4, f32x4{0.f, 0.f, 0.f, 0.f}, -INFINITY);
+        } else {
+            *reinterpret_cast<uint2 *>(a.out + row * kD + 4 * d4) = make_uint2(0, 0);
+            if (d4 == 0) a.lse[row] = -INFINITY;
+        }
         return;
     }
     const ChunkMap cm{W, a.chunks, a.split};
@@ -1151,9 +1166,13 @@ __global__ __launch_bounds__(kMaxGroup * 32) void suffix_fixup_kernel(const int3
     float4 o;
     float l;
     fold_cut<G>(a.part_o, a.part_lse, g, cm, hq, d4, ca, cb, o, l);
-    *reinterpret_cast<uint2 *>(a.out + row * kD + 4 * d4) =
-        make_uint2(pack_bf16x2(o.x, o.y), pack_bf16x2(o.z, o.w));
-    if (d4 == 0) a.lse[row] = l;
+    if constexpr (F32) {
+        write_f32_row(a, row, d4, f32x4{o.x, o.y, o.z, o.w}, l);
+    } else {
+        *reinterpret_cast<uint2 *>(a.out + row * kD + 4 * d4) =
+            make_uint2(pack_bf16x2(o.x, o.y), pack_bf16x2(o.z, o.w));
+        if (d4 == 0) a.lse[row] = l;
+    }
 }
 
 // Cascade epilogue (fused cascade decode): one workgroup of 32 G threads per
@@ -1389,17 +1408,17 @@ int launch_fused(const s1::Stage1Args &s1a, int64_t n1, const SuffixArgs &a, con
     CK_RETURN_LAUNCH();
 }
 
-template <int G>
+template <int G, bool F32 = false>
 int launch_suffix(const SuffixArgs &a, bool fixup, const EpilogueArgs *epi, hipStream_t st) {
     static std::atomic<uint64_t> lds_set{0};
     constexpr int kLds = SfxLds<G, 4, true>::kBytes;
-    int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(&suffix_stream_kernel<G>), kLds, lds_set);
+    int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(&suffix_stream_kernel<G, F32>), kLds, lds_set);
     if (rc != CK_OK) return rc;
-    hipLaunchKernelGGL(suffix_stream_kernel<G>, dim3((unsigned)(a.kv_heads * a.chunks)), dim3(256), kLds, st, a);
+    hipLaunchKernelGGL((suffix_stream_kernel<G, F32>), dim3((unsigned)(a.kv_heads * a.chunks)), dim3(256), kLds, st, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return static_cast<int>(e);
     if (fixup)
-        hipLaunchKernelGGL(suffix_fixup_kernel<G>, dim3((unsigned)(a.batch * a.kv_heads)), dim3(32 * G), 0, st,
+        hipLaunchKernelGGL((suffix_fixup_kernel<G, F32>), dim3((unsigned)(a.batch * a.kv_heads)), dim3(32 * G), 0, st,
                            (const int32_t *)a.cw_out, a.kv_heads, a.batch, a);
     if (epi) launch_epilogue<G>(*epi, (unsigned)(a.batch * a.kv_heads), st);
     CK_RETURN_LAUNCH();
@@ -1436,12 +1455,27 @@ int64_t suffix_group_batch(int64_t kv_cap) {
     return n < 1 ? 1 : n;
 }
 
-// Workgroups per kv head group: two resident workgroups per CU (16 waves of at
-// most 128 registers, under 80 KB of LDS each), so the grid holds 512
-// workgroups over all kv head groups and starts at once.
-int64_t suffix_default_chunks(int64_t num_heads, int64_t kv_heads) {
+// Chunks of the window list (workgroups) per kv head group: a grid that is resident
+// at once over all groups, one or two workgroups per CU, and no more chunks per
+// sequence than folding their partials is worth.
+// * One per CU above 5 query heads per group: two do not fit its LDS
+//   (suffix_stream_kernel), and a second generation pays the start-up again
+//   (64 / 8 heads, 64 suffixes of mean 512: 42.5 us with 512 workgroups, 36.3 with
+//   256; 256 suffixes 115 / 109; 4 of mean 64 27.7 / 10.8).
+// * Up to 5 heads, one per CU for long sequences, at most two per chunk: half the
+//   partials and start-ups (40 / 8 heads, 24 requests of 4096: 80.8 / 74.3 us; 7
+//   31.4 / 29.9; 32 / 8 heads, 64 suffixes of mean 512 36.9 / 37.0, of mean 1024
+//   57.1 / 55.3). Two per CU otherwise: with many short sequences per chunk the
+//   closes bound it (256 suffixes of mean 64: 25.4 / 30.7).
+// * A sequence of n windows spans chunks / batch chunks; its fold takes a memory
+//   round trip per 8 (about 0.15 us a chunk) and a chunk's windows about 0.5 us
+//   each: sqrt(cap / 8) chunks per sequence balance the two (8 / 1 heads, 7 requests
+//   of 4096: 26.2 us over 512 chunks, 13.8 over 112, 15.6 over 56).
+int64_t suffix_default_chunks(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap) {
     const int64_t groups = kv_heads * suffix_sub_groups(num_heads, kv_heads);
-    const int64_t p = 512 / groups;
+    const bool one = num_heads > 5 * groups || (kv_cap >= 1024 && batch <= 2 * 256 / groups);
+    const int64_t per_seq = std::max<int64_t>(8, (int64_t)std::sqrt((double)kv_cap / 8));
+    const int64_t p = std::min((one ? 256 : 512) / groups, batch * per_seq);
     return p > 0 ? p : 1;
 }
 
@@ -1460,7 +1494,8 @@ int suffix_launch_group(const void *q, const void *k, const void *v, const int32
                         const int64_t *kv_seqlens, int64_t b0, int64_t nb, int64_t num_heads, int64_t kv_heads,
                         int64_t num_blocks, int64_t kv_layout, float scale, int64_t kv_cap, int64_t chunks,
                         void *out, float *lse, void *group_ws, const Stage1Result *cascade, void *final_out,
-                        float *final_lse, hipStream_t stream, const s1::Stage1Args *fused, int64_t fused_units) {
+                        float *final_lse, hipStream_t stream, const s1::Stage1Args *fused, int64_t fused_units,
+                        bool f32_out) {
     const int64_t sub = suffix_sub_groups(num_heads, kv_heads);
     const int64_t G = num_heads / kv_heads / sub;  // query heads per workgroup
     const int64_t parts = group_parts(num_heads, chunks);
@@ -1517,6 +1552,18 @@ int suffix_launch_group(const void *q, const void *k, const void *v, const int32
             default: return launch_fused<8>(*fused, fused_units, a, e, stream);
         }
     }
+    if (f32_out) {  // stage-1's decode form
+        switch (G) {
+            case 1: return launch_suffix<1, true>(a, true, nullptr, stream);
+            case 2: return launch_suffix<2, true>(a, true, nullptr, stream);
+            case 3: return launch_suffix<3, true>(a, true, nullptr, stream);
+            case 4: return launch_suffix<4, true>(a, true, nullptr, stream);
+            case 5: return launch_suffix<5, true>(a, true, nullptr, stream);
+            case 6: return launch_suffix<6, true>(a, true, nullptr, stream);
+            case 7: return launch_suffix<7, true>(a, true, nullptr, stream);
+            default: return launch_suffix<8, true>(a, true, nullptr, stream);
+        }
+    }
     const bool fixup = cascade == nullptr;
     const EpilogueArgs *ep = cascade ? &e : nullptr;
     switch (G) {
@@ -1540,7 +1587,7 @@ extern "C" int ck_suffix_decode_plan(int64_t batch, int64_t num_heads, int64_t k
     int rc = check_suffix_dims(batch, num_heads, kv_heads, head_dim, kv_cap);
     if (rc != CK_OK) return rc;
     if (!num_splits || !workspace_bytes) return CK_E_NULL_PTR;
-    const int64_t chunks = suffix_default_chunks(num_heads, kv_heads);
+    const int64_t chunks = suffix_default_chunks(batch, num_heads, kv_heads, kv_cap);
     const int64_t nb = batch < suffix_group_batch(kv_cap) ? batch : suffix_group_batch(kv_cap);
     *num_splits = chunks;
     *workspace_bytes = batch > 0 ? suffix_group_ws_bytes(nb, num_heads, kv_heads, chunks) : 0;
@@ -1564,7 +1611,7 @@ extern "C" int ck_suffix_decode(const void *q, const void *k, const void *v, con
     if (!aligned_to(q, 16) || !aligned_to(k, 16) || !aligned_to(v, 16) || !aligned_to(out, 8) ||
         !aligned_to(lse, 4) || !aligned_to(workspace, 16))
         return CK_E_INVALID_ARG;
-    const int64_t chunks = num_splits > 0 ? num_splits : suffix_default_chunks(num_heads, kv_heads);
+    const int64_t chunks = num_splits > 0 ? num_splits : suffix_default_chunks(batch, num_heads, kv_heads, kv_cap);
     if (kv_heads * suffix_sub_groups(num_heads, kv_heads) * chunks > 0x7FFFFFFF || chunks > (1 << 20))
         return CK_E_INVALID_ARG;
     const int64_t per_launch = suffix_group_batch(kv_cap);
