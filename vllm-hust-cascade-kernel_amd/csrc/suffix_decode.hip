@@ -120,23 +120,24 @@ static_assert(kFusedSplit >= 128 && kFusedSplit < 256, "ChunkMap assumes a share
 // 8 token rows of 256 bytes at a 288-byte pitch (the pitch puts the 4 rows of a
 // transpose read in distinct bank groups).
 constexpr int kVtPitch = 288;
-template <int G, int NW, bool TOK = false>
+template <int G, int NW, bool TOK = false, int SEGS = kQSlots, int RING = (TOK || G <= 4 ? 2 : 1)>
 struct SfxLds {
+    static constexpr int kSegs = SEGS;                                   // segments per phase
     static constexpr int kCw = 0;                                        // int cw[kMaxBatch + 1]
     static constexpr int kLen = ((kMaxBatch + 1) * 4 + 15) / 16 * 16;   // int len[kMaxBatch]
     static constexpr int kWtot = kLen + kMaxBatch * 4;                   // int wtot[NW]
     static constexpr int kTab = kWtot + 64;               // int pair tab[kTable + 8] (8 padding entries)
     static constexpr int kPw = kTab + (kTable + 8) * 8;  // float pw[NW][8][8] p rows (dims-major)
-    static constexpr int kQs = kPw + NW * 8 * 8 * 4;                     // bf16 q[kQSlots][G][kD]
-    static constexpr int kX = TOK || G <= 4 ? 2 : 1;                     // exchange ring slots
-    static constexpr int kXo = kQs + kQSlots * G * kD * 2;               // float xo[kX][NW][G][kD]
+    static constexpr int kQs = kPw + NW * 8 * 8 * 4;                     // bf16 q[kSegs][G][kD]
+    static constexpr int kX = RING;                                      // exchange ring slots
+    static constexpr int kXo = kQs + kSegs * G * kD * 2;               // float xo[kX][NW][G][kD]
     static constexpr int kXml = kXo + kX * NW * G * kD * 4;              // float xml[kX][NW][G][2]
     static constexpr int kXsync = kXml + kX * NW * G * 2 * 4;            // int cnt[kX], gen[kX]
     static constexpr int kBar = kXsync + 2 * kX * 4;                     // int bar[2] (group barrier)
-    static constexpr int kSo = (kBar + 8 + 15) / 16 * 16;                // float so[kQSlots][G][kD] (TOK)
-    static constexpr int kSl = kSo + (TOK ? kQSlots * G * kD * 4 : 0);   // float sl[kQSlots][G]
-    static constexpr int kSb = kSl + (TOK ? kQSlots * G * 4 : 0);        // int sb[kQSlots]
-    static constexpr int kVt = (kSb + (TOK ? kQSlots * 4 : 0) + 15) / 16 * 16;  // char vt[NW][8][kVtPitch] (TOK)
+    static constexpr int kSo = (kBar + 8 + 15) / 16 * 16;                // float so[kSegs][G][kD] (TOK)
+    static constexpr int kSl = kSo + (TOK ? kSegs * G * kD * 4 : 0);   // float sl[kSegs][G]
+    static constexpr int kSb = kSl + (TOK ? kSegs * G * 4 : 0);        // int sb[kSegs]
+    static constexpr int kVt = (kSb + (TOK ? kSegs * 4 : 0) + 15) / 16 * 16;  // char vt[NW][8][kVtPitch] (TOK)
     static constexpr int kBytes = kVt + (TOK ? NW * 8 * kVtPitch : 0);
     static_assert(kTab % 16 == 0 && kPw % 16 == 0 && kQs % 16 == 0 && kXo % 16 == 0 && kXml % 8 == 0 &&
                       kSo % 16 == 0,
@@ -345,7 +346,7 @@ __device__ __forceinline__ void write_f32_row(const SuffixArgs &a, int64_t row, 
 // body's LDS) skips its own, waits until scan_flag is set and reads the other's
 // lengths and window prefix sums; the body given only scan_flag sets it once its
 // scan is complete.
-template <int G, int NW, int D, bool TOK, bool F32 = false, class Bar>
+template <int G, int NW, int D, bool TOK, bool F32 = false, class L = SfxLds<G, NW, TOK>, class Bar>
 __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS char *smem, int lb, int tid,
                                                    const Bar &bar, CK_LDS int *scan_flag = nullptr,
                                                    const CK_LDS char *scan_src = nullptr) {
@@ -355,7 +356,6 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     constexpr int kThr = NW * 64;
     constexpr int kWin = 8 * NW;         // tokens per window
     constexpr int kWpp = kPage / kWin;   // windows per page
-    using L = SfxLds<G, NW, TOK>;
     CK_LDS int *cw = (CK_LDS int *)((scan_src ? scan_src : smem) + L::kCw);
     CK_LDS int *len = (CK_LDS int *)((scan_src ? scan_src : smem) + L::kLen);
     CK_LDS int *wtot = (CK_LDS int *)(smem + L::kWtot);
@@ -618,7 +618,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     // close k - 2, the slot's previous use. Each step of a close costs an LDS round
     // trip, slow while the stage-1 waves keep the LDS busy, so the close has few.
     auto merge_share = [&](int k, int b, int e) __attribute__((always_inline)) {
-        static_assert(!TOK || R == 2, "the slot reuse argument above takes two slots");
+        static_assert(!TOK || R <= 2, "the slot reuse argument above takes two slots");
         const int r = k % R;
         const int target = NW * (k / R + 1);
         {
@@ -632,6 +632,10 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         static_assert(!TOK || (kPer * NW == 32 * G && kPer <= 64), "pairs split evenly over the waves");
         if (lane < kPer) merge_pair(wid * kPer + lane, r, b, e);
         if (wid == 0 && lane == 0) sb[e] = b;
+        if constexpr (TOK && R == 1) {  // this wave's reads of the slot are done (LDS operations run in order)
+            asm volatile("" ::: "memory");
+            if (lane == 0) __hip_atomic_fetch_add(xgen, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
     };
 
     // Token-major: the state of a new segment, set at the start and by every close
@@ -675,6 +679,14 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
             for (; *(volatile CK_LDS int *)(xgen + r) != want && spin < (1 << 22); ++spin)
                 __builtin_amdgcn_s_sleep(1);
             if (spin == (1 << 22)) count_giveup(&g_wait_giveups);
+        }
+        if constexpr (TOK && R == 1) {
+            // one slot: every wave's share of the previous close's merge is done
+            // (each has arrived there, so each finishes it; bounded)
+            int spin = 0;
+            for (; *(volatile CK_LDS int *)xgen < NW * nclose && spin < (1 << 22); ++spin) __builtin_amdgcn_s_sleep(1);
+            if (spin == (1 << 22)) count_giveup(&g_wait_giveups);
+            asm volatile("" ::: "memory");
         }
         CK_LDS float *xo_r = xo + r * NW * G * kD;
         CK_LDS float *xml_r = xml + r * NW * G * 2;
@@ -956,9 +968,9 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         const int bc = min(bq0 + lane, a.batch - 1);
         const int c_lo = cw[bc], c_hi = cw[bc + 1], c_len = len[bc];
         uint64_t segm = __builtin_amdgcn_ballot_w64(bq0 + lane < a.batch && c_hi > c_lo && c_lo < w1);
-        int segb[kQSlots], seg_lo[kQSlots], seg_hi[kQSlots], seg_len[kQSlots];
+        int segb[L::kSegs], seg_lo[L::kSegs], seg_hi[L::kSegs], seg_len[L::kSegs];
 #pragma unroll
-        for (int sg = 0; sg < kQSlots; ++sg) {
+        for (int sg = 0; sg < L::kSegs; ++sg) {
             seg_lo[sg] = 0x7FFFFFFF;  // never selected below
             segb[sg] = seg_hi[sg] = seg_len[sg] = 0;
             if (segm != 0) {
@@ -988,7 +1000,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
             const int wg = w0 + p0 + i;
             int b = segb[0], lo_b = seg_lo[0], hi_b = seg_hi[0], len_b = seg_len[0];
 #pragma unroll
-            for (int sg = 1; sg < kQSlots; ++sg) {
+            for (int sg = 1; sg < L::kSegs; ++sg) {
                 if (seg_lo[sg] <= wg) {  // the last segment starting at or before window wg
                     b = segb[sg];
                     lo_b = seg_lo[sg];
@@ -1336,7 +1348,7 @@ __global__ __launch_bounds__(kMaxGroup * 32) void cascade_epilogue_kernel(const 
 // for the other.
 constexpr int kFusedS1Lds = s1::wide_lds_bytes<3>();
 template <int G>
-using FusedSfx = SfxLds<G, 4, (G <= 4)>;  // the stream body's layout on 4 waves (token-major up to 4 heads)
+using FusedSfx = SfxLds<G, 4, true, (G <= 4 ? kQSlots : 4), (G <= 4 ? 2 : 1)>;  // the stream body's layout on 4 waves
 template <int G>
 constexpr int fused_lds_bytes() { return kFusedS1Lds + FusedSfx<G>::kBytes + 32; }
 static_assert(fused_lds_bytes<4>() <= 160 * 1024 && fused_lds_bytes<kMaxGroup>() <= 160 * 1024,
@@ -1374,7 +1386,7 @@ __global__ __launch_bounds__(512) void cascade_fused_kernel(s1::Stage1Args s1a, 
         constexpr int kRoleRot = 3;
         const int g = ((int)blockIdx.x + kRoleRot) % sa.kv_heads, j = (int)blockIdx.x / sa.kv_heads;
         // the streaming waves scan the lengths; the stage-1 waves reuse that scan
-        suffix_stream_body<G, 4, (G <= 4 ? kTokDepth : kFusedDepth), (G <= 4)>(
+        suffix_stream_body<G, 4, kTokDepth, true, false, FusedSfx<G>>(
             sa, smem + (role ? 0 : kFusedS1Lds), (2 * j + role) * sa.kv_heads + g, threadIdx.x & 255, bar, bars + 4,
             role ? smem + kFusedS1Lds : nullptr);
     }
