@@ -423,3 +423,28 @@ def test_suffix_bnsd_layout_against_oracle(case):
     abi.check(rc)
     torch.cuda.synchronize()
     _check_suffix(inp, bf16_to_np(out), lse.cpu().numpy(), H)
+
+
+# The fused kernel above 4 query heads per group: 4 segments per phase and one exchange
+# slot, so chunks of many short sequences run several phases and close back to back;
+# kv head groups of 5, 7, 8 and (two groups) 6 heads, row counts that fill no 128-row unit.
+@pytest.mark.parametrize("B,H,KVH,P", [(130, 64, 8, 384), (90, 40, 8, 1536), (33, 7, 1, 5120), (20, 48, 4, 896)])
+def test_fused_above_4_heads(B, H, KVH, P, no_wait_giveups):
+    rng = np.random.default_rng(B)
+    suf = rng.integers(0, 90, size=B)
+    suf[::max(1, B // 7)] = rng.integers(100, 1500, size=suf[::max(1, B // 7)].shape)
+    q16, k16, v16, bt_pre, bt_suf, suf = _cascade_inputs(B, H, KVH, P, suf, seed=B)
+    q, k, v = (torch_bf16(x, DEV) for x in (q16, k16, v16))
+    got, lse = _cascade_run(True, B, P, q, k, v, bt_pre, bt_suf, suf)
+    again, lse2 = _cascade_run(True, B, P, q, k, v, bt_pre, bt_suf, suf)
+    assert np.array_equal(got, again) and np.array_equal(lse, lse2)
+    qf, kf, vf = bits_to_f32(q16), bits_to_f32(k16), bits_to_f32(v16)
+    kp, vp = A.gather_kv(kf, vf, bt_pre[0], P)
+    for b in np.unique(np.r_[np.argsort(suf)[[0, 1, -2, -1]], rng.choice(B, 8)]):
+        ks, vs = A.gather_kv(kf, vf, bt_suf[b], int(suf[b]))
+        kc, vc = np.concatenate([kp, ks]), np.concatenate([vp, vs])
+        Od, Ld = A.dense(qf[b:b + 1], A.expand_heads(kc, H), A.expand_heads(vc, H))
+        err = np.abs(got[b:b + 1] - Od)
+        assert np.all(err <= 2e-3 + 2.0 ** -8 * np.abs(Od)), (b, err.max())
+        rel = np.abs(lse.reshape(B, H)[b] - Ld[0]) / np.maximum(np.abs(Ld[0]), 1.0)
+        assert rel.max() <= 1e-4, (b, rel.max())

@@ -24,7 +24,7 @@ int stage1_launch(const void *q, const void *k, const void *v, const int32_t *bl
 
 // fa_stage1.hip: the stage-1 role of the fused cascade kernel (suffix_decode.hip)
 // for B decode queries flattened into one request: 128-row units over splits of
-// the prefix, about `target` units. stage1_fused_plan sizes it (units, splits,
+// the prefix, at most `target` units where the rows allow. stage1_fused_plan sizes it (units, splits,
 // workspace bytes for the partials); stage1_fused_args validates the operands
 // and fills the kernel arguments (with one split, out/lse receive the result).
 void stage1_fused_plan(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap, int64_t target,

@@ -1,7 +1,6 @@
 // suffix_decode.hip - per-sequence paged decode attention over each sequence's
 // own suffix pages (cascade stage 2) on gfx950: the stand-alone op and the
-// fused cascade's streaming waves compute their windows on the matrix cores
-// (the fused kernel above 4 query heads per group on the vector ALU).
+// fused cascade's streaming waves compute their windows on the matrix cores.
 //
 // Role: replaces the closed CANN op npu_fused_infer_attention_score_v2 the
 // reference calls for stage 2 (ascend-kernel/README.md:186-197): one query
@@ -38,29 +37,26 @@
 //   address is a fixed offset; rows past the sequence's end fall outside the
 //   range (zeros, no bytes moved), and an invalid page id gets an empty range:
 //   its rows read as zeros, the semantics of the pool's unmapped pages.
-// * Token-major body (the stand-alone kernel, the fused kernel up to 4 heads):
-//   scores S^T = K q^T and values O^T += V^T P^T on 16x16 bf16 MFMAs, V^T
+// * Scores S^T = K q^T and values O^T += V^T P^T on 16x16 bf16 MFMAs, V^T
 //   through a per-wave LDS slot read back transposed (suffix_stream_body gives
-//   the lane layouts). Dims-major body (the fused kernel above 4 heads): 8
-//   packed bf16 dot products and a DPP sum per score, p through a per-wave LDS
-//   row, 4 value FMAs per token and head. Either way the running max moves only
-//   when a score exceeds it by more than 2^kTau (a wave-uniform branch), so
-//   rescaling is rare; any reference point gives the same O and LSE.
+//   the lane layouts). The running max moves only when a score exceeds it by more
+//   than 2^kTau (a wave-uniform branch), so rescaling is rare; any reference point
+//   gives the same O and LSE.
 // * Closing a sequence never stops the stream: each wave writes its partial
 //   (O, m, l) into the segment's slot of an LDS exchange ring and counts itself
-//   in with an LDS atomic. Token-major: once all partials are in, each wave
-//   merges its share into an LDS stash (one wave doing the whole merge fell
-//   behind the others by it at every close), written out after the phase's
-//   loop. Dims-major: the last wave in merges and writes the result while the
-//   others go on. A wave waits for a ring slot only if it runs a whole ring
-//   ahead of the slowest wave, which itself never waits, so every wait ends.
+//   in with an LDS atomic. Once all partials are in, each wave merges its share
+//   into an LDS stash (one wave doing the whole merge fell behind the others by
+//   it at every close), written out after the phase's loop. A wave waits only for
+//   arrivals (with one exchange slot, also for shares) of a close that every wave
+//   reaches without waiting for it, so every wait ends.
 // * Cascade (stage 1 + suffix + merge): one fused kernel, one workgroup per CU.
 //   Waves 0-3 run the stage-1 body (MFMA, LDS tiles: matrix cores and LDS),
 //   waves 4-7 stream suffix windows; each role synchronises only its own four
 //   waves through an LDS counter barrier, so the two run side by side instead
 //   of one kernel after the other, and a small epilogue kernel merges the two
 //   results.
-// * The range is processed in phases of at most 512 windows and 8 segments.
+// * The range is processed in phases of at most 512 windows and 8 segments (4 in
+//   the fused kernel above 4 heads, where 8 do not fit beside the stage-1 tiles).
 //   A phase starts with one round trip that fills the window table and copies
 //   the q rows of its segments into LDS; the phase's loop has no barrier.
 // * A segment that is a whole sequence writes bf16 O and the LSE directly; a
@@ -104,42 +100,44 @@ constexpr float kTau = 8.0f;        // log2 headroom before the running max move
 constexpr uint32_t kOob = 0x80000000u;  // a buffer offset past every window's range
 constexpr int kRsrcFlags = 0x00020000;  // buffer descriptor word 3 for gfx9 raw loads
 
-// windows of loads in flight per streaming wave: token-major, 2 (24 registers
-// per window and lane; 3 and 4 measured slower in the fused kernel), 1 in the
-// stand-alone kernel above 4 heads (1 measured faster than 2 and 3); dims-major (the fused kernel above 4 heads), 4.
+// windows of loads in flight per streaming wave: 2 (24 registers per window and
+// lane; 3 and 4 measured slower in the fused kernel), 1 in the stand-alone kernel
+// above 4 heads (1 measured faster than 2 and 3).
 constexpr int kTokDepth = 2;
-constexpr int kFusedDepth = 4;
 // Share of each fused workgroup's suffix windows that its streaming waves take
-// (in 1/256); the stage-1 waves take the rest after their stage-1 unit.
-constexpr int kFusedSplit = 208;
-static_assert(kFusedSplit >= 128 && kFusedSplit < 256, "ChunkMap assumes a share in [1/2, 1)");
+// (in 1/256); the stage-1 waves take the rest after their stage-1 unit. A batch has
+// more stage-1 rows per suffix byte the more heads share a kv head, so the share
+// is larger above 4 heads per group: 64 / 40 heads on 8192 tokens 53.7 us at 208,
+// 52.6 at 224; 47 / 64 on 6037 42.3, 41.5; 100 / 8 on 8000 30.0, 28.4; 110 / 64 on
+// 2000 44.2, 45.0. 64 / 32 on 8192: 51.3, 51.1 (the same within the runs).
+constexpr int fused_split(int64_t group) { return group > 4 ? 224 : 208; }
+static_assert(fused_split(8) >= 128 && fused_split(8) < 256 && fused_split(4) >= 128, "ChunkMap assumes a share in [1/2, 1)");
 
 // LDS layout (bytes) of the stream body for G query heads per group and NW waves;
-// TOK (the token-major body) adds the merged results of a phase's segments,
-// held until the phase's window loop is done, and each wave's V transpose slot:
+// SEGS segments per phase and RING exchange slots. The merged results of a phase's
+// segments are held until its window loop is done; each wave's V transpose slot is
 // 8 token rows of 256 bytes at a 288-byte pitch (the pitch puts the 4 rows of a
 // transpose read in distinct bank groups).
 constexpr int kVtPitch = 288;
-template <int G, int NW, bool TOK = false, int SEGS = kQSlots, int RING = (TOK || G <= 4 ? 2 : 1)>
+template <int G, int NW, int SEGS = kQSlots, int RING = 2>
 struct SfxLds {
     static constexpr int kSegs = SEGS;                                   // segments per phase
     static constexpr int kCw = 0;                                        // int cw[kMaxBatch + 1]
     static constexpr int kLen = ((kMaxBatch + 1) * 4 + 15) / 16 * 16;   // int len[kMaxBatch]
     static constexpr int kWtot = kLen + kMaxBatch * 4;                   // int wtot[NW]
     static constexpr int kTab = kWtot + 64;               // int pair tab[kTable + 8] (8 padding entries)
-    static constexpr int kPw = kTab + (kTable + 8) * 8;  // float pw[NW][8][8] p rows (dims-major)
-    static constexpr int kQs = kPw + NW * 8 * 8 * 4;                     // bf16 q[kSegs][G][kD]
+    static constexpr int kQs = kTab + (kTable + 8) * 8;                  // bf16 q[kSegs][G][kD]
     static constexpr int kX = RING;                                      // exchange ring slots
     static constexpr int kXo = kQs + kSegs * G * kD * 2;               // float xo[kX][NW][G][kD]
     static constexpr int kXml = kXo + kX * NW * G * kD * 4;              // float xml[kX][NW][G][2]
     static constexpr int kXsync = kXml + kX * NW * G * 2 * 4;            // int cnt[kX], gen[kX]
     static constexpr int kBar = kXsync + 2 * kX * 4;                     // int bar[2] (group barrier)
-    static constexpr int kSo = (kBar + 8 + 15) / 16 * 16;                // float so[kSegs][G][kD] (TOK)
-    static constexpr int kSl = kSo + (TOK ? kSegs * G * kD * 4 : 0);   // float sl[kSegs][G]
-    static constexpr int kSb = kSl + (TOK ? kSegs * G * 4 : 0);        // int sb[kSegs]
-    static constexpr int kVt = (kSb + (TOK ? kSegs * 4 : 0) + 15) / 16 * 16;  // char vt[NW][8][kVtPitch] (TOK)
-    static constexpr int kBytes = kVt + (TOK ? NW * 8 * kVtPitch : 0);
-    static_assert(kTab % 16 == 0 && kPw % 16 == 0 && kQs % 16 == 0 && kXo % 16 == 0 && kXml % 8 == 0 &&
+    static constexpr int kSo = (kBar + 8 + 15) / 16 * 16;                // float so[kSegs][G][kD]
+    static constexpr int kSl = kSo + kSegs * G * kD * 4;                // float sl[kSegs][G]
+    static constexpr int kSb = kSl + kSegs * G * 4;                     // int sb[kSegs]
+    static constexpr int kVt = (kSb + kSegs * 4 + 15) / 16 * 16;        // char vt[NW][8][kVtPitch]
+    static constexpr int kBytes = kVt + NW * 8 * kVtPitch;
+    static_assert(kTab % 16 == 0 && kQs % 16 == 0 && kXo % 16 == 0 && kXml % 8 == 0 &&
                       kSo % 16 == 0,
                   "aligned LDS rows");
 };
@@ -235,14 +233,8 @@ struct ChunkMap {
     }
 };
 
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-
-// Every control used below (quad_perm, row_half_mirror, row_ror) reads a lane of
-// the same 16-lane row, so bound_ctrl never applies; setting it lets the
-// compiler fold the move into the consuming add (v_add_f32_dpp).
-#define CK_DPP(x, ctrl) __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), ctrl, 0xF, 0xF, true))
 
 // x[l] op x[l ^ 16] and x[l] op x[l ^ 32] through v_permlane16_swap /
 // v_permlane32_swap: swapping x with itself leaves x[l] in one result and the
@@ -258,42 +250,6 @@ __device__ __forceinline__ float sum_xor16(float x) {
 __device__ __forceinline__ float sum_xor32(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// Sum over each aligned group of 8 lanes; every lane of the group gets the total.
-__device__ __forceinline__ float sum8(float x) {
-    x += CK_DPP(x, 0xB1);   // quad_perm [1,0,3,2]
-    x += CK_DPP(x, 0x4E);   // quad_perm [2,3,0,1]
-    x += CK_DPP(x, 0x141);  // row_half_mirror: the other quad of the 8
-    return x;
-}
-// Sum / max over the 8 lanes l, l^8, l^16, ..., l^56 (the token slots of a wave).
-__device__ __forceinline__ float sum_slots(float x) {
-    x += CK_DPP(x, 0x128);  // row_ror:8: the other 8 of the 16-lane row
-    return sum_xor32(sum_xor16(x));
-}
-__device__ __forceinline__ float max_slots(float x) {
-    x = fmaxf(x, CK_DPP(x, 0x128));
-    return max_xor32(max_xor16(x));
-}
-
-__device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c,
-                                           false);
-}
-// 16-dim bf16 dot product: one chain of 8 (the callers interleave one chain per
-// query head, which covers the chain's latency; two chains per head cost a
-// second zero-initialised accumulator and an add)
-__device__ __forceinline__ float dot16(const u32x4 &k0, const u32x4 &k1, const u32x4 &q0, const u32x4 &q1) {
-    // the chain's first product takes its zero as an inline constant (the
-    // compiler materialises the zero in a register for the tied-accumulator form)
-    float d;
-    asm("v_dot2_f32_bf16 %0, %1, %2, 0" : "=v"(d) : "v"(k0[0]), "v"(q0[0]));
-#pragma unroll
-    for (int i = 1; i < 4; ++i) d = dot2(k0[i], q0[i], d);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) d = dot2(k1[i], q1[i], d);
-    return d;
 }
 
 __device__ __forceinline__ int64_t clamp_len(const SuffixArgs &a, int64_t kvl) {
@@ -315,13 +271,7 @@ __device__ __forceinline__ void write_f32_row(const SuffixArgs &a, int64_t row, 
 // of a grid of a.kv_heads * a.chunks, with the group's LDS at smem and its own
 // barrier. Windows hold 8 NW tokens.
 //
-// Two bodies:
-// * TOK = false (dims-major, vector ALU; the fused kernel above 4 heads): lane
-//   (t, c) holds token t and dims 8c .. 8c+7 and 64+8c .. 64+8c+7 of K; lane
-//   (hf, dd) holds dims 4dd .. 4dd+3 of 4 tokens of V, p reaches it through a
-//   per-wave LDS row and q is read from LDS per window. 4 accumulators per head.
-// * TOK = true (token-major on the matrix cores, 4 waves): a wave owns 8
-//   tokens of every window, and lane (g, n) = (lane / 16, lane % 16):
+// A wave owns 8 tokens of every window, and lane (g, n) = (lane / 16, lane % 16):
 // * S^T = K q^T on v_mfma_f32_16x16x32_bf16: A = K, row n = token n of the wave's
 //   8 (rows 8-15 read nothing: zeros), dims 32 s + 8 g .. + 7 at step s, straight
 //   from global memory; B = q of head n, the same dims. The result puts token
@@ -346,11 +296,11 @@ __device__ __forceinline__ void write_f32_row(const SuffixArgs &a, int64_t row, 
 // body's LDS) skips its own, waits until scan_flag is set and reads the other's
 // lengths and window prefix sums; the body given only scan_flag sets it once its
 // scan is complete.
-template <int G, int NW, int D, bool TOK, bool F32 = false, class L = SfxLds<G, NW, TOK>, class Bar>
+template <int G, int NW, int D, bool F32 = false, class L = SfxLds<G, NW>, class Bar>
 __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS char *smem, int lb, int tid,
                                                    const Bar &bar, CK_LDS int *scan_flag = nullptr,
                                                    const CK_LDS char *scan_src = nullptr) {
-    static_assert(!TOK || NW == 4, "token-major body: 4 waves");
+    static_assert(NW == 4, "the lane layouts below");
     static_assert(D + 1 <= 8, "table padding: D + 1 entries past a phase");
     constexpr int NB = D + 1;  // register ring slots: D windows in flight + the one in use
     constexpr int kThr = NW * 64;
@@ -366,16 +316,14 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     CK_LDS float *xml = (CK_LDS float *)(smem + L::kXml);
     CK_LDS int *xcnt = (CK_LDS int *)(smem + L::kXsync);  // waves counted into each slot
     CK_LDS int *xgen = xcnt + R;                             // merges completed in each slot
-    CK_LDS float *so = (CK_LDS float *)(smem + L::kSo);      // TOK: merged O of the phase's segments
-    CK_LDS float *sl = (CK_LDS float *)(smem + L::kSl);      // TOK: their LSE
-    CK_LDS int *sb = (CK_LDS int *)(smem + L::kSb);          // TOK: their sequence
+    CK_LDS float *so = (CK_LDS float *)(smem + L::kSo);      // merged O of the phase's segments
+    CK_LDS float *sl = (CK_LDS float *)(smem + L::kSl);      // their LSE
+    CK_LDS int *sb = (CK_LDS int *)(smem + L::kSb);          // their sequence
 
     const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    const int t = lane >> 3;  // K: token slot, token 8 wid + t of each window
-    const int c = lane & 7;   // K: dims 8c .. 8c+7 and 64+8c .. 64+8c+7
-    const int hf = lane >> 5; // V: tokens hf, 2 + hf, 4 + hf, 6 + hf of the wave's 8
-    const int dd = lane & 31; // V: dims 4 dd .. 4 dd + 3
+    const int t = lane >> 3;  // V rows: token 8 wid + t of each window
+    const int c = lane & 7;   // V rows: bytes 16 c and 128 + 16 c
     const int g = lb % a.kv_heads;  // kv head group: query heads g * G .. + G
     const int chunk = lb / a.kv_heads;
     const int gk = g / a.kv_sub;            // the physical kv head they read
@@ -462,8 +410,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
 
     // ---- per-lane constants ------------------------------------------------------------
     const int64_t tokb = a.tok_stride * 2;                      // bytes between token rows
-    const uint32_t koff = (uint32_t)((8 * wid + t) * tokb + c * 16);   // K byte offset in a window
-    const uint32_t voff = (uint32_t)((8 * wid + hf) * tokb + dd * 8);  // dims-major V byte offset
+    const uint32_t koff = (uint32_t)((8 * wid + t) * tokb + c * 16);   // V byte offset in a window
     const uint32_t win_bytes = (uint32_t)(kWin * tokb);          // a window's buffer range
     const char *kbase = reinterpret_cast<const char *>(a.k) + (int64_t)gk * a.head_off * 2;
     const char *vbase = reinterpret_cast<const char *>(a.v) + (int64_t)gk * a.head_off * 2;
@@ -481,8 +428,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     const int vro = (4 * (mg & 1) + (mn >> 2)) * kVtPitch + 8 * (mn & 3);
     const float sbias = (mg < 2 && mn < G) ? 0.f : -INFINITY;
 
-    float m[G], l[G], acc[G][4];  // dims-major: per head, 4 value accumulators
-    // token-major: the O^T tiles (dims 16 T + 4 mg + r of head mn), head mn's
+    // the O^T tiles (dims 16 T + 4 mg + r of head mn), head mn's
     // softmax state (m; m + kTau, the rescale trigger; the exponent offset, m or
     // 0 while m = -inf; this lane's share of the row sum), q fragments, and the
     // P^T operand (hi, lo) of the pending window
@@ -492,14 +438,10 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     uint32_t ph[2], pl[2];
     int nclose = 0;  // segments closed so far (exchange ring position)
     int qslot = 0;   // segment of the current phase
-    u32x4 kbuf[NB][TOK ? 4 : 2];
-    using VSlot = std::conditional_t<TOK, u32x4[2], u32x2[4]>;
+    u32x4 kbuf[NB][4];
+    using VSlot = u32x4[2];
     VSlot vbuf[NB];
     int eyr[NB];               // packed table fields of the window in each ring slot
-    constexpr int kPwRow = (G + 3) / 4 * 4;  // floats per token in this wave's p rows
-    static_assert(kPwRow <= 8, "p row");
-    CK_LDS float *pw = (CK_LDS float *)(smem + L::kPw) + wid * 64;
-
     // A window's loads: the buffer descriptor of its rows (K or V) starts at the
     // window and spans its valid tokens, so the range check returns 0 for the rows
     // of tokens past the sequence's end (or of an invalid page: range 0) and the
@@ -516,24 +458,6 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         const int ey = __builtin_amdgcn_readfirstlane(e[1]);
         const uint64_t off = (uint64_t)(uint32_t)max(page, 0) * pg32 + (uint32_t)tab_sub(ey) * win32;
         return TokWin{(int64_t)off, page < 0 ? 0 : (int)(tab_tv(ey) * tok32)};
-    };
-
-    // K/V loads of the window with table entry e (e[0] < 0: invalid page; a padding
-    // entry past the phase end reads nothing) into one ring slot
-    auto issue = [&](i32x2 e, u32x4 &k0, u32x4 &k1, VSlot &vv) __attribute__((always_inline)) {
-        const TokWin w = tok_win(e);
-        const __amdgpu_buffer_rsrc_t rk =
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(kbase + w.off), (short)0, w.range, kRsrcFlags);
-        const __amdgpu_buffer_rsrc_t rv =
-            __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(vbase + w.off), (short)0, w.range, kRsrcFlags);
-        k0 = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, (int)koff, 0, 0));
-        k1 = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, (int)(koff + 128), 0, 0));
-        if constexpr (!TOK) {  // the dims-major body's loads
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                vv[j] = __builtin_bit_cast(
-                    u32x2, __builtin_amdgcn_raw_buffer_load_b64(rv, (int)(voff + (uint32_t)(2 * j * tokb)), 0, 0));
-        }
     };
 
     // token-major: a window's K rows as the 4 A fragments of its score MFMAs
@@ -578,9 +502,8 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     };
 
     // Merges query-head / dim pair u (h = u / 32, dims 4 (u % 32) .. + 3) of the NW
-    // partials in exchange slot r: TOK into stash entry e, else straight out for
-    // sequence b.
-    auto merge_pair = [&](int u, int r, int b, int e) __attribute__((always_inline)) {
+    // partials in exchange slot r into stash entry e.
+    auto merge_pair = [&](int u, int r, int e) __attribute__((always_inline)) {
         const CK_LDS float *xo_r = xo + r * NW * G * kD;
         const CK_LDS float *xml_r = xml + r * NW * G * 2;
         const int h = u >> 5, d4 = u & 31;
@@ -601,15 +524,11 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         const float inv = lt > 0.f ? 1.0f / lt : 0.f;
         const float lse_v = lt > 0.f ? (mx + __log2f(lt)) * kLn2 : -INFINITY;
         const f32x4 on = f32x4{o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
-        if constexpr (TOK) {
-            *reinterpret_cast<CK_LDS f32x4 *>(so + (e * G + h) * kD + 4 * d4) = on;
-            if (d4 == 0) sl[e * G + h] = lse_v;
-        } else {
-            write_result(b, h, d4, on, lse_v);
-        }
+        *reinterpret_cast<CK_LDS f32x4 *>(so + (e * G + h) * kD + 4 * d4) = on;
+        if (d4 == 0) sl[e * G + h] = lse_v;
     };
 
-    // TOK: this wave's share of the merge of close k (exchange slot k % R, sequence
+    // This wave's share of the merge of close k (exchange slot k % R, sequence
     // b, stash entry e) once all NW partials are in (bounded wait: every wave
     // closes the same segments), so no single wave carries the whole merge. The
     // slot's arrival count only grows, NW per use, so use k / R is complete at
@@ -618,7 +537,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     // close k - 2, the slot's previous use. Each step of a close costs an LDS round
     // trip, slow while the stage-1 waves keep the LDS busy, so the close has few.
     auto merge_share = [&](int k, int b, int e) __attribute__((always_inline)) {
-        static_assert(!TOK || R <= 2, "the slot reuse argument above takes two slots");
+        static_assert(R <= 2, "the slot reuse argument above");
         const int r = k % R;
         const int target = NW * (k / R + 1);
         {
@@ -629,10 +548,10 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         }
         asm volatile("" ::: "memory");
         constexpr int kPer = 32 * G / NW;  // pairs per wave
-        static_assert(!TOK || (kPer * NW == 32 * G && kPer <= 64), "pairs split evenly over the waves");
-        if (lane < kPer) merge_pair(wid * kPer + lane, r, b, e);
+        static_assert(kPer * NW == 32 * G && kPer <= 64, "pairs split evenly over the waves");
+        if (lane < kPer) merge_pair(wid * kPer + lane, r, e);
         if (wid == 0 && lane == 0) sb[e] = b;
-        if constexpr (TOK && R == 1) {  // this wave's reads of the slot are done (LDS operations run in order)
+        if constexpr (R == 1) {  // this wave's reads of the slot are done (LDS operations run in order)
             asm volatile("" ::: "memory");
             if (lane == 0) __hip_atomic_fetch_add(xgen, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
@@ -650,37 +569,14 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         for (int T = 0; T < 8; ++T) oacc[T] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
 
-    // Closes segment b (sequence b's windows in this range): folds the lanes' partial
-    // sums, hands the wave's (O, m, l) to the exchange ring, and the last wave in
-    // merges the NW partials and writes the result (TOK: into the phase's stash).
+    // Closes segment b (sequence b's windows in this range): hands the wave's (O, m, l)
+    // to the exchange ring and merges its share of the NW partials into the phase's stash.
     auto close_seg = [&](int b) __attribute__((always_inline)) {
-        // token-major: head mn's row sum over the 4 groups; O^T needs no reduction
-        // (the MFMAs summed over the tokens). Dims-major: each head's row sum over
-        // the 8 token slots, its accumulators over the two half-waves.
-        float lt1 = 0.f;
-        if constexpr (TOK) {
-            lt1 = sum_xor32(sum_xor16(l1));
-        } else {
-#pragma unroll
-            for (int h = 0; h < G; ++h) l[h] = sum_slots(l[h]);
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[h][e] = sum_xor32(acc[h][e]);
-            }
-        }
+        // head mn's row sum over the 4 groups; O^T needs no reduction (the MFMAs
+        // summed over the tokens)
+        const float lt1 = sum_xor32(sum_xor16(l1));
         const int r = nclose % R;
-        const int want = nclose / R;  // merges the slot has seen before this segment
-        // dims-major: the slot's previous segment must be merged (bounded: a wait
-        // that never ended would mean a broken invariant, and results then are
-        // wrong, not hung; such a wait is counted). Token-major: see merge_share.
-        if constexpr (!TOK) {
-            int spin = 0;
-            for (; *(volatile CK_LDS int *)(xgen + r) != want && spin < (1 << 22); ++spin)
-                __builtin_amdgcn_s_sleep(1);
-            if (spin == (1 << 22)) count_giveup(&g_wait_giveups);
-        }
-        if constexpr (TOK && R == 1) {
+        if constexpr (R == 1) {
             // one slot: every wave's share of the previous close's merge is done
             // (each has arrived there, so each finishes it; bounded)
             int spin = 0;
@@ -690,150 +586,26 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         }
         CK_LDS float *xo_r = xo + r * NW * G * kD;
         CK_LDS float *xml_r = xml + r * NW * G * 2;
-        if constexpr (TOK) {
-            if (mn < G) {
+        if (mn < G) {
 #pragma unroll
-                for (int T = 0; T < 8; ++T)
-                    *reinterpret_cast<CK_LDS f32x4 *>(xo_r + (wid * G + mn) * kD + 16 * T + 4 * mg) = oacc[T];
-                if (mg == 0) {
-                    xml_r[(wid * G + mn) * 2] = m1;
-                    xml_r[(wid * G + mn) * 2 + 1] = lt1;
-                }
-            }
-        } else if (hf == 0) {
-#pragma unroll
-            for (int h = 0; h < G; ++h)
-                *reinterpret_cast<CK_LDS f32x4 *>(xo_r + (wid * G + h) * kD + 4 * dd) =
-                    f32x4{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
-        }
-        if (!TOK && lane == 0) {
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                xml_r[(wid * G + h) * 2] = m[h];
-                xml_r[(wid * G + h) * 2 + 1] = l[h];
+            for (int T = 0; T < 8; ++T)
+                *reinterpret_cast<CK_LDS f32x4 *>(xo_r + (wid * G + mn) * kD + 16 * T + 4 * mg) = oacc[T];
+            if (mg == 0) {
+                xml_r[(wid * G + mn) * 2] = m1;
+                xml_r[(wid * G + mn) * 2 + 1] = lt1;
             }
         }
         // a wave's LDS operations are performed in the order it issues them: its rows
-        // are in before its arrival counts (token-major: no wait for that; the
-        // dims-major path waits, as before)
-        if constexpr (TOK) asm volatile("" ::: "memory");
-        else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if constexpr (TOK) {
-            if (lane == 0) __hip_atomic_fetch_add(xcnt + r, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            merge_share(nclose, b, qslot);
-        } else {
-            int old = 0;
-            if (lane == 0) old = __hip_atomic_fetch_add(xcnt + r, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            old = __builtin_amdgcn_readfirstlane(old);
-            if (old == NW - 1) {
-                // the last wave in: merge the NW partials of every query head
-                asm volatile("" ::: "memory");
-#pragma unroll 1
-                for (int u0 = 0; u0 < 32 * G; u0 += 64) {
-                    if (u0 + lane < 32 * G) merge_pair(u0 + lane, r, b, 0);
-                }
-                // free the slot: reset its count, then publish the merge
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                if (lane == 0) xcnt[r] = 0;
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                if (lane == 0) xgen[r] = want + 1;
-            }
-        }
+        // are in before its arrival counts
+        asm volatile("" ::: "memory");
+        if (lane == 0) __hip_atomic_fetch_add(xcnt + r, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        merge_share(nclose, b, qslot);
         ++nclose;
         ++qslot;
-        if constexpr (TOK) reset_seg();
+        reset_seg();
     };
 
     i32x2 enext = i32x2{-1, 0};  // the table entry of the next window to issue
-    // One window of a phase: issue window n + D into the slot freed last step,
-    // compute window n from slot J = n % NB, close its segment if it ends here.
-    auto step = [&](auto jc, int n, int np) __attribute__((always_inline)) {
-      if constexpr (!TOK) {
-        constexpr int J = decltype(jc)::value;
-        constexpr int JI = (J + D) % NB;  // slot of window n + D (freed by window n - 1)
-        const i32x2 ei = enext;           // tab[n + D], read a step ahead
-        issue(ei, kbuf[JI][0], kbuf[JI][1], vbuf[JI]);
-        eyr[JI] = __builtin_amdgcn_readfirstlane(ei[1]);
-        const int ey = eyr[J];
-        enext = tab[n + D + 1];  // at most np + D: a padding entry past the phase
-        const int b = tab_b(ey);
-        const int t1 = min(max(tab_tv(ey) - 8 * wid, 0), 8);
-        const CK_LDS char *qrow = qs + qslot * G * (kD * 2) + c * 16;
-        if (tab_first(ey)) {
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                m[h] = -INFINITY;
-                l[h] = 0.f;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[h][e] = 0.f;
-            }
-        }
-        if (t1 > 0) {
-            const u32x4 k0 = kbuf[J][0], k1 = kbuf[J][1];
-            float s[G];  // scores, then p in place
-            bool trig = false;
-#pragma unroll
-            for (int h = 0; h < G; ++h) {  // q from LDS per window
-                const u32x4 q0 = *reinterpret_cast<const CK_LDS u32x4 *>(qrow + h * (kD * 2));
-                const u32x4 q1 = *reinterpret_cast<const CK_LDS u32x4 *>(qrow + h * (kD * 2) + 128);
-                s[h] = sum8(dot16(k0, k1, q0, q1)) * a.scale_log2;
-            }
-            if (t1 < 8) {
-#pragma unroll
-                for (int h = 0; h < G; ++h) s[h] = t < t1 ? s[h] : -INFINITY;
-            }
-#pragma unroll
-            for (int h = 0; h < G; ++h) trig |= s[h] > m[h] + kTau;  // m = -inf: always
-            if (__builtin_amdgcn_ballot_w64(trig)) {
-#pragma unroll
-                for (int h = 0; h < G; ++h) {
-                    const float m_new = fmaxf(m[h], max_slots(s[h]));
-                    if (m_new > m[h]) {
-                        const float f = exp2_fast(m[h] - m_new);  // 0 from -inf
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[h][e] *= f;
-                        l[h] *= f;
-                        m[h] = m_new;
-                    }
-                }
-            }
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                s[h] = exp2_fast(s[h] - (m[h] == -INFINITY ? 0.f : m[h]));  // 0 for masked tokens
-                l[h] += s[h];
-            }
-            // p of token t -> this wave's row t (lanes c = 0), read back per V token
-            if (c == 0) {
-#pragma unroll
-                for (int h4 = 0; h4 < kPwRow; h4 += 4)
-                    *reinterpret_cast<CK_LDS f32x4 *>(pw + t * 8 + h4) =
-                        f32x4{s[h4], h4 + 1 < G ? s[h4 + 1] : 0.f, h4 + 2 < G ? s[h4 + 2] : 0.f,
-                              h4 + 3 < G ? s[h4 + 3] : 0.f};
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const u32x2 vv = vbuf[J][j];
-                const float v0 = bf16_lo(vv[0]), v1 = bf16_hi(vv[0]), v2 = bf16_lo(vv[1]), v3 = bf16_hi(vv[1]);
-#pragma unroll
-                for (int h4 = 0; h4 < kPwRow; h4 += 4) {
-                    const f32x4 pv = *reinterpret_cast<const CK_LDS f32x4 *>(pw + (2 * j + hf) * 8 + h4);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if (h4 + e < G) {
-                            acc[h4 + e][0] = fmaf(pv[e], v0, acc[h4 + e][0]);
-                            acc[h4 + e][1] = fmaf(pv[e], v1, acc[h4 + e][1]);
-                            acc[h4 + e][2] = fmaf(pv[e], v2, acc[h4 + e][2]);
-                            acc[h4 + e][3] = fmaf(pv[e], v3, acc[h4 + e][3]);
-                        }
-                    }
-                }
-            }
-        }
-
-        if (tab_last(ey)) close_seg(b);
-      }
-    };
-
     int eypend = 0;  // packed table fields of window n - 1 (token-major)
     // Token-major values of the pending window: its V rows (lane (t, c) holds 32
     // bytes of token t) into the wave's LDS slot, back as the V^T fragments of the 8
@@ -841,7 +613,6 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     // written and read by this wave only, whose LDS operations run in issue order.
     typedef short s16x4 __attribute__((ext_vector_type(4)));
     auto pv_tok = [&](const VSlot &vv) __attribute__((always_inline)) {
-      if constexpr (TOK) {
         *reinterpret_cast<CK_LDS u32x4 *>(vt + vwo) = vv[0];
         *reinterpret_cast<CK_LDS u32x4 *>(vt + vwo + 128) = vv[1];
         uint2 vtf[8];
@@ -855,7 +626,6 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
             oacc[T] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bh, oacc[T], 0, 0, 0);
             oacc[T] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bl, oacc[T], 0, 0, 0);
         }
-      }
     };
     // Token-major window step, pipelined by one window: step n issues the K rows of
     // window n + D, computes the scores of window n and the values of window n - 1
@@ -866,7 +636,6 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     // softmax. The table entry of the window to issue was read one step ahead and
     // the packed fields of each window travel in the ring with its data.
     auto step_tok = [&](auto jc, int n, int np) __attribute__((always_inline)) {
-      if constexpr (TOK) {
         constexpr int J = decltype(jc)::value;
         constexpr int JI = (J + D) % NB;  // window n + D, into the slot of window n - 1
         const i32x2 ei = enext;
@@ -938,24 +707,21 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
             pl[i] = pack_bf16x2(s[2 * i] - __uint_as_float(u0 & 0xFFFF0000u),
                                 s[2 * i + 1] - __uint_as_float(u1 & 0xFFFF0000u));
         }
-      }
     };
     // after a phase's last window (np - 1, in slot (np - 1) % NB): its values and
     // its segment's close
     auto drain_tok = [&](int np) __attribute__((always_inline)) {
-      if constexpr (TOK) {
         const int js = (np - 1) % NB;  // wave-uniform
         static_for<NB>([&](auto jc) __attribute__((always_inline)) {
             if (js == decltype(jc)::value) pv_tok(vbuf[decltype(jc)::value]);
         });
         if (tab_last(eypend)) close_seg(tab_b(eypend));
-      }
     };
 
     // ---- phases of up to kTable windows and kQSlots segments: table and q rows,
     //      prologue loads, streaming loop --------------------------------------------
     const int nwin = w1 - w0;
-    if constexpr (TOK) reset_seg();  // the chunk's first window opens a segment
+    reset_seg();  // the chunk's first window opens a segment
     for (int p0 = 0; p0 < nwin;) {
         if (p0 > 0) {
             wait_vmcnt<0>();
@@ -1022,48 +788,36 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         qslot = 0;
 #pragma unroll
         for (int j = 0; j < D; ++j) {
-            if constexpr (TOK) {
-                const i32x2 e = tab[j];  // j < D: a padding entry when j >= np
-                const TokWin w = tok_win(e);
-                issue_kfrag(w, kbuf[j]);
-                issue_v(w, vbuf[j][0], vbuf[j][1]);
-                eyr[j] = __builtin_amdgcn_readfirstlane(e[1]);
-            } else {
-                const i32x2 e = tab[j];  // j < D: a padding entry when j >= np
-                issue(e, kbuf[j][0], kbuf[j][1], vbuf[j]);
-                eyr[j] = __builtin_amdgcn_readfirstlane(e[1]);
-            }
+            const i32x2 e = tab[j];  // j < D: a padding entry when j >= np
+            const TokWin w = tok_win(e);
+            issue_kfrag(w, kbuf[j]);
+            issue_v(w, vbuf[j][0], vbuf[j][1]);
+            eyr[j] = __builtin_amdgcn_readfirstlane(e[1]);
         }
-        if constexpr (!TOK) enext = tab[D];
-        if constexpr (TOK) {
-            enext = tab[D];
-            // "window -1" of the pipelined step (slot NB - 1): no values, no close;
-            // its V slot is zeroed so that p = 0 times it stays 0
-            ph[0] = ph[1] = pl[0] = pl[1] = 0u;
-            vbuf[NB - 1][0] = u32x4{0u, 0u, 0u, 0u};
-            vbuf[NB - 1][1] = u32x4{0u, 0u, 0u, 0u};
-            eypend = 0;
-        }
+        enext = tab[D];
+        // "window -1" of the pipelined step (slot NB - 1): no values, no close;
+        // its V slot is zeroed so that p = 0 times it stays 0
+        ph[0] = ph[1] = pl[0] = pl[1] = 0u;
+        vbuf[NB - 1][0] = u32x4{0u, 0u, 0u, 0u};
+        vbuf[NB - 1][1] = u32x4{0u, 0u, 0u, 0u};
+        eypend = 0;
         // full rounds of NB steps, then the rest: the ring slot of every step is a
         // compile-time constant and no step leaves the loop early, so the
         // compiler's vmcnt bookkeeping sees one path around the back edge
         int n = 0;
         for (int it = np / NB; it > 0; --it) {
             static_for<NB>([&](auto jc) __attribute__((always_inline)) {
-                if constexpr (TOK) step_tok(jc, n + decltype(jc)::value, np);
-                else step(jc, n + decltype(jc)::value, np);
+                step_tok(jc, n + decltype(jc)::value, np);
             });
             n += NB;
         }
         const int rem = np - n;
         static_for<NB>([&](auto jc) __attribute__((always_inline)) {
             if (decltype(jc)::value < rem) {
-                if constexpr (TOK) step_tok(jc, n + decltype(jc)::value, np);
-                else step(jc, n + decltype(jc)::value, np);
+                step_tok(jc, n + decltype(jc)::value, np);
             }
         });
         drain_tok(np);
-        if constexpr (TOK) {
             // the phase's merged results out, by every wave of the role: each merge
             // is done once every wave is past its last close
             bar.sync();
@@ -1074,7 +828,6 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
                 write_result(sb[e], h, d4, *reinterpret_cast<const CK_LDS f32x4 *>(so + (e * G + h) * kD + 4 * d4),
                              sl[e * G + h]);
             }
-        }
         p0 = p1;
     }
 }
@@ -1086,11 +839,11 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
 template <int G, bool F32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void suffix_stream_kernel(SuffixArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    suffix_stream_body<G, 4, (G > 4 ? 1 : kTokDepth), true, F32>(a, (CK_LDS char *)smem_raw, blockIdx.x, threadIdx.x,
+    suffix_stream_body<G, 4, (G > 4 ? 1 : kTokDepth), F32>(a, (CK_LDS char *)smem_raw, blockIdx.x, threadIdx.x,
                                                            WgBarrier{});
 }
-static_assert(SfxLds<5, 4, true>::kBytes <= 80 * 1024, "two stand-alone workgroups per CU up to 5 heads");
-static_assert(SfxLds<kMaxGroup, 4, true>::kBytes <= 160 * 1024, "one above");
+static_assert(SfxLds<5, 4>::kBytes <= 80 * 1024, "two stand-alone workgroups per CU up to 5 heads");
+static_assert(SfxLds<kMaxGroup, 4>::kBytes <= 160 * 1024, "one above");
 
 // Folds the partials of one query head of a sequence cut by chunk boundaries
 // (chunks ca < cb): the tail slot (1) of chunk ca and the head slot (0) of every
@@ -1348,7 +1101,7 @@ __global__ __launch_bounds__(kMaxGroup * 32) void cascade_epilogue_kernel(const 
 // for the other.
 constexpr int kFusedS1Lds = s1::wide_lds_bytes<3>();
 template <int G>
-using FusedSfx = SfxLds<G, 4, true, (G <= 4 ? kQSlots : 4), (G <= 4 ? 2 : 1)>;  // the stream body's layout on 4 waves
+using FusedSfx = SfxLds<G, 4, (G <= 4 ? kQSlots : 4), (G <= 4 ? 2 : 1)>;  // the stream body's layout on 4 waves
 template <int G>
 constexpr int fused_lds_bytes() { return kFusedS1Lds + FusedSfx<G>::kBytes + 32; }
 static_assert(fused_lds_bytes<4>() <= 160 * 1024 && fused_lds_bytes<kMaxGroup>() <= 160 * 1024,
@@ -1386,7 +1139,7 @@ __global__ __launch_bounds__(512) void cascade_fused_kernel(s1::Stage1Args s1a, 
         constexpr int kRoleRot = 3;
         const int g = ((int)blockIdx.x + kRoleRot) % sa.kv_heads, j = (int)blockIdx.x / sa.kv_heads;
         // the streaming waves scan the lengths; the stage-1 waves reuse that scan
-        suffix_stream_body<G, 4, kTokDepth, true, false, FusedSfx<G>>(
+        suffix_stream_body<G, 4, kTokDepth, false, FusedSfx<G>>(
             sa, smem + (role ? 0 : kFusedS1Lds), (2 * j + role) * sa.kv_heads + g, threadIdx.x & 255, bar, bars + 4,
             role ? smem + kFusedS1Lds : nullptr);
     }
@@ -1423,7 +1176,7 @@ int launch_fused(const s1::Stage1Args &s1a, int64_t n1, const SuffixArgs &a, con
 template <int G, bool F32 = false>
 int launch_suffix(const SuffixArgs &a, bool fixup, const EpilogueArgs *epi, hipStream_t st) {
     static std::atomic<uint64_t> lds_set{0};
-    constexpr int kLds = SfxLds<G, 4, true>::kBytes;
+    constexpr int kLds = SfxLds<G, 4>::kBytes;
     int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(&suffix_stream_kernel<G, F32>), kLds, lds_set);
     if (rc != CK_OK) return rc;
     hipLaunchKernelGGL((suffix_stream_kernel<G, F32>), dim3((unsigned)(a.kv_heads * a.chunks)), dim3(256), kLds, st, a);
@@ -1474,18 +1227,19 @@ int64_t suffix_group_batch(int64_t kv_cap) {
 //   (suffix_stream_kernel), and a second generation pays the start-up again
 //   (64 / 8 heads, 64 suffixes of mean 512: 42.5 us with 512 workgroups, 36.3 with
 //   256; 256 suffixes 115 / 109; 4 of mean 64 27.7 / 10.8).
-// * Up to 5 heads, one per CU for long sequences, at most two per chunk: half the
-//   partials and start-ups (40 / 8 heads, 24 requests of 4096: 80.8 / 74.3 us; 7
-//   31.4 / 29.9; 32 / 8 heads, 64 suffixes of mean 512 36.9 / 37.0, of mean 1024
-//   57.1 / 55.3). Two per CU otherwise: with many short sequences per chunk the
-//   closes bound it (256 suffixes of mean 64: 25.4 / 30.7).
+// * Up to 5 heads, one per CU for long sequences, at most one per chunk (two at 5
+//   heads): half the partials and start-ups (two / one per CU: 40 / 8 heads, 24
+//   requests of 4096 80.8 / 74.3 us, 64 suffixes of mean 512 37.5 / 36.1; 32 / 8
+//   heads, 16 of mean 512 17.2 / 16.4, 64 36.9 / 37.0). Two per CU otherwise: with
+//   many short sequences per chunk the closes bound it (256 of mean 64: 25.4 / 30.7).
 // * A sequence of n windows spans chunks / batch chunks; its fold takes a memory
 //   round trip per 8 (about 0.15 us a chunk) and a chunk's windows about 0.5 us
 //   each: sqrt(cap / 8) chunks per sequence balance the two (8 / 1 heads, 7 requests
 //   of 4096: 26.2 us over 512 chunks, 13.8 over 112, 15.6 over 56).
 int64_t suffix_default_chunks(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap) {
     const int64_t groups = kv_heads * suffix_sub_groups(num_heads, kv_heads);
-    const bool one = num_heads > 5 * groups || (kv_cap >= 1024 && batch <= 2 * 256 / groups);
+    const int64_t g = num_heads / groups;
+    const bool one = g > 5 || (kv_cap >= 1024 && batch <= (g > 4 ? 2 : 1) * 256 / groups);
     const int64_t per_seq = std::max<int64_t>(8, (int64_t)std::sqrt((double)kv_cap / 8));
     const int64_t p = std::min((one ? 256 : 512) / groups, batch * per_seq);
     return p > 0 ? p : 1;
@@ -1533,7 +1287,7 @@ int suffix_launch_group(const void *q, const void *k, const void *v, const int32
     a.kv_sub = (int)sub;
     a.kv_cap = (int)kv_cap;
     a.chunks = (int)chunks;
-    a.split = fused && cascade ? kFusedSplit : 0;
+    a.split = fused && cascade ? fused_split(G) : 0;
     a.scale_log2 = scale * kLog2e;
     EpilogueArgs e;
     if (cascade) {
