@@ -116,8 +116,9 @@ int ck_lse_merge(const void *o1, int o1_dtype, const void *o2, int o2_dtype,
  * row sums use the unrounded fp32 values, as
  * third_party/catlass/.../block_epilogue_online_softmax_no_mask.hpp:487-594 does.
  * With one query token per request (q_len_uniform == 1), kv_cap >= 1024, the
- * plan's split count and its workspace, the requests are streamed as
- * ck_suffix_decode does, with P at fp32 precision.
+ * plan's split count and a workspace of at least ck_suffix_decode_plan's bytes
+ * too, the requests are streamed as ck_suffix_decode does, with P at fp32
+ * precision.
  * Replaces OPS/fa_fp32_stage1/op_kernel/kernel_fa_fp32_stage1.cpp:848-863.
  * ========================================================================== */
 int ck_fa_fp32_stage1_plan(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_heads,
@@ -145,8 +146,9 @@ int ck_fa_fp32_stage1(const void *q, const void *k, const void *v, const int32_t
  *                gets out = 0 and lse = -inf (an empty suffix)
  *   kv_cap       upper bound of kv_seqlens(b), <= bt_cols * 128
  *   num_splits   workgroups per kv head group that share the list of 64-token
- *                windows (<= 0: the plan's count, as many as are resident at
- *                once); the plan sizes the workspace for it. A GQA group of
+ *                windows (<= 0 or the plan's count: as many as suit the batch
+ *                and kv_cap, at most the plan's); the plan sizes the workspace
+ *                for it. A GQA group of
  *                more than 8 query heads per kv head is split into the fewest
  *                equal groups of at most 8, each streamed as its own kv head
  *                group (the K/V pages are then read once per group).

@@ -202,8 +202,8 @@ bool decode_form(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv
     return max_q_len == 1 && batch > 0 && kv_cap >= kDecodeMinCap && num_heads <= (1 << 16) &&
            batch <= suffix_group_batch(kv_cap);
 }
-int64_t decode_ws_bytes(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap) {
-    return suffix_group_ws_bytes(batch, num_heads, kv_heads, suffix_default_chunks(batch, num_heads, kv_heads, kv_cap));
+int64_t decode_ws_bytes(int64_t batch, int64_t num_heads, int64_t kv_heads) {
+    return suffix_group_ws_bytes(batch, num_heads, kv_heads, suffix_plan_chunks(num_heads, kv_heads));
 }
 
 int check_dims(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_heads, int64_t head_dim,
@@ -231,8 +231,6 @@ extern "C" int ck_fa_fp32_stage1_plan(int64_t batch, int64_t max_q_len, int64_t 
     make_plan(batch, max_q_len, num_heads, kv_heads, kv_cap, 0, &p);
     *num_splits = p.splits;
     *workspace_bytes = p.ws_bytes;
-    if (decode_form(batch, max_q_len, num_heads, kv_heads, kv_cap))
-        *workspace_bytes = std::max(p.ws_bytes, decode_ws_bytes(batch, num_heads, kv_heads, kv_cap));
     return CK_OK;
 }
 
@@ -263,11 +261,11 @@ int ck::stage1_launch(const void *q, const void *k, const void *v, const int32_t
 
     Plan p;
     make_plan(batch, max_q_len, num_heads, kv_heads, kv_cap, 0, &p);
-    // the decode form with the plan's split count and workspace; a caller's own split
-    // count, or a workspace sized for the splits alone, runs the tiles
+    // the decode form with the plan's split count and a workspace that also holds the
+    // suffix plan's; a caller's own split count, or a smaller workspace, runs the tiles
     if (combine && q_len_uniform == 1 && decode_form(batch, max_q_len, num_heads, kv_heads, kv_cap) &&
         (num_splits <= 0 || num_splits == p.splits) && workspace != nullptr &&
-        workspace_bytes >= decode_ws_bytes(batch, num_heads, kv_heads, kv_cap))
+        workspace_bytes >= decode_ws_bytes(batch, num_heads, kv_heads))
         return suffix_launch_group(q, k, v, block_table, bt_cols, kv_seqlens, 0, batch, num_heads, kv_heads,
                                    num_blocks, CK_KV_NHD, scale, kv_cap,
                                    suffix_default_chunks(batch, num_heads, kv_heads, kv_cap), out, lse, workspace, nullptr, nullptr, nullptr, s, nullptr, 0, true);

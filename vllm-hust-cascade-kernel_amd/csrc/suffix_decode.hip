@@ -1245,6 +1245,13 @@ int64_t suffix_default_chunks(int64_t batch, int64_t num_heads, int64_t kv_heads
     return p > 0 ? p : 1;
 }
 
+// The chunk count the plan reports, whatever the batch: two workgroups per CU. A call
+// that passes it (or none) gets suffix_default_chunks, which is never more.
+int64_t suffix_plan_chunks(int64_t num_heads, int64_t kv_heads) {
+    const int64_t p = 512 / (kv_heads * suffix_sub_groups(num_heads, kv_heads));
+    return p > 0 ? p : 1;
+}
+
 int64_t suffix_fused_chunks(int64_t num_heads, int64_t kv_heads) {
     const int64_t groups = kv_heads * suffix_sub_groups(num_heads, kv_heads);
     const int64_t p = 256 / groups;
@@ -1353,7 +1360,7 @@ extern "C" int ck_suffix_decode_plan(int64_t batch, int64_t num_heads, int64_t k
     int rc = check_suffix_dims(batch, num_heads, kv_heads, head_dim, kv_cap);
     if (rc != CK_OK) return rc;
     if (!num_splits || !workspace_bytes) return CK_E_NULL_PTR;
-    const int64_t chunks = suffix_default_chunks(batch, num_heads, kv_heads, kv_cap);
+    const int64_t chunks = suffix_plan_chunks(num_heads, kv_heads);
     const int64_t nb = batch < suffix_group_batch(kv_cap) ? batch : suffix_group_batch(kv_cap);
     *num_splits = chunks;
     *workspace_bytes = batch > 0 ? suffix_group_ws_bytes(nb, num_heads, kv_heads, chunks) : 0;
@@ -1377,7 +1384,9 @@ extern "C" int ck_suffix_decode(const void *q, const void *k, const void *v, con
     if (!aligned_to(q, 16) || !aligned_to(k, 16) || !aligned_to(v, 16) || !aligned_to(out, 8) ||
         !aligned_to(lse, 4) || !aligned_to(workspace, 16))
         return CK_E_INVALID_ARG;
-    const int64_t chunks = num_splits > 0 ? num_splits : suffix_default_chunks(batch, num_heads, kv_heads, kv_cap);
+    const int64_t chunks = num_splits > 0 && num_splits != suffix_plan_chunks(num_heads, kv_heads)
+                               ? num_splits
+                               : suffix_default_chunks(batch, num_heads, kv_heads, kv_cap);
     if (kv_heads * suffix_sub_groups(num_heads, kv_heads) * chunks > 0x7FFFFFFF || chunks > (1 << 20))
         return CK_E_INVALID_ARG;
     const int64_t per_launch = suffix_group_batch(kv_cap);

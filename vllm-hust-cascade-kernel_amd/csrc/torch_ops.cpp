@@ -213,6 +213,12 @@ std::tuple<at::Tensor, at::Tensor> fa_fp32_stage1_impl(const at::Tensor &query, 
     check_launch(ck_fa_fp32_stage1_plan(batch, max_q_len, num_heads, kv_heads, embed, kv_cap, &num_splits,
                                         &ws_bytes),
                  "fa_fp32_stage1");
+    // one token per request from a kv bound of 1024: with room for the suffix plan's
+    // partials the requests are streamed (below, the kernel would not use it)
+    int64_t sfx_splits = 0, sfx_bytes = 0;
+    if (max_q_len == 1 && kv_cap >= 1024 &&
+        ck_suffix_decode_plan(batch, num_heads, kv_heads, embed, kv_cap, &sfx_splits, &sfx_bytes) == CK_OK)
+        ws_bytes = std::max(ws_bytes, sfx_bytes);
     at::Tensor ws;
     if (ws_bytes > 0) ws = at::empty({ws_bytes}, query.options().dtype(at::kByte));
     const float scale = static_cast<float>(1.0 / std::sqrt(1.0 * embed));
