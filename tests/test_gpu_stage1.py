@@ -395,3 +395,21 @@ def test_decode_form(case):
         l3.data_ptr(), ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
     assert abi.wait_giveups() == 0
     _check(inp, o3.cpu().numpy(), l3.cpu().numpy(), H, name + " tiles")
+
+
+def test_decode_form_infinite_values():
+    """An infinite V element reaches its own dim of the heads that read it as an
+    infinity of the same sign (p > 0 of every token); every other output is finite."""
+    B, H, KVH, kvs = 3, 40, 8, [1024, 7, 801]
+    inp = paged_inputs(B, kvs, H, KVH, seed=23, q_len=1, permute=True, block_cols=8)
+    q, k, v, bt, qs, kl = _dev(inp)
+    want = {}
+    for b, tok, g, d, val in [(0, 0, 0, 5, np.inf), (0, 1023, 3, 127, -np.inf), (1, 6, 7, 0, np.inf),
+                              (2, 800, 2, 64, np.inf), (2, 333, 2, 64, np.inf)]:
+        v[int(bt[b, tok // 128]), tok % 128, g, d] = val
+        want[b, g, d] = val
+    out = torch.ops.npu.fa_fp32_stage1(q, k, v, bt, qs, kl, 1)[0].cpu().numpy().reshape(B, KVH, H // KVH, 128)
+    for (b, g, d), val in want.items():
+        assert (out[b, g, :, d] == val).all(), (b, g, d, out[b, g, :, d])
+        out[b, g, :, d] = 0
+    assert np.isfinite(out).all()

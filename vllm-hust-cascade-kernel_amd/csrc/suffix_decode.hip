@@ -611,6 +611,10 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     // bytes of token t) into the wave's LDS slot, back as the V^T fragments of the 8
     // dim tiles, then O^T += V^T P^T for the hi and the lo term of P. The slot is
     // written and read by this wave only, whose LDS operations run in issue order.
+    // F32 zeroes the V^T fragments of the operand's token rows 8-15 (copies of rows
+    // 0-7 whose P is 0): stage-1 keeps an infinite V element infinite, and inf * 0
+    // is NaN.
+    const uint32_t vmask = mg < 2 ? 0xFFFFFFFFu : 0u;
     typedef short s16x4 __attribute__((ext_vector_type(4)));
     auto pv_tok = [&](const VSlot &vv) __attribute__((always_inline)) {
         *reinterpret_cast<CK_LDS u32x4 *>(vt + vwo) = vv[0];
@@ -622,6 +626,10 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         const s16x4 bl = __builtin_bit_cast(s16x4, uint2{pl[0], pl[1]});
 #pragma unroll
         for (int T = 0; T < 8; ++T) {
+            if constexpr (F32) {
+                vtf[T].x &= vmask;
+                vtf[T].y &= vmask;
+            }
             const s16x4 av = __builtin_bit_cast(s16x4, vtf[T]);
             oacc[T] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bh, oacc[T], 0, 0, 0);
             oacc[T] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bl, oacc[T], 0, 0, 0);
@@ -699,13 +707,19 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
             l1 += s[r];
         }
         // P^T of window n for the next step: hi = p truncated to bf16 (exact in fp32),
-        // lo = p - hi (exact) rounded to bf16
+        // lo = p - hi (exact) rounded to bf16. F32: lo is at least 2^-40 p, so that it is
+        // 0 only where p is (an infinite V element times a zero lo would be NaN).
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const uint32_t u0 = __float_as_uint(s[2 * i]), u1 = __float_as_uint(s[2 * i + 1]);
+            const float p0 = s[2 * i], p1 = s[2 * i + 1];
+            const uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
             ph[i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-            pl[i] = pack_bf16x2(s[2 * i] - __uint_as_float(u0 & 0xFFFF0000u),
-                                s[2 * i + 1] - __uint_as_float(u1 & 0xFFFF0000u));
+            float lo0 = p0 - __uint_as_float(u0 & 0xFFFF0000u), lo1 = p1 - __uint_as_float(u1 & 0xFFFF0000u);
+            if constexpr (F32) {
+                lo0 = fmaxf(lo0, p0 * 0x1p-40f);
+                lo1 = fmaxf(lo1, p1 * 0x1p-40f);
+            }
+            pl[i] = pack_bf16x2(lo0, lo1);
         }
     };
     // after a phase's last window (np - 1, in slot (np - 1) % NB): its values and
