@@ -413,3 +413,22 @@ def test_decode_form_infinite_values():
         assert (out[b, g, :, d] == val).all(), (b, g, d, out[b, g, :, d])
         out[b, g, :, d] = 0
     assert np.isfinite(out).all()
+
+
+# Two wave sets share a split's pages, one 64-token tile of each page per set: lengths
+# that end in the first set's tile, on a tile or page edge, one token into either; rows
+# that fill no 128-row unit; several splits (the first cases have one).
+PAIR = [("q3_h40", 3, [129, 192, 193, 256, 257, 1], 40, 8), ("q17_h64", 17, [200, 447], 64, 8),
+        ("q9_gqa16", 9, [2048, 2113], 16, 1), ("q130_h8", 130, [1000], 8, 8), ("q2_h8", 2, [6400, 65, 6337], 8, 1)]
+
+
+@pytest.mark.parametrize("case", PAIR, ids=[c[0] for c in PAIR])
+def test_two_wave_sets(case):
+    name, n, kvs, H, KVH = case
+    B = len(kvs)
+    inp = paged_inputs(B, kvs, H, KVH, seed=29, q_len=n, permute=True, block_cols=max(2, (max(kvs) + 127) // 128))
+    out, lse = _run(inp, n)
+    _check(inp, out, lse, H, name)
+    again, lse2 = _run(inp, n)
+    assert np.array_equal(out.view(np.uint32), again.view(np.uint32))
+    assert np.array_equal(lse.view(np.uint32), lse2.view(np.uint32))

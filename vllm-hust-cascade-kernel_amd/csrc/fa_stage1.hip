@@ -20,11 +20,12 @@
 // * Every wave owns 32 query rows and all tokens of them, so a row has one
 //   online-softmax state over the whole split and P is rounded on the row's
 //   own running maximum (moved once per 64-token tile; for kv <= 64 that is
-//   the row maximum the reference rounds on). Two kernels run the same body
+//   the row maximum the reference rounds on). Three kernels run the same body
 //   (stage1_wide.h):
-//   - stage1_narrow_kernel (m-tile of 128 rows): 4 waves with at most 256
-//     registers each and a 3-slot K/V ring, the body the fused cascade kernel
-//     runs as its stage-1 role.
+//   - stage1_pair_kernel (m-tile of 128 rows): two sets of 4 waves, one 64-token
+//     tile of each page per set, a 2-slot K/V ring each; (O, m, l) of the sets are
+//     merged in LDS. Splits of a single page run stage1_narrow_kernel: one set and a
+//     3-slot ring, the body the fused cascade kernel runs as its stage-1 role.
 //   - stage1_wide_kernel (m-tile of 256 rows, when a request has more than 128
 //     rows per kv head and enough kv to fill the chip): 8 waves, two per SIMD;
 //     every 64-token K/V tile in LDS feeds 256 rows, and one wave of a SIMD
@@ -72,8 +73,19 @@ __global__ __launch_bounds__(kWW * 64) void stage1_wide_kernel(Stage1Args a) {
     stage1_wide_body<kWW, kWSlots>(a, (CK_LDS char *)smem_raw, blockIdx.x, gridDim.x, threadIdx.x, WgBarrier{});
 }
 
-// 128-row m-tiles: the same whole-row body on 4 waves with a 3-slot ring (the
-// stage-1 role of the fused cascade kernel, as a kernel of its own)
+// 128-row m-tiles: the whole-row body on two sets of 4 waves that take the two
+// 64-token tiles of each page. A lone wave per SIMD spends three quarters of a tile
+// waiting on its own chain (LDS reads, row max, exp), so the second set's work fits
+// beside the first's. One set / two: 64 queries of 32 / 8 heads on 8192 tokens 22.3 /
+// 21.5 us; 200 of 64 / 8 on 1500 36.9 / 33.0; 24 requests of 2 x 40 / 8 on up to 4000
+// 88.4 / 78; 20 of 8 / 1 on 20000 22.6 / 20.6; 64 requests of 2 on 200 21.4 / 20.7.
+__global__ __launch_bounds__(512) void stage1_pair_kernel(Stage1Args a) {
+    extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+    stage1_wide_body<4, 2, 2>(a, (CK_LDS char *)smem_raw, blockIdx.x, gridDim.x, threadIdx.x, WgBarrier{});
+}
+
+// 128-row m-tiles over splits of one page: one set of 4 waves (two sets take one tile
+// each and then merge, which costs more than the second tile)
 constexpr int kNLds = wide_lds_bytes<3>();
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void stage1_narrow_kernel(Stage1Args a) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -307,6 +319,11 @@ int ck::stage1_launch(const void *q, const void *k, const void *v, const int32_t
         rc = ensure_dynamic_lds(reinterpret_cast<const void *>(&stage1_wide_kernel), kWLds, lds_set_w);
         if (rc != CK_OK) return rc;
         hipLaunchKernelGGL(stage1_wide_kernel, dim3((unsigned)grid), dim3(kWW * 64), kWLds, s, a);
+    } else if (p.split_len > kPage) {
+        static std::atomic<uint64_t> lds_set2{0};
+        rc = ensure_dynamic_lds(reinterpret_cast<const void *>(&stage1_pair_kernel), kPairLds, lds_set2);
+        if (rc != CK_OK) return rc;
+        hipLaunchKernelGGL(stage1_pair_kernel, dim3((unsigned)grid), dim3(512), kPairLds, s, a);
     } else {
         static std::atomic<uint64_t> lds_set1{0};
         rc = ensure_dynamic_lds(reinterpret_cast<const void *>(&stage1_narrow_kernel), kNLds, lds_set1);

@@ -66,23 +66,38 @@ constexpr int kTBytes = kTTok * kD * 2;              // 16 KB of K (or V) per ti
 // The body is shared with the fused cascade kernel, where 4 waves run it (128
 // rows, a 3-slot ring) beside 4 waves of suffix streaming: NW waves, SLOTS ring
 // slots, its own barrier, workgroup lb of nlb, thread tid of the NW * 64.
+// HALVES = 2 (the 128-row stand-alone kernel): two sets of NW waves share the rows;
+// each step takes one page, set h its 64-token tile h into a ring of its own, in
+// lockstep on the one barrier, and the two softmax states meet in LDS at the end.
+// Two waves per SIMD then hide each other's LDS, DMA and softmax latencies, which
+// are three quarters of a lone wave's time per tile.
 constexpr int kWW = 8;
 constexpr int kWSlots = 4;
 constexpr int kWStage = 2 * kTBytes;  // K + V of one tile (32 KB)
 template <int SLOTS>
 constexpr int wide_lds_bytes() { return SLOTS * kWStage + kMaxSplitPages * 4; }
 constexpr int kWLds = wide_lds_bytes<kWSlots>();
+// two rings of two slots, the page ids, (m, l) of 2 x 128 rows
+constexpr int kPairLds = 2 * 2 * kWStage + kMaxSplitPages * 4 + 2 * 128 * 8;
 
-template <int NW, int SLOTS, class Bar>
+template <int NW, int SLOTS, int HALVES = 1, class Bar>
 __device__ __forceinline__ void stage1_wide_body(const Stage1Args &a, CK_LDS char *smem, int lb, int nlb, int tid,
                                                  const Bar &bar) {
     constexpr int kWRows = NW * 32;
     constexpr int kWBlk = kTBytes / 1024 / NW;  // 1-KB DMAs of K (and of V) per wave per tile
     static_assert(SLOTS >= 2 && SLOTS <= 4, "ring depth");
     static_assert(NW * 32 * kD * 4 <= SLOTS * kWStage, "epilogue slabs fit the ring");
-    CK_LDS int *s_pages = (CK_LDS int *)(smem + SLOTS * kWStage);
+    static_assert(HALVES == 1 || (HALVES == 2 && kPage == 2 * kTTok), "one tile of each page per set");
+    constexpr int kThr = HALVES * NW * 64;
+    constexpr int kStep = HALVES * kTTok;  // tokens per step
+    constexpr int kStepsPerPage = kPage / kStep;
+    CK_LDS int *s_pages = (CK_LDS int *)(smem + HALVES * SLOTS * kWStage);
 
-    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: DMA LDS addresses in SGPRs
+    // wave-uniform: DMA LDS addresses in SGPRs
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = HALVES == 1 ? 0 : wave / NW;
+    const int wid = wave - half * NW;
+    CK_LDS char *ring = smem + half * SLOTS * kWStage;
     const int lane = tid & 63;
     const int hh = lane >> 5;
 
@@ -127,7 +142,7 @@ __device__ __forceinline__ void stage1_wide_body(const Stage1Args &a, CK_LDS cha
         const int pg0 = kv_lo / kPage;
         const int64_t avail = a.bt_cols - pg0;
         const int pg_n = (int)min((int64_t)(a.split_len / kPage), avail > 0 ? avail : (int64_t)0);
-        for (int pi = tid; pi < pg_n; pi += NW * 64) {
+        for (int pi = tid; pi < pg_n; pi += kThr) {
             const int page = a.bt[(int64_t)b * a.bt_cols + pg0 + pi];
             s_pages[pi] = (page >= 0 && (int64_t)page < a.num_blocks) ? page : -1;
         }
@@ -140,7 +155,7 @@ __device__ __forceinline__ void stage1_wide_body(const Stage1Args &a, CK_LDS cha
     int kv_hi = kv_lo + a.split_len;
     if (kv_hi > (int)kvl) kv_hi = (int)kvl;
     const int ntok = kv_hi > kv_lo ? kv_hi - kv_lo : 0;
-    const int ntiles = (ntok + kTTok - 1) / kTTok;
+    const int ntiles = (ntok + kStep - 1) / kStep;  // steps: a tile of every set
 
     wait_vmcnt<0>();
     bar.sync();  // s_pages visible
@@ -161,10 +176,10 @@ __device__ __forceinline__ void stage1_wide_body(const Stage1Args &a, CK_LDS cha
     const uint32_t page_bytes = 2 * tile_bytes;
     auto issue = [&](int t, int raw, int slot) {
         raw = __builtin_amdgcn_readfirstlane(raw);
-        const uint64_t base = (uint64_t)(uint32_t)max(raw, 0) * page_bytes + ((t & 1) ? tile_bytes : 0u);
+        const uint64_t base = (uint64_t)(uint32_t)max(raw, 0) * page_bytes + ((HALVES == 2 ? half : t & 1) ? tile_bytes : 0u);
         const ck_rsrc_t rk = buf_rsrc(reinterpret_cast<const char *>(a.k) + base, tile_bytes);
         const ck_rsrc_t rv = buf_rsrc(reinterpret_cast<const char *>(a.v) + base, tile_bytes);
-        CK_LDS char *kd = smem + slot * kWStage + wid * kWBlk * 1024;
+        CK_LDS char *kd = ring + slot * kWStage + wid * kWBlk * 1024;
 #pragma unroll
         for (int j = 0; j < kWBlk; ++j) {
             dma16_buf(rk, (int)(dma_off[j] * 2), 0, kd + j * 1024);
@@ -190,34 +205,39 @@ __device__ __forceinline__ void stage1_wide_body(const Stage1Args &a, CK_LDS cha
         return tile_off(t1, d >> 3) + (d & 7) * 2;
     };
 
-    for (int t = 0; t < SLOTS - 1 && t < ntiles; ++t) issue(t, s_pages[t >> 1], t);
+    // (the whole ring at the start measured 2-8% slower: the first tile then waits
+    // behind the issue of the others)
+    for (int t = 0; t < SLOTS - 1 && t < ntiles; ++t) issue(t, s_pages[t / kStepsPerPage], t);
     int slot = 0;  // t % SLOTS
     for (int t = 0; t < ntiles; ++t) {
         // page ids of tile t and of the tile issued below, read before the waits
-        const int pg_t = s_pages[t >> 1];
-        const int pg_i = t + SLOTS - 1 < ntiles ? s_pages[(t + SLOTS - 1) >> 1] : 0;
+        const int pg_t = s_pages[t / kStepsPerPage];
+        const bool more = t + SLOTS - 1 < ntiles;
+        const int pg_i = more ? s_pages[(t + SLOTS - 1) / kStepsPerPage] : 0;
         // tile t has landed once at most the DMAs of the tiles after it remain
         const int after = min(SLOTS - 2, ntiles - 1 - t);
-        if (after >= 2) wait_vmcnt<4 * kWBlk>();
+        if (after >= 3) wait_vmcnt<6 * kWBlk>();
+        else if (after == 2) wait_vmcnt<4 * kWBlk>();
         else if (after == 1) wait_vmcnt<2 * kWBlk>();
         else wait_vmcnt<0>();
         bar.sync();  // ... in every wave; every wave is done with tile t - 1
-        const int nv = min(kTTok, ntok - t * kTTok);
+        // tokens of this step's tile (none in set 1 where the split ends in set 0's)
+        const int nv = max(0, min(kTTok, ntok - t * kStep - half * kTTok));
         const bool ok = pg_t >= 0;
-        CK_LDS char *kb = smem + slot * kWStage;
+        CK_LDS char *kb = ring + slot * kWStage;
         CK_LDS char *vb = kb + kTBytes;
-        if (nv < kTTok || !ok) {
+        if (ntok - t * kStep < kStep || !ok) {  // the same in both sets: they share the barrier
             // rows past the split's end or of an invalid page: zero them so 0 * V
             // cannot produce a NaN (an invalid page reads as zero rows)
             const int z0 = ok ? nv : 0;
-            for (int idx = tid; idx < (kTTok - z0) * 16; idx += NW * 64) {
+            for (int idx = tid - half * NW * 64; idx < (kTTok - z0) * 16; idx += NW * 64) {
                 const int tt = z0 + (idx >> 4), c = idx & 15;
                 *reinterpret_cast<CK_LDS u32x4 *>(kb + tt * 256 + c * 16) = u32x4{0, 0, 0, 0};
                 *reinterpret_cast<CK_LDS u32x4 *>(vb + tt * 256 + c * 16) = u32x4{0, 0, 0, 0};
             }
             bar.sync();
         }
-        if (t + SLOTS - 1 < ntiles) issue(t + SLOTS - 1, pg_i, slot == 0 ? SLOTS - 1 : slot - 1);  // tile t - 1's slot
+        if (more) issue(t + SLOTS - 1, pg_i, slot == 0 ? SLOTS - 1 : slot - 1);  // tile t - 1's slot
         slot = slot == SLOTS - 1 ? 0 : slot + 1;
         if (!wave_active) continue;
 
@@ -312,13 +332,27 @@ __device__ __forceinline__ void stage1_wide_body(const Stage1Args &a, CK_LDS cha
     }
 
     // ---- normalise and write whole rows through the idle ring ------------------------
-    const float l_run = l_part + __shfl_xor(l_part, 32);
-    bar.sync();  // every wave is past its last ring read
-    if (!wave_active) return;  // wave-uniform
-    const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;
-    const float lse_v = l_run > 0.f ? (m_run + __log2f(l_run)) * kLn2 : -INFINITY;
-    CK_LDS float *slab = (CK_LDS float *)smem + wid * (32 * kD);
+    float l_run = l_part + __shfl_xor(l_part, 32);
     const int my_row = lane & 31;
+    CK_LDS float *ml = (CK_LDS float *)(s_pages + kMaxSplitPages) + 2 * (wid * 32 + my_row);  // + 64 NW per set
+    if (HALVES == 2 && hh == 0) {
+        ml[half * 64 * NW] = m_run;
+        ml[half * 64 * NW + 1] = l_run;
+    }
+    bar.sync();  // every wave is past its last ring read
+    if (HALVES == 1 && !wave_active) return;  // wave-uniform
+    float wgt = 1.f;  // of this set's O
+    if constexpr (HALVES == 2) {
+        const float m_other = ml[(1 - half) * 64 * NW], l_other = ml[(1 - half) * 64 * NW + 1];
+        const float m_all = fmaxf(m_run, m_other);
+        const float m_use = m_all == -INFINITY ? 0.f : m_all;
+        wgt = exp2_fast(m_run - m_use);
+        l_run = fmaf(l_run, wgt, l_other * exp2_fast(m_other - m_use));
+        m_run = m_all;
+    }
+    const float inv = l_run > 0.f ? wgt / l_run : 0.f;
+    const float lse_v = l_run > 0.f ? (m_run + __log2f(l_run)) * kLn2 : -INFINITY;
+    CK_LDS float *slab = (CK_LDS float *)ring + wid * (32 * kD);
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -328,7 +362,7 @@ __device__ __forceinline__ void stage1_wide_body(const Stage1Args &a, CK_LDS cha
             const int chunk = (8 * db + 2 * c4 + hh) ^ my_row;
             *reinterpret_cast<CK_LDS f32x4 *>(slab + my_row * kD + chunk * 4) = o;
         }
-    if (row_valid) {
+    if (row_valid && half == 0) {
         if (a.num_splits == 1) {
             const float4 lv = make_float4(lse_v, lse_v, lse_v, lse_v);
             *reinterpret_cast<float4 *>(a.lse + qrow * 8 + 4 * hh) = lv;
@@ -338,11 +372,15 @@ __device__ __forceinline__ void stage1_wide_body(const Stage1Args &a, CK_LDS cha
     }
     float *base = a.num_splits == 1 ? a.out : a.part_o + (int64_t)sp * a.num_rows * kD;
     const int chunk = lane & 31;
+    if (HALVES == 2) bar.sync();  // both sets' slabs are in; each set writes half the rows
+    const CK_LDS float *slab2 = (const CK_LDS float *)(smem + (1 - half) * SLOTS * kWStage) + wid * (32 * kD);
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
+    for (int j0 = 0; j0 < 16 / HALVES; ++j0) {
+        const int j = j0 + half * (16 / HALVES);
         const int rr = 2 * j + (lane >> 5);
         const int64_t qr = __shfl((int)qrow, rr);
-        const f32x4 o = *reinterpret_cast<const CK_LDS f32x4 *>(slab + rr * kD + ((chunk ^ rr) * 4));
+        f32x4 o = *reinterpret_cast<const CK_LDS f32x4 *>(slab + rr * kD + ((chunk ^ rr) * 4));
+        if constexpr (HALVES == 2) o += *reinterpret_cast<const CK_LDS f32x4 *>(slab2 + rr * kD + ((chunk ^ rr) * 4));
         // non-temporal: read once, by another kernel (combine, cascade epilogue)
         if (wrow0 + rr < rows_b) __builtin_nontemporal_store(o, reinterpret_cast<f32x4 *>(base + qr * kD + chunk * 4));
     }
