@@ -368,9 +368,9 @@ def test_decode_form(case):
     B = len(kvs)
     inp = paged_inputs(B, kvs, H, KVH, seed=17, q_len=1, permute=True, block_cols=max(8, (max(kvs) + 127) // 128))
     out, lse = _run(inp, 1)
-    # P enters as two bf16 terms within 2^-16 of fp32 P, so O is within 2^-16 max|V| (about
-    # 8e-5) of exact attention plus the fp32 sums' rounding. (The bf16-P oracle itself is
-    # up to 2^-9 max|V| from exact on the shortest requests.)
+    # P holds fp32 (three bf16 terms), so O is within 2^-16 max|V| (about 8e-5) of exact
+    # attention with room to spare. (The bf16-P oracle itself is up to 2^-9 max|V| from
+    # exact on the shortest requests.)
     o_ref, l_ref = A.stage1(inp["q"], inp["k"], inp["v"], inp["block_table"], np.ones(B, dtype=np.int64),
                             inp["kv_seqlens"], quantize_p=False)
     assert np.abs(out - o_ref).max() <= 2.0 ** -16 * np.abs(inp["v"]).max() + 2e-5

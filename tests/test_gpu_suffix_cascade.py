@@ -448,3 +448,72 @@ def test_fused_above_4_heads(B, H, KVH, P, no_wait_giveups):
         assert np.all(err <= 2e-3 + 2.0 ** -8 * np.abs(Od)), (b, err.max())
         rel = np.abs(lse.reshape(B, H)[b] - Ld[0]) / np.maximum(np.abs(Ld[0]), 1.0)
         assert rel.max() <= 1e-4, (b, rel.max())
+
+
+# Fused cascades of 1 to 8 heads per group and (two groups) 16 per kv head; prefix work
+# above 2^26, where the suffix stream is a kernel of its own; the stand-alone op.
+INF_CASES = [("fused_g1", 5, 8, 8, 256), ("fused_g4", 7, 32, 8, 384), ("fused_g5", 7, 40, 8, 384),
+             ("fused_g8", 7, 64, 8, 1500), ("fused_gqa16", 5, 64, 4, 256), ("serial_g8", 65, 64, 8, 16384),
+             ("suffix_g4", 7, 32, 8, None), ("suffix_g7", 7, 14, 2, None)]
+
+
+@pytest.mark.parametrize("case", INF_CASES, ids=[c[0] for c in INF_CASES])
+def test_infinite_suffix_values(case):
+    """An infinite suffix V element reaches its own dim of the heads that read it as an
+    infinity of the same sign (p > 0 of every token); every other output is finite."""
+    _, B, H, KVH, P = case
+    suf = np.r_[[700, 33, 129, 8, 1200], np.full(B, 40)][:B].astype(np.int64)
+    q16, k16, v16, bt_pre, bt_suf, suf = _cascade_inputs(B, H, KVH, P or 128, suf, seed=B)
+    v16 = v16.copy()
+    want = {}
+    for b, tok, g, d, val in [(0, 0, 0, 5, np.inf), (0, 699, KVH - 1, 127, -np.inf), (1, 32, 1, 0, np.inf),
+                              (2, 128, KVH - 1, 64, np.inf), (3, 7, 0, 16, -np.inf), (4, 555, 0, 100, np.inf),
+                              (4, 31, 0, 101, -np.inf)]:
+        v16[bt_suf[b, tok // 128], tok % 128, g, d] = 0x7F80 if val > 0 else 0xFF80
+        want[b, g, d] = val
+    q, k, v = (torch_bf16(x, DEV) for x in (q16, k16, v16))
+    if P is None:
+        out, lse = torch.ops.npu.suffix_decode(q, k, v, torch.from_numpy(bt_suf).to(DEV), torch.from_numpy(suf).to(DEV))
+        got, lse = bf16_to_np(out), lse.cpu().numpy()
+    else:
+        got, lse = _cascade_run(True, B, P, q, k, v, bt_pre, bt_suf, suf)
+    got = got.reshape(B, KVH, H // KVH, 128).copy()
+    for (b, g, d), val in want.items():
+        assert (got[b, g, :, d] == val).all(), (b, g, d, got[b, g, :, d])
+        got[b, g, :, d] = 0
+    assert np.isfinite(got).all() and np.isfinite(lse).all()
+
+
+@pytest.mark.parametrize("H,KVH", [(5, 1), (40, 8), (24, 4), (14, 2), (64, 8)])
+def test_fused_above_4_heads_full_precision_p(H, KVH):
+    """Two-token suffixes whose values cancel to about 2^-8 for one head per group: P's own
+    error then stands at 2^8 times its size in O. P holds fp32 (its terms sum to p
+    within 2^-24 p); the fp32 scores and exp2 add a few 2^-23, so |error| <= half a
+    bf16 ulp of O + 2^-19 (p1 |v1| + p2 |v2|). Two bf16 terms (2^-16 p) exceed it."""
+    B, D = 96, 128
+    rng = np.random.default_rng(H)
+    suf = np.full(B, 2, dtype=np.int64)
+    q16, k16, v16, bt_pre, bt_suf, suf = _cascade_inputs(B, H, KVH, 0, suf, seed=H)
+    q = bits_to_f32(q16).astype(np.float64)
+    kf = bits_to_f32(k16).astype(np.float64)
+    v16 = v16.copy()
+    G = H // KVH
+    pages = bt_suf[:, 0]
+    ks = kf[pages][:, :2]                                            # [B, 2, KVH, D]
+    s = np.einsum("bghd,btgd->bght", q.reshape(B, KVH, G, D), ks) / np.sqrt(D)
+    p = np.exp(s - s.max(axis=-1, keepdims=True))
+    p /= p.sum(axis=-1, keepdims=True)                                # [B, KVH, G, 2]
+    h0 = rng.integers(0, G, size=(B, KVH))
+    p0 = np.take_along_axis(p, h0[..., None, None], axis=2)[:, :, 0]  # [B, KVH, 2]
+    v1 = bits_to_f32(bf16_bits(rng.uniform(64, 128, size=(B, KVH, D)).astype(np.float32)))
+    v2 = -v1 * (p0[..., :1] / p0[..., 1:]).astype(np.float32)
+    v2 = bits_to_f32(bf16_bits(v2.astype(np.float32)))
+    v16[pages, 0], v16[pages, 1] = bf16_bits(v1), bf16_bits(v2)
+    qd, kd, vd = (torch_bf16(x, DEV) for x in (q16, k16, v16))
+    got, _ = _cascade_run(True, B, 0, qd, kd, vd, bt_pre, bt_suf, suf)
+    got = got.reshape(B, KVH, G, D).astype(np.float64)
+    vv = np.stack([v1, v2], axis=2).astype(np.float64)                # [B, KVH, 2, D]
+    ref = np.einsum("bght,bgtd->bghd", p, vv)
+    mag = np.einsum("bght,bgtd->bghd", p, np.abs(vv))
+    excess = float(((np.abs(got - ref) - 2.0 ** -8 * np.abs(ref)) / mag).max())
+    assert excess <= 2.0 ** -19

@@ -247,9 +247,32 @@ __device__ __forceinline__ float sum_xor16(float x) {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+// x in lanes 0-31, y of lane - 32 in lanes 32-63
+__device__ __forceinline__ float swap_halves(float x, float y) {
+    return __uint_as_float(
+        __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false)[0]);
+}
 __device__ __forceinline__ float sum_xor32(float x) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// bf16 terms of a probability (p >= 0): two values truncated to bf16 in one register;
+// p - hi, at least min(p, 2^-100) (the median of three is max(p - hi, min(p, c)), as
+// p - hi <= p); and r - mid plus 2^-23 r, positive with r and exact in the bits of r
+// that truncation to bf16 keeps
+__device__ __forceinline__ uint32_t term_hi(float p0, float p1) {
+    return __builtin_amdgcn_perm(__float_as_uint(p1), __float_as_uint(p0), 0x07060302u);
+}
+__device__ __forceinline__ float trunc_bf16(float p) { return __uint_as_float(__float_as_uint(p) & 0xFFFF0000u); }
+__device__ __forceinline__ float term_rest(float p) {
+    return __builtin_amdgcn_fmed3f(p - trunc_bf16(p), p, 0x1p-100f);
+}
+__device__ __forceinline__ float term_rest2(float r) { return __builtin_fmaf(r, 1.0f + 0x1p-23f, -trunc_bf16(r)); }
+// both bf16 values (>= 0) halved through their exponents; zero stays zero
+__device__ __forceinline__ uint32_t halve_bf16x2(uint32_t x) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, x), u16x2{0x80, 0x80}));
 }
 
 __device__ __forceinline__ int64_t clamp_len(const SuffixArgs &a, int64_t kvl) {
@@ -277,12 +300,17 @@ __device__ __forceinline__ void write_f32_row(const SuffixArgs &a, int64_t row, 
 //   from global memory; B = q of head n, the same dims. The result puts token
 //   4 g + r, head n in register r of lane (g, n); lanes of rows 8-15 (g >= 2) and
 //   of heads n >= G get score -inf through the scale's addend, hence p = 0.
-// * O^T += V^T P^T on v_mfma_f32_16x16x16_bf16, one 16-dim tile of O per MFMA: B =
-//   P^T is the score layout itself (lane (g, n): tokens 4 g .. 4 g + 3 of head n),
-//   and A = V^T comes from the V rows through the wave's LDS slot by
-//   ds_read_b64_tr_b16 (lane (g, n): dim n of the tile, tokens 4 g .. 4 g + 3).
-//   P enters as two bf16 terms, hi = p truncated and lo = p - hi rounded (|p - hi|
-//   < 2^-7 p, so p = hi + lo within 2^-16 p): fp32 P for the arithmetic's purposes.
+// * O^T += V^T P^T on v_mfma_f32_16x16x16_bf16, 16-dim tiles of O: B = P^T is the
+//   score layout itself (lane (g, n): tokens 4 g .. 4 g + 3 of head n), and A = V^T
+//   comes from the V rows through the wave's LDS slot by ds_read_b64_tr_b16 (lane
+//   (g, n): dim n of the tile, tokens 4 (g % 2) .. + 3). The operand's rows 8-15 are
+//   the same 8 tokens again and carry another term of P. P enters as bf16 terms: hi
+//   = p truncated and lo = p - hi rounded (|p - hi| < 2^-7 p, so p = hi + lo within
+//   2^-16 p), one MFMA per tile; with EXACTP three truncated terms, which hold all
+//   24 bits of p, two MFMAs per tile.
+// * Every term is positive where p is (p - hi is taken as at least min(p, 2^-100), far
+//   below the row sum, which is at least 1), so an infinite V element stays infinite:
+//   a zero term, or a zero row beside it in the operand, would make NaN of it.
 // * The softmax state of head n sits in lane (g, n), the same for every g: the
 //   running max is reduced over the 4 groups when it moves, the row sum when the
 //   segment closes, and O^T needs no reduction (the MFMA summed the tokens).
@@ -296,7 +324,7 @@ __device__ __forceinline__ void write_f32_row(const SuffixArgs &a, int64_t row, 
 // body's LDS) skips its own, waits until scan_flag is set and reads the other's
 // lengths and window prefix sums; the body given only scan_flag sets it once its
 // scan is complete.
-template <int G, int NW, int D, bool F32 = false, class L = SfxLds<G, NW>, class Bar>
+template <int G, int NW, int D, bool F32, bool EXACTP, class L = SfxLds<G, NW>, class Bar>
 __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS char *smem, int lb, int tid,
                                                    const Bar &bar, CK_LDS int *scan_flag = nullptr,
                                                    const CK_LDS char *scan_src = nullptr) {
@@ -431,11 +459,12 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     // the O^T tiles (dims 16 T + 4 mg + r of head mn), head mn's
     // softmax state (m; m + kTau, the rescale trigger; the exponent offset, m or
     // 0 while m = -inf; this lane's share of the row sum), q fragments, and the
-    // P^T operand (hi, lo) of the pending window
+    // P^T operands of the pending window (one per MFMA of a tile)
     f32x4 oacc[8];
     float m1, mt1, mz1, l1;
     u32x4 qf[4];
-    uint32_t ph[2], pl[2];
+    constexpr int kPv = EXACTP ? 2 : 1;
+    uint32_t pb[kPv][2];
     int nclose = 0;  // segments closed so far (exchange ring position)
     int qslot = 0;   // segment of the current phase
     u32x4 kbuf[NB][4];
@@ -609,12 +638,8 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     int eypend = 0;  // packed table fields of window n - 1 (token-major)
     // Token-major values of the pending window: its V rows (lane (t, c) holds 32
     // bytes of token t) into the wave's LDS slot, back as the V^T fragments of the 8
-    // dim tiles, then O^T += V^T P^T for the hi and the lo term of P. The slot is
-    // written and read by this wave only, whose LDS operations run in issue order.
-    // F32 zeroes the V^T fragments of the operand's token rows 8-15 (copies of rows
-    // 0-7 whose P is 0): stage-1 keeps an infinite V element infinite, and inf * 0
-    // is NaN.
-    const uint32_t vmask = mg < 2 ? 0xFFFFFFFFu : 0u;
+    // dim tiles, then O^T += V^T P^T over the terms of P. The slot is written and read
+    // by this wave only, whose LDS operations run in issue order.
     typedef short s16x4 __attribute__((ext_vector_type(4)));
     auto pv_tok = [&](const VSlot &vv) __attribute__((always_inline)) {
         *reinterpret_cast<CK_LDS u32x4 *>(vt + vwo) = vv[0];
@@ -622,18 +647,13 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         uint2 vtf[8];
 #pragma unroll
         for (int T = 0; T < 8; ++T) vtf[T] = lds_read_tr16(vt + vro + 32 * T);
-        const s16x4 bh = __builtin_bit_cast(s16x4, uint2{ph[0], ph[1]});
-        const s16x4 bl = __builtin_bit_cast(s16x4, uint2{pl[0], pl[1]});
 #pragma unroll
-        for (int T = 0; T < 8; ++T) {
-            if constexpr (F32) {
-                vtf[T].x &= vmask;
-                vtf[T].y &= vmask;
-            }
-            const s16x4 av = __builtin_bit_cast(s16x4, vtf[T]);
-            oacc[T] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bh, oacc[T], 0, 0, 0);
-            oacc[T] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bl, oacc[T], 0, 0, 0);
-        }
+        for (int T = 0; T < 8; ++T)
+#pragma unroll
+            for (int i = 0; i < kPv; ++i)
+                oacc[T] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                    __builtin_bit_cast(s16x4, vtf[T]), __builtin_bit_cast(s16x4, uint2{pb[i][0], pb[i][1]}), oacc[T], 0,
+                    0, 0);
     };
     // Token-major window step, pipelined by one window: step n issues the K rows of
     // window n + D, computes the scores of window n and the values of window n - 1
@@ -706,20 +726,26 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
             s[r] = exp2_fast(s[r] - mz1);  // 0 for masked tokens and padding lanes
             l1 += s[r];
         }
-        // P^T of window n for the next step: hi = p truncated to bf16 (exact in fp32),
-        // lo = p - hi (exact) rounded to bf16. F32: lo is at least 2^-40 p, so that it is
-        // 0 only where p is (an infinite V element times a zero lo would be NaN).
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const float p0 = s[2 * i], p1 = s[2 * i + 1];
-            const uint32_t u0 = __float_as_uint(p0), u1 = __float_as_uint(p1);
-            ph[i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
-            float lo0 = p0 - __uint_as_float(u0 & 0xFFFF0000u), lo1 = p1 - __uint_as_float(u1 & 0xFFFF0000u);
-            if constexpr (F32) {
-                lo0 = fmaxf(lo0, p0 * 0x1p-40f);
-                lo1 = fmaxf(lo1, p1 * 0x1p-40f);
+        // P^T of window n for the next step: hi = p truncated to bf16 (exact in fp32), the
+        // rest rounded to bf16; EXACTP truncates the rest too and takes what remains as
+        // the third term. Only lanes 0-31 hold probabilities: lanes 32-63 take tokens
+        // 2, 3 of lane - 32 for the arithmetic, and one swap of two terms then puts
+        // the first in lanes 0-31 (rows 0-7) and the second in lanes 32-63 (rows 8-15)
+        // of both operand registers. The third fills both, half of it in each.
+        {
+            const float p0 = swap_halves(s[0], s[2]), p1 = swap_halves(s[1], s[3]);
+            const float r0 = term_rest(p0), r1 = term_rest(p1);
+            const uint32_t hi = term_hi(p0, p1);
+            const uint32_t mid = EXACTP ? term_hi(r0, r1) : pack_bf16x2(r0, r1);
+            const auto b0 = __builtin_amdgcn_permlane32_swap(hi, mid, false, false);
+            pb[0][0] = b0[0];
+            pb[0][1] = b0[1];
+            if constexpr (EXACTP) {
+                const uint32_t lo = halve_bf16x2(term_hi(term_rest2(r0), term_rest2(r1)));
+                const auto b1 = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+                pb[1][0] = b1[0];
+                pb[1][1] = b1[1];
             }
-            pl[i] = pack_bf16x2(lo0, lo1);
         }
     };
     // after a phase's last window (np - 1, in slot (np - 1) % NB): its values and
@@ -811,7 +837,8 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         enext = tab[D];
         // "window -1" of the pipelined step (slot NB - 1): no values, no close;
         // its V slot is zeroed so that p = 0 times it stays 0
-        ph[0] = ph[1] = pl[0] = pl[1] = 0u;
+#pragma unroll
+        for (int i = 0; i < kPv; ++i) pb[i][0] = pb[i][1] = 0u;
         vbuf[NB - 1][0] = u32x4{0u, 0u, 0u, 0u};
         vbuf[NB - 1][1] = u32x4{0u, 0u, 0u, 0u};
         eypend = 0;
@@ -853,8 +880,8 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
 template <int G, bool F32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void suffix_stream_kernel(SuffixArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    suffix_stream_body<G, 4, (G > 4 ? 1 : kTokDepth), F32>(a, (CK_LDS char *)smem_raw, blockIdx.x, threadIdx.x,
-                                                           WgBarrier{});
+    suffix_stream_body<G, 4, (G > 4 ? 1 : kTokDepth), F32, F32>(a, (CK_LDS char *)smem_raw, blockIdx.x, threadIdx.x,
+                                                                WgBarrier{});
 }
 static_assert(SfxLds<5, 4>::kBytes <= 80 * 1024, "two stand-alone workgroups per CU up to 5 heads");
 static_assert(SfxLds<kMaxGroup, 4>::kBytes <= 160 * 1024, "one above");
@@ -1153,7 +1180,7 @@ __global__ __launch_bounds__(512) void cascade_fused_kernel(s1::Stage1Args s1a, 
         constexpr int kRoleRot = 3;
         const int g = ((int)blockIdx.x + kRoleRot) % sa.kv_heads, j = (int)blockIdx.x / sa.kv_heads;
         // the streaming waves scan the lengths; the stage-1 waves reuse that scan
-        suffix_stream_body<G, 4, kTokDepth, false, FusedSfx<G>>(
+        suffix_stream_body<G, 4, kTokDepth, false, (G > 4), FusedSfx<G>>(
             sa, smem + (role ? 0 : kFusedS1Lds), (2 * j + role) * sa.kv_heads + g, threadIdx.x & 255, bar, bars + 4,
             role ? smem + kFusedS1Lds : nullptr);
     }
