@@ -83,6 +83,54 @@ def test_precision(mode, dtype, name, shape, has_beta):
         assert y.numel() == 0
 
 
+def _y(x, gamma, beta, eps):
+    _, _, y = torch.ops.npu.add_rms_norm_stats(x.to(DEV), x.to(DEV), gamma.to(DEV), beta.to(DEV), eps, 1)
+    return y.cpu().view(torch.int16).numpy()
+
+
+def _bits(y64, dt):
+    """bit patterns of the oracle's y (dtype values in fp64; torch's cast keeps -0)"""
+    return torch.from_numpy(y64).to(dt).view(torch.int16).numpy()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+def test_signed_zeros(dtype):
+    """x = -0 gives m = -0, and m * gamma + beta its IEEE sign."""
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    x = torch.zeros(4, 64).to(dt)
+    x[:, 1::2] = -0.0
+    x[1:, :8] = 1.5
+    gamma = torch.ones(64).to(dt)
+    gamma[::4] = -1.0
+    gamma[2::4] = -0.0
+    beta = torch.zeros(64).to(dt)
+    beta[:48] = -0.0
+    want = ref_op(x.double().numpy(), None, gamma.double().numpy(), beta.double().numpy(), EPS, 1, dtype)[2]
+    assert np.array_equal(_y(x, gamma, beta, EPS), _bits(want, dt))
+
+
+@pytest.mark.parametrize("dtype,keep", [("bf16", 8), ("fp16", 11)])
+def test_products_at_rounding_ties(dtype, keep):
+    """x * rstd within 2^-49 of the fp32 midpoint beside a dtype tie, on either side (eps
+    sets rstd to the last fp64 bit): the two roundings must see the fp64 product."""
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    x = torch.full((8, 16), 0.25).to(dt)
+    x[:, 0], x[:, 1] = 1.0, -1.0
+    mean = float((x[0].double() ** 2).mean())
+    gamma, beta = torch.ones(16).to(dt), torch.zeros(16).to(dt)
+    seen = 0
+    for side in (-1.0, 1.0):
+        target = 1.0 + 2.0 ** -keep + side * 2.0 ** -24
+        base = 1.0 / target ** 2 - mean
+        for j in range(-12, 13):
+            eps = base + j * 2.0 ** -53
+            rstd = 1.0 / np.sqrt(mean + eps)
+            seen += abs(rstd - target) <= 2.0 ** -49 and rstd != target
+            want = ref_op(x.double().numpy(), None, gamma.double().numpy(), beta.double().numpy(), eps, 1, dtype)[2]
+            assert np.array_equal(_y(x, gamma, beta, eps), _bits(want, dt)), (side, j)
+    assert seen >= 8
+
+
 def test_mode1_ignores_x2_and_matches_mode0_stats():
     x1, x2, gamma, beta = (t.to(DEV) for t in make_inputs(64, 1024, "bf16", 3, has_beta=True))
     xo, r0, _ = torch.ops.npu.add_rms_norm_stats(x1, x2, gamma, beta, EPS, 0)

@@ -15,10 +15,16 @@
 // mean, sqrt and the reciprocal run in fp64 (each
 // square of a 16-bit value is exact in fp32 and 5120 of them sum in fp64 with a
 // relative error below 1e-12), and every rd() is fp64 -> fp32 -> dtype, both
-// RNE. The apply takes the same values from fp32 operations: x * rstd with rstd
-// as two floats (mul_split), and m * gamma + beta as one fma, which rounds the
-// exact sum once (the product of two 16-bit values is exact in fp64 and in an
-// fma alike). x1 + x2 of two 16-bit values is exact in fp32 up to a 16-binade gap
+// RNE. The apply gives the same bits from fp32 operations:
+// * m = rd(x * rstd) is monotone in rstd, every step of it (the fp64 product, both
+//   roundings). With floats rlo <= rstd <= rhi, whose products with a 16-bit x are
+//   exact in fp64, rd(x * rlo) == rd(x * rhi) therefore is m. Where they differ (a
+//   dtype tie between them: about 2 in 2^16 bf16 and 2 in 2^13 fp16 elements), the
+//   wave computes those 512 elements in fp64.
+// * m * gamma + beta is one fma: the product (at most 22 bits) is exact in fp64, and
+//   so is the sum, or its smaller part lies below 2^-30 of the larger and changes
+//   neither fp32 rounding.
+// x1 + x2 of two 16-bit values is exact in fp32 up to a 16-binade gap
 // and otherwise lands far from a dtype tie, so rd(x1 + x2) is computed from
 // the fp32 sum. rstd is returned as fp32 (RNE of the fp64 value).
 //
@@ -28,14 +34,13 @@
 // returns zeros past its end, so there is no branch and all of a wave's loads
 // are in flight together) and kept in registers between the statistics pass
 // and the write pass, so every input byte is read once.
-// 2048 x 5120 bf16, traced: mode 0 12.1 us (62.9 MB, 5.2 TB/s), mode 1 10.6 us
-// (42 MB; 11.9 us with the apply in fp64, whose conversions and products held
-// the stores back).
+// 2048 x 5120 bf16, traced: mode 0 13.5 us (62.9 MB, 4.7 TB/s), mode 1 10.9 us (42 MB).
+// Residual add + norm, the apply in fp64 / as it is: 23.3 / 21.8 us, in fp16 with beta
+// 24.8 / 22.8 (the fp64 conversions and products held the stores back).
 // Four rows per 256-thread workgroup; the grid also covers the padding rows
 // of rstd (ceil(M / 8) * 8 rows, the reference's 32-byte output groups,
 // op_host/add_rms_norm_stats.cpp:111-113), which are written 0.
 #include <cmath>
-#include <type_traits>
 
 #include "ck_common.h"
 
@@ -92,31 +97,12 @@ __device__ __forceinline__ float to_f32_opaque(double x) {
     asm volatile("" : "+v"(f));
     return f;
 }
-// rd() of an fp64 value as the reference casts it: fp64 -> fp32 -> dtype
-template <bool kBf16>
-__device__ __forceinline__ float rd64(double x) {
-    const float f = to_f32_opaque(x);
-    if constexpr (kBf16) return bf16_lo(pack_bf16x2(f, 0.f));
-    else return (float)(_Float16)f;
-}
-
 // fp32 kept opaque likewise in fp16: LLVM folds an fp32 fma or add and its fp16
 // conversion into one v_fma_mixlo_f16, which rounds once.
 template <bool kBf16>
 __device__ __forceinline__ float rounded_f32(float f) {
     if constexpr (!kBf16) asm("" : "+v"(f));
     return f;
-}
-
-// RNE fp32 of x * (rh + rl): the product with rh as the exact pair p + e (fma),
-// the product with rl and e folded in before the one rounding that counts. Within
-// 2^-48 of the fp64 product before that rounding, at 4 fp32 operations instead of
-// two conversions and an fp64 multiply. No contraction: p must be the rounded product.
-__device__ __forceinline__ float mul_split(float x, float rh, float rl) {
-#pragma clang fp contract(off)
-    const float p = x * rh;
-    const float e = __builtin_fmaf(x, rh, -p);
-    return p + __builtin_fmaf(x, rl, e);
 }
 
 // Buffer resource over `bytes` bytes at p: loads past the end return 0 and
@@ -199,42 +185,43 @@ __global__ __launch_bounds__(kRowsPerBlock * kWave) void add_rms_norm_kernel(Nor
         u32x4 gw[kMaxChunks];
 #pragma unroll
         for (int i = 0; i < kMaxChunks; ++i) gw[i] = bload(rg, (lane + kWave * i) * 16);
-        // rstd as two floats (rh + rl = rstd within 2^-48): fits whenever rstd is
-        // far from fp32's limits, a wave-uniform test (eps below 1e-36 on a
-        // near-zero row, or a row with an infinity or NaN, take the fp64 form)
-        const float rh = (float)rstd;
-        const float rl = (float)(rstd - (double)rh);
-        const bool fits = rstd > 0x1p-60 && rstd < 0x1p+60;
+        // the floats around rstd; outside fp32's normal range (an infinity or NaN in the
+        // row, or eps and the row near zero) every chunk takes the fp64 product
+        const bool fits = rstd > 0x1p-100 && rstd < 0x1p+100;
+        const float rn = (float)rstd;
+        const bool below = (double)rn < rstd;
+        const float rlo = below ? rn : __uint_as_float(__float_as_uint(rn) - 1);
+        const float rhi = below ? __uint_as_float(__float_as_uint(rn) + 1) : rn;
         // one chunk at a time (the fences keep the temporaries of one chunk live at
         // once, so the kernel keeps 4 waves per SIMD)
-        auto apply = [&](auto split) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < kMaxChunks; ++i) {
-                const int off = (lane + kWave * i) * 16;
-                const u32x4 bw = kBeta ? bload(rb, off) : u32x4{0, 0, 0, 0};
-                u32x4 out;
+        for (int i = 0; i < kMaxChunks; ++i) {
+            const int off = (lane + kWave * i) * 16;
+            const u32x4 bw = kBeta ? bload(rb, off) : u32x4{0, 0, 0, 0};
+            u32x4 m;
+            uint32_t differ = fits ? 0u : 1u;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float x0 = lo16<kBf16>(xo[i][e]), x1 = hi16<kBf16>(xo[i][e]);
-                    if constexpr (decltype(split)::value) {
-                        const uint32_t m = pack16<kBf16>(rounded_f32<kBf16>(mul_split(x0, rh, rl)),
-                                                         rounded_f32<kBf16>(mul_split(x1, rh, rl)));
-                        const float y0 = fmaf(lo16<kBf16>(m), lo16<kBf16>(gw[i][e]), lo16<kBf16>(bw[e]));
-                        const float y1 = fmaf(hi16<kBf16>(m), hi16<kBf16>(gw[i][e]), hi16<kBf16>(bw[e]));
-                        out[e] = pack16<kBf16>(rounded_f32<kBf16>(y0), rounded_f32<kBf16>(y1));
-                    } else {
-                        const double m0 = rd64<kBf16>((double)x0 * rstd), m1 = rd64<kBf16>((double)x1 * rstd);
-                        const double y0 = m0 * (double)lo16<kBf16>(gw[i][e]) + (double)lo16<kBf16>(bw[e]);
-                        const double y1 = m1 * (double)hi16<kBf16>(gw[i][e]) + (double)hi16<kBf16>(bw[e]);
-                        out[e] = pack16<kBf16>(to_f32_opaque(y0), to_f32_opaque(y1));
-                    }
-                }
-                bstore(ry, off, out);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int e = 0; e < 4; ++e) {
+                const float x0 = lo16<kBf16>(xo[i][e]), x1 = hi16<kBf16>(xo[i][e]);
+                m[e] = pack16<kBf16>(rounded_f32<kBf16>(x0 * rlo), rounded_f32<kBf16>(x1 * rlo));
+                differ |= m[e] ^ pack16<kBf16>(rounded_f32<kBf16>(x0 * rhi), rounded_f32<kBf16>(x1 * rhi));
             }
-        };
-        if (fits) apply(std::true_type{});
-        else apply(std::false_type{});
+            if (__builtin_amdgcn_ballot_w64(differ != 0)) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    m[e] = pack16<kBf16>(to_f32_opaque((double)lo16<kBf16>(xo[i][e]) * rstd),
+                                         to_f32_opaque((double)hi16<kBf16>(xo[i][e]) * rstd));
+            }
+            u32x4 out;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float y0 = fmaf(lo16<kBf16>(m[e]), lo16<kBf16>(gw[i][e]), lo16<kBf16>(bw[e]));
+                const float y1 = fmaf(hi16<kBf16>(m[e]), hi16<kBf16>(gw[i][e]), hi16<kBf16>(bw[e]));
+                out[e] = pack16<kBf16>(rounded_f32<kBf16>(y0), rounded_f32<kBf16>(y1));
+            }
+            bstore(ry, off, out);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
 }
 
