@@ -115,10 +115,6 @@ int ck_lse_merge(const void *o1, int o1_dtype, const void *o2, int o2_dtype,
  * P = exp(S - rowmax) is rounded to bf16 (RNE) before the PV product and the
  * row sums use the unrounded fp32 values, as
  * third_party/catlass/.../block_epilogue_online_softmax_no_mask.hpp:487-594 does.
- * With one query token per request (q_len_uniform == 1), kv_cap >= 1024, the
- * plan's split count and a workspace of at least ck_suffix_decode_plan's bytes
- * too, the requests are streamed as ck_suffix_decode does, with P at fp32
- * precision.
  * Replaces OPS/fa_fp32_stage1/op_kernel/kernel_fa_fp32_stage1.cpp:848-863.
  * ========================================================================== */
 int ck_fa_fp32_stage1_plan(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_heads,
@@ -132,6 +128,26 @@ int ck_fa_fp32_stage1(const void *q, const void *k, const void *v, const int32_t
                       int64_t head_dim, int64_t num_blocks, int64_t block_size, float scale,
                       int64_t kv_cap, int64_t num_splits, float *out, float *lse,
                       void *workspace, int64_t workspace_bytes, void *stream);
+
+/* ============================================================================
+ * Stage 1 with one query token per request, streamed by the kernels of
+ * ck_suffix_decode: the results of ck_fa_fp32_stage1 with q_len_uniform == 1, but P
+ * keeps fp32 in the PV product (three bf16 terms per value) instead of bf16.
+ * Arguments as there (q bf16 [batch, num_heads, 128], out and lse laid out alike).
+ *   *preferred       1 where this is the faster of the two forms (the torch op then
+ *                    runs it), else 0; the call accepts either
+ *   *workspace_bytes of ck_fa_fp32_stage1_decode (CK_E_WORKSPACE for less)
+ * batch is at most 1024 and batch * kv_cap below 2^31, num_heads at most 65536
+ * (CK_E_UNSUPPORTED otherwise). No counterpart in the reference.
+ * ========================================================================== */
+int ck_fa_fp32_stage1_decode_plan(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t head_dim,
+                                  int64_t kv_cap, int64_t *preferred, int64_t *workspace_bytes);
+
+int ck_fa_fp32_stage1_decode(const void *q, const void *k, const void *v, const int32_t *block_table,
+                             int64_t bt_cols, const int64_t *kv_seqlens, int64_t batch, int64_t num_heads,
+                             int64_t kv_heads, int64_t head_dim, int64_t num_blocks, int64_t block_size,
+                             float scale, int64_t kv_cap, float *out, float *lse, void *workspace,
+                             int64_t workspace_bytes, void *stream);
 
 /* ============================================================================
  * Per-sequence paged decode attention over each sequence's own suffix
@@ -272,7 +288,7 @@ int ck_add_rms_norm_stats(const void *x1, const void *x2, const void *gamma, con
 /* ============================================================================
  * Health counter of the bounded waits inside the suffix and fused cascade
  * kernels (ck_suffix_decode, ck_cascade_decode, ck_cascade_decode_noalloc, and
- * ck_fa_fp32_stage1 with one query token per request).
+ * ck_fa_fp32_stage1_decode).
  * Their waves wait on each other only through LDS counters whose waits are
  * bounded (a hang is never possible); a wait that runs out means a broken
  * invariant and wrong results, and is counted on the device. *count receives

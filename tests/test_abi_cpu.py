@@ -173,3 +173,32 @@ def test_add_rms_norm_validation_without_launch():
     odd = ctypes.c_void_p(24)
     assert L.ck_add_rms_norm_stats(odd, p, p, None, p, p, p, 4, 64, bf16, 0, 1e-6, None) == -1  # x1 alignment
     assert L.ck_add_rms_norm_stats(p, p, odd, None, p, p, p, 4, 64, bf16, 1, 1e-6, None) == -1  # gamma alignment
+
+
+def test_stage1_decode_plan_and_validation():
+    L = abi.lib()
+    preferred, w = abi.stage1_decode_plan(64, 32, 8, 128, 8192)
+    assert preferred and w >= abi.suffix_plan(64, 32, 8, 128, 8192)[1]
+    assert not abi.stage1_decode_plan(64, 32, 8, 128, 128)[0]       # one page: the tiles
+    assert abi.stage1_decode_plan(0, 32, 8, 128, 8192) == (False, 0)
+    out = ctypes.c_int64(0)
+    r = ctypes.byref(out)
+    assert L.ck_fa_fp32_stage1_decode_plan(1025, 32, 8, 128, 1024, r, r) == -4       # one launch group
+    assert L.ck_fa_fp32_stage1_decode_plan(4, 32, 8, 128, 1 << 30, r, r) == -4       # batch * kv_cap < 2^31
+    assert L.ck_fa_fp32_stage1_decode_plan(1, 1 << 17, 1 << 14, 128, 1024, r, r) == -4
+    assert L.ck_fa_fp32_stage1_decode_plan(1, 30, 8, 128, 1024, r, r) == -1          # H % KVH
+    assert L.ck_fa_fp32_stage1_decode_plan(1, 32, 8, 64, 1024, r, r) == -4           # D != 128
+    assert L.ck_fa_fp32_stage1_decode_plan(1, 32, 8, 128, 1024, None, r) == -2
+    p = ctypes.c_void_p(16)  # never dereferenced: every call below fails validation first
+
+    def call(batch=4, cols=8, block=128, scale=0.1, cap=1024, q=p, lse=p, ws=p, wsb=1 << 30):
+        return L.ck_fa_fp32_stage1_decode(q, p, p, p, cols, p, batch, 32, 8, 128, 1, block, scale, cap, p, lse, ws, wsb,
+                                          None)
+    assert call(block=64) == -4
+    assert call(cap=1025) == -1                     # kv bound beyond the table
+    assert call(scale=float("nan")) == -1 and call(scale=0.0) == -1
+    assert call(q=None) == -2
+    assert call(lse=ctypes.c_void_p(24)) == -1 and call(ws=ctypes.c_void_p(24)) == -1
+    need = abi.stage1_decode_plan(4, 32, 8, 128, 1024)[1]
+    assert call(wsb=need - 1) == -3 and call(ws=None) == -3
+    assert call(batch=0) == 0

@@ -397,6 +397,44 @@ def test_decode_form(case):
     _check(inp, o3.cpu().numpy(), l3.cpu().numpy(), H, name + " tiles")
 
 
+@pytest.mark.parametrize("kvs,H,KVH", [([1024, 700], 16, 4), ([1100, 5, 2048], 32, 8)])
+def test_one_token_forms_by_entry_point(kvs, H, KVH):
+    """One query token per request: ck_fa_fp32_stage1 runs the tiles with bf16 P whatever the
+    size of the workspace, ck_fa_fp32_stage1_decode is what the torch op runs here."""
+    from cascade_amd import abi
+    B = len(kvs)
+    inp = paged_inputs(B, kvs, H, KVH, seed=5, q_len=1, permute=True)
+    q, k, v, bt, qs, kl = _dev(inp)
+    cap = bt.shape[1] * 128
+    scale, st = float(np.float32(1 / np.sqrt(128))), torch.cuda.current_stream().cuda_stream
+    preferred, dec_bytes = abi.stage1_decode_plan(B, H, KVH, 128, cap)
+    assert preferred
+    splits, ws_bytes = abi.stage1_plan(B, 1, H, KVH, 128, cap)
+
+    def outputs():
+        return (torch.empty(B, H, 128, dtype=torch.float32, device=DEV),
+                torch.empty(B * H * 8, dtype=torch.float32, device=DEV))
+    tiles = []
+    for n, count in ((ws_bytes, splits), (max(ws_bytes, dec_bytes), splits), (max(ws_bytes, dec_bytes), 0)):
+        ws = torch.empty(max(n, 1), dtype=torch.uint8, device=DEV)
+        o, l = outputs()
+        abi.check(abi.lib().ck_fa_fp32_stage1(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), bt.data_ptr(), bt.shape[1], qs.data_ptr(), kl.data_ptr(), None,
+            B, 1, 1, B, H, KVH, 128, k.shape[0], 128, scale, cap, count, o.data_ptr(), l.data_ptr(), ws.data_ptr(), n,
+            st))
+        tiles.append((o, l))
+    for o, l in tiles[1:]:
+        assert torch.equal(o, tiles[0][0]) and torch.equal(l, tiles[0][1])
+    ws = torch.empty(dec_bytes, dtype=torch.uint8, device=DEV)
+    o, l = outputs()
+    abi.check(abi.lib().ck_fa_fp32_stage1_decode(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), bt.data_ptr(), bt.shape[1], kl.data_ptr(), B, H, KVH, 128,
+        k.shape[0], 128, scale, cap, o.data_ptr(), l.data_ptr(), ws.data_ptr(), dec_bytes, st))
+    o2, l2 = torch.ops.npu.fa_fp32_stage1(q, k, v, bt, qs, kl, 1)
+    assert torch.equal(o, o2) and torch.equal(l, l2)
+    assert not torch.equal(o, tiles[0][0])
+
+
 def test_decode_form_infinite_values():
     """An infinite V element reaches its own dim of the heads that read it as an
     infinity of the same sign (p > 0 of every token); every other output is finite."""

@@ -28,6 +28,9 @@ SIGNATURES = {
     "ck_fa_fp32_stage1_plan": (_int, [_i64, _i64, _i64, _i64, _i64, _i64, _p64, _p64]),
     "ck_fa_fp32_stage1": (_int, [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64,
                                  _i64, _i64, _i64, _f32, _i64, _i64, _vp, _vp, _vp, _i64, _vp]),
+    "ck_fa_fp32_stage1_decode_plan": (_int, [_i64, _i64, _i64, _i64, _i64, _p64, _p64]),
+    "ck_fa_fp32_stage1_decode": (_int, [_vp, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _i64,
+                                        _vp, _vp, _vp, _i64, _vp]),
     "ck_suffix_decode_plan": (_int, [_i64, _i64, _i64, _i64, _i64, _p64, _p64]),
     "ck_suffix_decode": (_int, [_vp, _vp, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32,
                                 _i64, _i64, _vp, _vp, _vp, _i64, _vp]),
@@ -90,6 +93,13 @@ def stage1_plan(batch, max_q_len, num_heads, kv_heads, head_dim, kv_cap):
     check(lib().ck_fa_fp32_stage1_plan(batch, max_q_len, num_heads, kv_heads, head_dim, kv_cap,
                                        ctypes.byref(s), ctypes.byref(w)), "ck_fa_fp32_stage1_plan")
     return s.value, w.value
+
+
+def stage1_decode_plan(batch, num_heads, kv_heads, head_dim, kv_cap):
+    p, w = ctypes.c_int64(0), ctypes.c_int64(0)
+    check(lib().ck_fa_fp32_stage1_decode_plan(batch, num_heads, kv_heads, head_dim, kv_cap, ctypes.byref(p),
+                                              ctypes.byref(w)), "ck_fa_fp32_stage1_decode_plan")
+    return bool(p.value), w.value
 
 
 def suffix_plan(batch, num_heads, kv_heads, head_dim, kv_cap):

@@ -56,7 +56,6 @@
 //   (O, LSE) pairs are folded by an N-way LSE merge (stage1_combine_kernel).
 // * Block order is XCD-aware: the m-tiles that read the same kv pages are
 //   placed on the same XCD so the later reads hit that XCD's L2.
-#include <algorithm>
 #include <cmath>
 
 #include "ck_common.h"
@@ -210,13 +209,6 @@ int make_plan(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_he
 // 1024 33.4 and 26.0). A kv bound of one 128-token page, where the reference's
 // rounding of P is checked, stays on the tiles.
 constexpr int64_t kDecodeMinCap = 1024;
-bool decode_form(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_heads, int64_t kv_cap) {
-    return max_q_len == 1 && batch > 0 && kv_cap >= kDecodeMinCap && num_heads <= (1 << 16) &&
-           batch <= suffix_group_batch(kv_cap);
-}
-int64_t decode_ws_bytes(int64_t batch, int64_t num_heads, int64_t kv_heads) {
-    return suffix_group_ws_bytes(batch, num_heads, kv_heads, suffix_plan_chunks(num_heads, kv_heads));
-}
 
 int check_dims(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_heads, int64_t head_dim,
                int64_t kv_cap) {
@@ -272,16 +264,7 @@ int ck::stage1_launch(const void *q, const void *k, const void *v, const int32_t
     if (num_tokens * num_heads > ((int64_t)1 << 31)) return CK_E_INVALID_ARG;
 
     Plan p;
-    make_plan(batch, max_q_len, num_heads, kv_heads, kv_cap, 0, &p);
-    // the decode form with the plan's split count and a workspace that also holds the
-    // suffix plan's; a caller's own split count, or a smaller workspace, runs the tiles
-    if (combine && q_len_uniform == 1 && decode_form(batch, max_q_len, num_heads, kv_heads, kv_cap) &&
-        (num_splits <= 0 || num_splits == p.splits) && workspace != nullptr &&
-        workspace_bytes >= decode_ws_bytes(batch, num_heads, kv_heads))
-        return suffix_launch_group(q, k, v, block_table, bt_cols, kv_seqlens, 0, batch, num_heads, kv_heads,
-                                   num_blocks, CK_KV_NHD, scale, kv_cap,
-                                   suffix_default_chunks(batch, num_heads, kv_heads, kv_cap), out, lse, workspace, nullptr, nullptr, nullptr, s, nullptr, 0, true);
-    if (num_splits > 0) make_plan(batch, max_q_len, num_heads, kv_heads, kv_cap, num_splits, &p);
+    make_plan(batch, max_q_len, num_heads, kv_heads, kv_cap, num_splits, &p);
     if (splits_used) *splits_used = p.splits;
     const int64_t need = p.splits > 1 ? p.splits * num_tokens * num_heads * (kD + 1) * (int64_t)sizeof(float) : 0;
     if (need > 0 && (workspace == nullptr || workspace_bytes < need)) return CK_E_WORKSPACE;
@@ -419,4 +402,47 @@ extern "C" int ck_fa_fp32_stage1(const void *q, const void *k, const void *v, co
                          max_q_len, num_tokens, num_heads, kv_heads, head_dim, num_blocks, block_size, scale,
                          kv_cap, num_splits, out, lse, workspace, workspace_bytes, true,
                          reinterpret_cast<hipStream_t>(stream), nullptr);
+}
+
+// One launch group of the suffix kernels: their batch and head limits hold.
+static int check_decode_dims(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t head_dim, int64_t kv_cap) {
+    int rc = check_dims(batch, 1, num_heads, kv_heads, head_dim, kv_cap);
+    if (rc != CK_OK) return rc;
+    if (num_heads > (1 << 16) || batch > suffix_group_batch(kv_cap)) return CK_E_UNSUPPORTED;
+    return CK_OK;
+}
+
+extern "C" int ck_fa_fp32_stage1_decode_plan(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t head_dim,
+                                             int64_t kv_cap, int64_t *preferred, int64_t *workspace_bytes) {
+    int rc = check_decode_dims(batch, num_heads, kv_heads, head_dim, kv_cap);
+    if (rc != CK_OK) return rc;
+    if (!preferred || !workspace_bytes) return CK_E_NULL_PTR;
+    *preferred = batch > 0 && kv_cap >= kDecodeMinCap;
+    *workspace_bytes = batch > 0 ? suffix_group_ws_bytes(batch, num_heads, kv_heads,
+                                                         suffix_plan_chunks(num_heads, kv_heads))
+                                 : 0;
+    return CK_OK;
+}
+
+extern "C" int ck_fa_fp32_stage1_decode(const void *q, const void *k, const void *v, const int32_t *block_table,
+                                        int64_t bt_cols, const int64_t *kv_seqlens, int64_t batch, int64_t num_heads,
+                                        int64_t kv_heads, int64_t head_dim, int64_t num_blocks, int64_t block_size,
+                                        float scale, int64_t kv_cap, float *out, float *lse, void *workspace,
+                                        int64_t workspace_bytes, void *stream) {
+    int64_t preferred = 0, need = 0;
+    int rc = ck_fa_fp32_stage1_decode_plan(batch, num_heads, kv_heads, head_dim, kv_cap, &preferred, &need);
+    if (rc != CK_OK) return rc;
+    if (block_size != kPage) return CK_E_UNSUPPORTED;
+    if (bt_cols < 0 || num_blocks < 0 || kv_cap > bt_cols * kPage) return CK_E_INVALID_ARG;
+    if (!(scale > 0.f) || !std::isfinite(scale)) return CK_E_INVALID_ARG;
+    if (batch == 0) return CK_OK;
+    if (!q || !k || !v || !block_table || !kv_seqlens || !out || !lse) return CK_E_NULL_PTR;
+    if (!aligned_to(q, 16) || !aligned_to(k, 16) || !aligned_to(v, 16) || !aligned_to(out, 16) ||
+        !aligned_to(lse, 16) || !aligned_to(workspace, 16))
+        return CK_E_INVALID_ARG;
+    if (workspace == nullptr || workspace_bytes < need) return CK_E_WORKSPACE;
+    return suffix_launch_group(q, k, v, block_table, bt_cols, kv_seqlens, 0, batch, num_heads, kv_heads, num_blocks,
+                               CK_KV_NHD, scale, kv_cap, suffix_default_chunks(batch, num_heads, kv_heads, kv_cap),
+                               out, lse, workspace, nullptr, nullptr, nullptr, reinterpret_cast<hipStream_t>(stream),
+                               nullptr, 0, true);
 }

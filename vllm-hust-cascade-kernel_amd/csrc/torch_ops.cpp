@@ -209,19 +209,25 @@ std::tuple<at::Tensor, at::Tensor> fa_fp32_stage1_impl(const at::Tensor &query, 
     if (query.device().is_meta()) return {out, lse};
 
     c10::OptionalDeviceGuard guard(query.device());
+    const float scale = static_cast<float>(1.0 / std::sqrt(1.0 * embed));
+    int64_t streamed = 0, stream_bytes = 0;
+    if (max_q_len == 1 && ck_fa_fp32_stage1_decode_plan(batch, num_heads, kv_heads, embed, kv_cap, &streamed,
+                                                        &stream_bytes) == CK_OK && streamed) {
+        at::Tensor ws = at::empty({stream_bytes}, query.options().dtype(at::kByte));
+        check_launch(ck_fa_fp32_stage1_decode(query.data_ptr(), key.data_ptr(), value.data_ptr(),
+                                              block_table.data_ptr<int32_t>(), cols,
+                                              actual_kv_seqlens.data_ptr<int64_t>(), batch, num_heads, kv_heads, embed,
+                                              key.size(0), block_size, scale, kv_cap, out.data_ptr<float>(),
+                                              lse.data_ptr<float>(), ws.data_ptr(), stream_bytes, stream_of(query)),
+                     "fa_fp32_stage1");
+        return {out, lse};
+    }
     int64_t num_splits = 0, ws_bytes = 0;
     check_launch(ck_fa_fp32_stage1_plan(batch, max_q_len, num_heads, kv_heads, embed, kv_cap, &num_splits,
                                         &ws_bytes),
                  "fa_fp32_stage1");
-    // one token per request from a kv bound of 1024: with room for the suffix plan's
-    // partials the requests are streamed (below, the kernel would not use it)
-    int64_t sfx_splits = 0, sfx_bytes = 0;
-    if (max_q_len == 1 && kv_cap >= 1024 &&
-        ck_suffix_decode_plan(batch, num_heads, kv_heads, embed, kv_cap, &sfx_splits, &sfx_bytes) == CK_OK)
-        ws_bytes = std::max(ws_bytes, sfx_bytes);
     at::Tensor ws;
     if (ws_bytes > 0) ws = at::empty({ws_bytes}, query.options().dtype(at::kByte));
-    const float scale = static_cast<float>(1.0 / std::sqrt(1.0 * embed));
     check_launch(ck_fa_fp32_stage1(query.data_ptr(), key.data_ptr(), value.data_ptr(),
                                    block_table.data_ptr<int32_t>(), cols, actual_q_seqlens.data_ptr<int64_t>(),
                                    actual_kv_seqlens.data_ptr<int64_t>(),
