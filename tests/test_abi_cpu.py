@@ -181,6 +181,13 @@ def test_stage1_decode_plan_and_validation():
     assert preferred and w >= abi.suffix_plan(64, 32, 8, 128, 8192)[1]
     assert not abi.stage1_decode_plan(64, 32, 8, 128, 128)[0]       # one page: the tiles
     assert abi.stage1_decode_plan(0, 32, 8, 128, 8192) == (False, 0)
+    # more than 8 heads per kv head: K and V are read once per group of heads, so only
+    # while batch * kv_cap * kv_heads * groups stays within 2^16
+    for batch, h, kvh, cap, want in [(64, 64, 8, 8192, True), (1000, 8, 8, 8192, True), (8, 64, 4, 1024, True),
+                                     (9, 64, 4, 1024, False), (8, 128, 8, 4096, False), (4, 48, 4, 1152, True),
+                                     (16, 32, 1, 1024, True), (17, 32, 1, 1024, False), (5, 11, 1, 1024, True),
+                                     (16, 11, 1, 2048, False), (64, 71, 1, 1536, False), (1, 71, 1, 8192, False)]:
+        assert abi.stage1_decode_plan(batch, h, kvh, 128, cap)[0] == want, (batch, h, kvh, cap)
     out = ctypes.c_int64(0)
     r = ctypes.byref(out)
     assert L.ck_fa_fp32_stage1_decode_plan(1025, 32, 8, 128, 1024, r, r) == -4       # one launch group

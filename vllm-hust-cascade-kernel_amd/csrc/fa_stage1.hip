@@ -199,16 +199,30 @@ int make_plan(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_he
 }
 
 // Decode form (one query token per request): a request has H / KVH query rows per
-// kv head of the 128-row tile, so one of its 4 waves computes, in a chain of
-// 64-token tiles, and every tile's MFMAs run for mostly padding. The suffix
-// kernels stream the same pages instead (16-column MFMA tiles, all requests'
-// windows balanced over the chip), with P at fp32 precision: 40 / 8 heads, 7 requests
-// of 1024-4096 tokens 28.4 -> 22.5 us, of 4096-16384 97 -> 58, 24 of 4096 95 -> 75.
-// From a kv bound of 1024: below, the tiles' chain is short and the fix-up kernel
-// costs more than it saves (24 requests of 512: 16.6 us tiles, 18.8 streamed; of
-// 1024 33.4 and 26.0). A kv bound of one 128-token page, where the reference's
-// rounding of P is checked, stays on the tiles.
+// kv head of the 128-row tile, so one of its waves computes, in a chain of 64-token
+// tiles, and every tile's MFMAs run for mostly padding. The suffix kernels stream
+// the same pages instead (16-column MFMA tiles, all requests' windows balanced over
+// the chip), with P in fp32. Tiles / streamed, us, ragged requests:
+// * 40 / 8 heads: 7 of up to 4096 tokens 25.8 / 16.5, 24 of 2048 49.3 / 35.8, 64 of 1024
+//   50.1 / 42.6, 200 of 1024 133.0 / 114.1, 8 of 2048 19.9 / 18.7.
+// * From a kv bound of 1024, the least at which it was faster for every number of
+//   requests (1 to 200) and of heads: at 512, 24 requests of 40 / 8 16.7 / 17.5, 64 of 16 /
+//   4 17.7 / 19.4 (though 200 of 40 / 8 89.1 / 66.7); at 256, 24 of 40 / 8 11.6 / 14.8. A
+//   bound of one 128-token page, where the reference's rounding of P is checked,
+//   stays on the tiles.
+// * Above 8 heads per kv head the stream reads K and V once per group of at most 8
+//   (suffix_sub_groups: 11 and 71 heads are prime, groups of one), the tiles once. It
+//   stays ahead while those reads are short next to the start-up: 8 requests of 1024 on
+//   64 / 4 heads (2 groups, 2^16 token rows) 16.8 / 13.8, 16 on 32 / 1 (4) 15.8 / 14.1,
+//   4 on 11 / 1 (11) 14.4 / 12.6; 2 of 4096 on 128 / 8 (2^17) 18.1 / 18.3, 8 of 4096 on 32
+//   / 1 (2^17) 16.9 / 17.6, 32 of 1024 on 11 / 1 16.5 / 23.8, 64 on 71 / 1 21 / 145.
 constexpr int64_t kDecodeMinCap = 1024;
+constexpr int64_t kDecodeMaxGroupedRows = (int64_t)1 << 16;
+bool decode_preferred(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap) {
+    const int64_t sub = suffix_sub_groups(num_heads, kv_heads);
+    return batch > 0 && kv_cap >= kDecodeMinCap &&
+           (sub == 1 || batch * kv_cap * kv_heads * sub <= kDecodeMaxGroupedRows);
+}
 
 int check_dims(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_heads, int64_t head_dim,
                int64_t kv_cap) {
@@ -417,7 +431,7 @@ extern "C" int ck_fa_fp32_stage1_decode_plan(int64_t batch, int64_t num_heads, i
     int rc = check_decode_dims(batch, num_heads, kv_heads, head_dim, kv_cap);
     if (rc != CK_OK) return rc;
     if (!preferred || !workspace_bytes) return CK_E_NULL_PTR;
-    *preferred = batch > 0 && kv_cap >= kDecodeMinCap;
+    *preferred = decode_preferred(batch, num_heads, kv_heads, kv_cap);
     *workspace_bytes = batch > 0 ? suffix_group_ws_bytes(batch, num_heads, kv_heads,
                                                          suffix_plan_chunks(num_heads, kv_heads))
                                  : 0;
