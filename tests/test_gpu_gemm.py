@@ -336,3 +336,25 @@ def test_decode_sized_tiles(M, K, I, mode):
         assert np.array_equal(bf16_to_np(d), c[:, :I])
         rows = np.arange(M) if rows is None else rows
         _c_check(c[rows], a[rows], b)
+
+
+# Which kernel runs at M <= 128 (launch_gemm): a K quarter per wave (M <= 32, K % 256 == 0)
+# at few K steps, above I = 4096 up to M = 16 and in a short second round of workgroups,
+# on both sides of each bound; the 256-row tile from 33 rows in short rounds.
+@pytest.mark.parametrize("M,K,I", [
+    (1, 256, 128), (16, 768, 128), (16, 1024, 128), (17, 256, 256), (32, 256, 8192), (17, 512, 256),
+    (16, 1024, 4224), (16, 1024, 4096), (3, 8192, 4224), (5, 7936, 4224), (1, 256, 16640), (32, 512, 24576),
+    (9, 256, 24704), (32, 384, 16640), (64, 256, 20480), (64, 256, 20608), (65, 256, 10240), (96, 256, 10368),
+    (96, 128, 24576), (96, 2304, 24576), (80, 128, 32896), (97, 256, 8192), (128, 256, 13056), (128, 256, 13184)])
+@pytest.mark.parametrize("mode", [1, 0])
+def test_decode_sized_dispatch_edges(M, K, I, mode):
+    a16, b16 = _inputs(M, K, I, seed=M + K + I)
+    a, b = bits_to_f32(a16), bits_to_f32(b16)
+    d, ws = torch.ops.npu.f3_gateup_epilogue(torch_bf16(a16, DEV), torch_bf16(b16, DEV), None, None, mode)
+    rows = np.unique(np.r_[0, M - 1, np.random.default_rng(K).choice(M, min(M, 4))])
+    if mode == 1:
+        _swiglu_check(bf16_to_np(d), a, b, rows)
+    else:
+        c = bf16_to_np(ws)
+        assert np.array_equal(bf16_to_np(d), c[:, :I])
+        _c_check(c[rows], a[rows], b)

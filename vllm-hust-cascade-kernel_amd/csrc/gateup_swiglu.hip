@@ -40,10 +40,11 @@
 //   64 up rows, three 48-KB stages) runs when the full-width grid would leave
 //   CUs idle (a few m-tiles, e.g. M = 256 at I = 14336: 224 workgroups instead
 //   of 112). K = 32 mod 64 runs the same kernel on 32-deep stages (4-stage ring).
-// * Decode-sized kernel (M <= 128, K % 128 == 0): the weight stream bounds the op, so
-//   weights go straight from global memory into MFMA operand registers, several
-//   steps ahead, the activations through LDS, and K is split over wave groups
-//   where the columns alone would leave CUs idle.
+// * Decode-sized kernels: the weight stream bounds the op, so weights go straight from
+//   global memory into MFMA operand registers, several steps ahead. One has the
+//   activations in LDS and splits K over wave groups where the columns alone would
+//   leave CUs idle (M <= 128, K % 128 == 0), one streams a K quarter per wave (M <=
+//   32, K % 256 == 0). launch_gemm has which of the three runs where.
 // * General kernel (any K % 16 == 0): 8 waves of 128 x (32 + 32), operands
 //   staged global -> registers -> LDS.
 // * Tiles are ordered M-fastest and XCD-aware so the workgroups sharing a
@@ -539,6 +540,136 @@ __global__ __launch_bounds__(kDThreads, 1) void gateup_dma_kernel(GemmArgs p) {
     }
 }
 
+// ---- decode-sized activations (M <= 32), K quarters per wave ----------------------
+// A workgroup takes 32 gate + 32 up weight rows against all activation rows (I / 32
+// workgroups, two per CU), and each of its 4 waves streams a quarter of K, weights and
+// activations, straight from global memory into MFMA operand registers, several
+// steps ahead; the four partial accumulators meet in LDS once at the end. No step has
+// a barrier, so it starts sooner than the kernel below and packs uneven grids
+// better (quarter_k_better has where).
+//   On v_mfma_f32_16x16x32_bf16 four lanes share a row (K groups of 8), so a
+//   16-byte-per-lane load covers 16 rows x 64 B: 16 address lines per
+//   instruction, half what the 32x32 layout (two lanes per row) needs per weight
+//   byte. Per 64-deep K step, lane (row r, group q) loads 32 contiguous bytes of
+//   its row, K [64 s + 16 q, +16); MFMA j (of 2) takes the j-th 16 bytes of both
+//   operands, i.e. K {64 s + 16 q + 8 j + t}, the same permutation on both sides,
+//   hence the exact product. Each wave holds 4 weight tiles (gate/up x 2 blocks of
+//   16 rows) per 16-row activation block (NB = 1 up to M = 16, 2 up to M = 32).
+//   Activation rows past M load row M - 1: they feed only output rows that are
+//   not stored.
+constexpr int kSThreads = 256;  // 4 waves, wave w reduces K quarter w
+constexpr int kSN = 32;         // gate rows (and as many up rows) per workgroup
+constexpr int kSStep = 64;      // K per pipeline step
+constexpr int kSDepth = 4;      // steps whose loads are in flight per wave (NB = 1)
+constexpr int kSMaxM = 32;
+
+template <int MODE, int NB>  // NB = 16-row activation blocks (M <= 16 NB)
+__global__ __launch_bounds__(kSThreads) void gateup_skinny16_kernel(GemmArgs p) {
+    typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
+    // [wave][weight tile: gate b0, gate b1, up b0, up b1][activation block][register][lane]
+    __shared__ float red[4][4][NB][4][64];
+    const int tid = threadIdx.x;
+    const int wid = tid >> 6;
+    const int lane = tid & 63;
+    const int r16 = lane & 15;
+    const int q4 = lane >> 4;
+    const int64_t n0 = (int64_t)blockIdx.x * kSN;
+    const int64_t kq = p.k / 4;
+    const int steps = (int)(kq / kSStep);
+    const int64_t koff = wid * kq + 16 * q4;
+    const uint4 *wp[4];  // gate rows n0 + 16 b + r16, up rows n_half + n0 + 16 b + r16
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        wp[t] = reinterpret_cast<const uint4 *>(p.b + ((t < 2 ? 0 : p.n_half) + n0 + 16 * (t & 1) + r16) * p.k + koff);
+    const uint4 *xp[NB];
+#pragma unroll
+    for (int ab = 0; ab < NB; ++ab) {
+        const int64_t arow = 16 * ab + r16 < p.m ? 16 * ab + r16 : p.m - 1;
+        xp[ab] = reinterpret_cast<const uint4 *>(p.a + arow * p.k + koff);
+    }
+    constexpr int kStepVec = kSStep * 2 / 16;  // uint4 per row per step (8)
+    constexpr int kDepth = NB == 1 ? kSDepth : 3;  // registers: 48 per step at NB = 2
+
+    uint4 W[kDepth][4][2], X[kDepth][NB][2];
+    f32x4_t acc[4][NB];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int ab = 0; ab < NB; ++ab)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[t][ab][e] = 0.f;
+#define CK_SKINNY16_LOAD(slot, st)                                          \
+    do {                                                                    \
+        const int64_t o_ = (int64_t)(st) * kStepVec;                        \
+        _Pragma("unroll") for (int j_ = 0; j_ < 2; ++j_) {                  \
+            _Pragma("unroll") for (int t_ = 0; t_ < 4; ++t_) W[slot][t_][j_] = wp[t_][o_ + j_]; \
+            _Pragma("unroll") for (int b_ = 0; b_ < NB; ++b_) X[slot][b_][j_] = xp[b_][o_ + j_]; \
+        }                                                                   \
+    } while (0)
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d)
+        if (d < steps) CK_SKINNY16_LOAD(d, d);
+    for (int s = 0; s < steps; s += kDepth) {
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d) {
+            if (s + d < steps) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int ab = 0; ab < NB; ++ab) {
+                        const bf16x8 xf = __builtin_bit_cast(bf16x8, X[d][ab][j]);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            acc[t][ab] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                __builtin_bit_cast(bf16x8, W[d][t][j]), xf, acc[t][ab], 0, 0, 0);
+                    }
+                if (s + d + kDepth < steps) CK_SKINNY16_LOAD(d, s + d + kDepth);
+            }
+        }
+    }
+#undef CK_SKINNY16_LOAD
+
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int ab = 0; ab < NB; ++ab)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) red[wid][t][ab][e][lane] = acc[t][ab][e];
+    __syncthreads();
+    // thread -> (weight tile pair b: gate b and up b, activation block ab, accumulator
+    // lane l): output row 16 ab + l % 16, columns n0 + 16 b + 4 (l / 16) + 0..3
+    if (tid >= 2 * NB * 64) return;
+    const int b = tid / (NB * 64);
+    const int ab = (tid / 64) % NB;
+    const int l = tid & 63;
+    const int64_t gm = 16 * ab + (l & 15);
+    if (gm >= p.m) return;
+    float g[4], u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        g[i] = red[0][b][ab][i][l] + red[1][b][ab][i][l] + red[2][b][ab][i][l] + red[3][b][ab][i][l];
+        u[i] = red[0][2 + b][ab][i][l] + red[1][2 + b][ab][i][l] + red[2][2 + b][ab][i][l] + red[3][2 + b][ab][i][l];
+    }
+    const int64_t col = n0 + 16 * b + 4 * (l >> 4);
+    if (MODE == 1) {
+        *reinterpret_cast<uint2 *>(p.d + gm * p.d_stride + col) =
+            make_uint2(pack_bf16x2(silu_mul(g[0], u[0]), silu_mul(g[1], u[1])),
+                       pack_bf16x2(silu_mul(g[2], u[2]), silu_mul(g[3], u[3])));
+    } else {
+        const uint2 gv = make_uint2(pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3]));
+        const uint2 uv = make_uint2(pack_bf16x2(u[0], u[1]), pack_bf16x2(u[2], u[3]));
+        uint16_t *crow = p.c + gm * (2 * p.n_half);
+        *reinterpret_cast<uint2 *>(crow + col) = gv;
+        *reinterpret_cast<uint2 *>(crow + p.n_half + col) = uv;
+        if (MODE == 0 || MODE == 5)
+            *reinterpret_cast<uint2 *>(p.d + gm * p.d_stride + col) = gv;
+        else if (MODE == 4)
+            *reinterpret_cast<uint2 *>(p.d + gm * p.d_stride + col) = uv;
+        else if (MODE == 8)
+            *reinterpret_cast<uint2 *>(p.d + gm * p.d_stride + col) = make_uint2(0, 0);
+    }
+}
+
 // ---- decode-sized activations (M <= 128) -----------------------------------------
 // With few activation rows the op is bound by the weight stream (2I x K bf16),
 // not by MFMA; the 256-row tile above spends most of its LDS and DMAs on padding
@@ -562,9 +693,9 @@ __global__ __launch_bounds__(kDThreads, 1) void gateup_dma_kernel(GemmArgs p) {
 //   the workgroups of every XCD (blockIdx % 8) over all steps.
 // * Depth: 2 / 3 / 4 steps of weights 54 / 50 / 51 us (same start); non-temporal
 //   weight loads 59.
-// Against the kernel with a K quarter per wave and no LDS copy of the activations
-// that ran up to M = 32: M = 1 41.0 -> 40.7 us, M = 16 45.7 -> 41.8, M = 32
-// 52.6 -> 42.4 us, M = 64 59.9 -> 46.4; K = 8192, I = 3584: M = 1 35.1 -> 25.0 us.
+// K quarters per wave / this kernel at K = 4096, I = 14336: M = 1 41.0 / 40.7 us, M = 16
+// 45.7 / 41.8, M = 32 52.6 / 42.4; 256-row tile / this: M = 64 59.9 / 46.4. K = 8192, I
+// = 3584: M = 1 35.1 / 25.0 us.
 constexpr int kMStep = 128;  // K per step
 constexpr int kMDepth = 3;   // steps of weights in flight per wave
 constexpr int kMMaxM = 128;
@@ -797,14 +928,69 @@ int launch_mid(GemmArgs p, hipStream_t s) {
 }
 
 template <int MODE>
+int launch_quarter_k(const GemmArgs &p, hipStream_t s) {
+    if (p.m <= 16)
+        hipLaunchKernelGGL((gateup_skinny16_kernel<MODE, 1>), dim3((unsigned)(p.n_half / kSN)), dim3(kSThreads), 0, s,
+                           p);
+    else
+        hipLaunchKernelGGL((gateup_skinny16_kernel<MODE, 2>), dim3((unsigned)(p.n_half / kSN)), dim3(kSThreads), 0, s,
+                           p);
+    CK_RETURN_LAUNCH();
+}
+
+// The rules below compare the decode-sized kernel with a K group (64 columns a
+// workgroup, whose time is the latency of its K steps whatever the columns) with
+// the two others. One round of it costs the same for 130 workgroups as for 256, and
+// a second round of a few as much as the first: `fill` is its workgroups per round.
+int64_t mid_fill(int64_t n_half, int64_t *rounds) {
+    const int64_t wgs = n_half / 64;
+    *rounds = (wgs + kNumCus - 1) / kNumCus;
+    return wgs / *rounds;
+}
+
+// A K quarter per wave instead, M <= 32 and K % 256 == 0 (quarter / other, us):
+// * up to I = 8192 and few K steps: K = 256, I = 1024 M = 1 3.11 / 3.68, M = 32 3.65 /
+//   3.80; K = 512 M = 1 4.35 / 4.48; K = 768 M = 16 0.96 of the time (M = 24 1.06);
+// * up to M = 16 where K is split over two groups: K = 2048, I = 6144 M = 1 12.22 /
+//   12.98, K = 4096 20.75 / 21.81, M = 16 23.0 / 23.2 (M = 24 25.0 / 24.1; K = 8192 M =
+//   1 46.9 / 39.6);
+// * a second round of up to 3/4 of the CUs: I = 18944, K = 4096 M = 1 0.82 of the time,
+//   M = 32 0.95; I = 24576 0.85 and 0.96, I = 25600 1.03 and 1.19.
+bool quarter_k_better(const GemmArgs &p) {
+    if (p.n_half <= 32 * kNumCus)
+        return p.k <= (p.m <= 16 ? 768 : 256) || (p.m <= 16 && p.n_half > 16 * kNumCus && p.k < 8192);
+    int64_t rounds;
+    const int64_t fill = mid_fill(p.n_half, &rounds);
+    return rounds > 1 && fill <= 192;
+}
+
+// The decode-sized kernel, not the 256-row tile (tile's time / decode-sized's):
+// * M <= 64: a single round always (K = 4096, I = 9216 M = 64 1.15, I = 14336 1.29), a
+//   second one above 5/8 of the CUs (I = 18432 M = 64 0.99, M = 48 1.06 and K = 5120
+//   0.90; I = 22016 1.10);
+// * M <= 96: the activations' share of the L2 and LDS traffic costs more, so above 5/8
+//   in a single round (M = 96, I = 9216 K = 3072 0.95, K = 4096 0.99; I = 11776 1.01,
+//   1.06), and in the second from 3/4 on (I = 24576 M = 96 K = 4096 1.03, K = 5120 0.94)
+//   where the tile's own loads collide: its workgroups walk K in step, and operand
+//   rows a power of two apart then meet on few channels. From the third on (I =
+//   33024 1.38, K = 5120 1.21) the tile itself needs a second round;
+// * above: a single round from 4/5 on, at those K (M = 128, K = 4096 I = 12288 1.00, I =
+//   13824 1.04; I = 11008 0.98; K = 5120, I = 13824 0.94).
+bool mid_better(const GemmArgs &p) {
+    if (p.n_half <= 32 * kNumCus) return true;
+    int64_t rounds;
+    const int64_t fill = mid_fill(p.n_half, &rounds);
+    const bool collide = p.k <= 2048 || p.k % 4096 == 0;
+    if (p.m <= 64) return rounds == 1 || fill > 160;
+    if (p.m <= 96) return rounds == 1 ? fill > 160 : rounds > 2 || (fill >= 192 && collide);
+    return rounds == 1 && fill >= 205 && collide;
+}
+
+template <int MODE>
 int launch_gemm(const GemmArgs &p, hipStream_t s) {
-    if (p.m <= kMMaxM && p.k % kMStep == 0 && p.k <= kMaxDmaK) {
-        // above 96 rows the activations' share of the L2 and LDS traffic costs what the
-        // padding rows of the 256-row tile do: ahead only in one round of workgroups
-        // (M = 128, K = 8192, I = 28672: 218 us against 208; K = 4096, I = 14336: 57.2
-        // against 58.3)
-        if (p.m <= 96 || p.n_half <= 64 * kNumCus) return launch_mid<MODE>(p, s);
-    }
+    if (p.m <= kSMaxM && p.k % (4 * kSStep) == 0 && (p.k > kMaxDmaK || quarter_k_better(p)))
+        return launch_quarter_k<MODE>(p, s);
+    if (p.m <= kMMaxM && p.k % kMStep == 0 && p.k <= kMaxDmaK && mid_better(p)) return launch_mid<MODE>(p, s);
     const int64_t grid = (int64_t)p.mtiles * p.ntiles;
     if (p.k % 32 == 0 && p.k <= kMaxDmaK) {
         // The half-width tile (WB = 1) does about 3/4 of the full tile's work per
