@@ -158,6 +158,16 @@ def test_cascade_plan_and_validation():
     assert call(batch=0) == 0                       # empty batch: nothing to do
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(32, 8), (40, 8), (64, 8), (8, 1), (64, 4), (8, 8)])
+def test_cascade_workspace_of_the_largest_suffix_bound_serves_the_smaller(heads, kv_heads):
+    """With or without the fused kernel (prefix work up to 2^26), the plan does not shrink as
+    the suffix bound grows: a workspace planned once for the longest suffixes is enough."""
+    for batch in (1, 8, 32, 33, 64, 256):
+        for prefix in (1024, (1 << 26) // (batch * heads) // 128 * 128 + 128):
+            w = [abi.cascade_plan(batch, heads, kv_heads, 128, prefix, cap) for cap in (128, 512, 1024, 4096, 32768)]
+            assert w == sorted(w), (batch, prefix, w)
+
+
 def test_add_rms_norm_validation_without_launch():
     L = abi.lib()
     p = ctypes.c_void_p(16)

@@ -89,7 +89,10 @@ int cascade_layout(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t h
     L->s1_bytes = align_up(s1 > 1 ? s1_ws : final_bytes);
     L->chunks = L->fused ? ck::suffix_fused_chunks(num_heads, kv_heads)
                          : ck::suffix_default_chunks(batch, num_heads, kv_heads, suffix_cap);
-    L->sfx_bytes = align_up(ck::suffix_group_ws_bytes(L->group_batch, num_heads, kv_heads, L->chunks));
+    // room for the most chunks of any batch and suffix bound, so that a workspace planned
+    // for the largest call also serves the smaller ones
+    const int64_t most = L->fused ? L->chunks : ck::suffix_plan_chunks(num_heads, kv_heads);
+    L->sfx_bytes = align_up(ck::suffix_group_ws_bytes(L->group_batch, num_heads, kv_heads, most));
     L->whole_bytes = align_up(L->group_batch * num_heads * (kD * 2 + 4));
     L->total = batch > 0 ? L->s1_bytes + L->sfx_bytes + L->whole_bytes : 0;
     return CK_OK;
