@@ -1,5 +1,5 @@
 """The window -> chunk arithmetic of the suffix kernels, the fix-up and the
-cascade epilogue (`ChunkMap` in csrc/suffix_decode.hip), checked on the host.
+cascade epilogue (`ChunkMap` in csrc/chunk_map.h), checked on the host.
 
 The kernels take floor(x / d) as the truncated IEEE double quotient
 (`div_nonneg`) for 0 <= x <= W P and 1 <= d < 2^31, where W < 2^31 windows (the
@@ -8,7 +8,12 @@ division is the same correctly rounded IEEE operation, so these tests pin the
 identity on random and adversarial operands (quotients just below an integer,
 the largest operands), show that a single-precision quotient fails them, and
 check the chunk map built on it: chunk c covers [lo(c), lo(c + 1)) and owner(p)
-is the chunk whose range holds window p."""
+is the chunk whose range holds window p. The header itself is compiled for the host
+and checked too: it is the code the kernels run."""
+import ctypes
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -122,3 +127,59 @@ def test_no_empty_chunk_inside_a_cut_sequence(P, split):
         assert (size >= 0).all()
         np.testing.assert_array_equal(np.repeat(np.arange(P), size), own)
         assert (size[own.min():own.max() + 1] >= 1).all()
+
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "vllm-hust-cascade-kernel_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def header(tmp_path_factory):
+    """lo and owner of csrc/chunk_map.h, compiled for the host"""
+    d = tmp_path_factory.mktemp("chunk_map")
+    src = d / "chunk_map.cpp"
+    src.write_text("""#include "chunk_map.h"
+extern "C" void lo(int64_t W, int P, int split, const int64_t *c, int64_t n, int64_t *out) {
+    const ck::ChunkMap m{W, P, split};
+    for (int64_t i = 0; i < n; ++i) out[i] = m.lo((int)c[i]);
+}
+extern "C" void owner(int64_t W, int P, int split, const int64_t *p, int64_t n, int64_t *out) {
+    const ck::ChunkMap m{W, P, split};
+    for (int64_t i = 0; i < n; ++i) out[i] = m.owner(p[i]);
+}
+""")
+    lib = d / "chunk_map.so"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-I", CSRC, str(src), "-o", str(lib)], check=True)
+    handle = ctypes.CDLL(str(lib))
+
+    def call(name, x, W, P, split):
+        x = np.ascontiguousarray(x, dtype=np.int64)
+        out = np.empty_like(x)
+        ptr = ctypes.POINTER(ctypes.c_int64)
+        getattr(handle, name)(ctypes.c_int64(W), ctypes.c_int(P), ctypes.c_int(split), x.ctypes.data_as(ptr),
+                              ctypes.c_int64(x.size), out.ctypes.data_as(ptr))
+        return out
+    return call
+
+
+@pytest.mark.parametrize("P,split", [(1, 0), (64, 0), (512, 0), (73, 0), (2, 208), (64, 208), (64, 224), (512, 224),
+                                     (64, 128), (64, 255)])
+def test_compiled_header(header, P, split):
+    """Every window has one owner, every chunk between the owners of two windows holds
+    windows, and from one window per chunk on the ranges are the exact shares."""
+    for W in sorted({1, 2, 3, 4, 5, P // 2, P - 2, P - 1, P, P + 1, 3 * P + 1, 20011, 2 ** 31 - 1}):
+        if W < 1:
+            continue
+        c = np.arange(P + 1, dtype=np.int64)
+        lo = header("lo", c, W, P, split)
+        assert lo[0] == 0 and lo[-1] == W and (np.diff(lo) >= 0).all(), (W, lo)
+        if W >= P:
+            h = max(P // 2, 1)
+            a, b = c // 2 * W // h, (c // 2 + 1) * W // h
+            np.testing.assert_array_equal(lo, c * W // P if split == 0 else
+                                          np.where(c % 2 == 0, a, a + (b - a) * split // 256))
+        p = np.arange(W, dtype=np.int64) if W <= 1 << 16 else np.unique(np.r_[
+            np.random.default_rng(3).integers(0, W, 1 << 14), lo[1:-1] - 1, lo[1:-1], 0, W - 1])
+        own = header("owner", p, W, P, split)
+        assert (own >= 0).all() and (own < P).all()
+        assert (lo[own] <= p).all() and (p < lo[own + 1]).all()
+        assert (np.diff(lo)[own.min():own.max() + 1] >= 1).all(), W

@@ -67,6 +67,7 @@
 #include <type_traits>
 
 #include "ck_common.h"
+#include "chunk_map.h"
 #include "ck_internal.h"
 
 // Bounded waits of this file's kernels that ran out (a broken invariant, never
@@ -174,63 +175,6 @@ struct SuffixArgs {
     int chunks;  // chunks of the window list per kv head group
     int split;   // 0: equal chunks; else chunk pairs, the first taking split/256 (ChunkMap)
     float scale_log2;
-};
-
-// Window ranges of the chunks of one kv head group (W windows): chunk c covers
-// [lo(c), lo(c + 1)). split == 0: P equal chunks, lo(c) = c W / P. split > 0 (P
-// even): chunks 2j and 2j + 1 share the j-th of P / 2 equal ranges, the first
-// taking split / 256 of it (the fused cascade kernel's two roles on one CU).
-// floor(x / d) for 0 <= x < 2^52, 1 <= d < 2^31 (here x <= W P with W < 2^31
-// windows and P <= 2^20 chunks) from one IEEE double division: with
-// n = floor(x / d), a quotient that is not the integer n is at most
-// n + 1 - 1 / d, and rounding moves it up by at most (n + 1) 2^-53 < 1 / d
-// (as (n + 1) d <= x + d < 2^53), so it truncates to n; an integer quotient is
-// exact. A 64-bit integer division would expand to a few hundred scalar
-// instructions per use, inline between the hot blocks of the kernels that map
-// windows to chunks (the epilogue was 85% such code and missed the
-// instruction cache on 6% of its fetches).
-__device__ __forceinline__ int64_t div_nonneg(int64_t x, int64_t d) {
-    return (int64_t)((double)x / (double)d);
-}
-
-// With fewer windows than chunks the first chunks take one window each (split > 0:
-// the first pairs two, one per chunk; an odd last window joins the last pair, and
-// a single window is the first pair's second chunk's), in closed form without a
-// division. So no chunk between two that hold windows is ever empty, and folding a
-// cut sequence's partials tests nothing (ranges spread over all P chunks left
-// empty ones inside a sequence there, and testing them, two chunk bounds per chunk
-// of dependent double divisions, cost the cascade epilogue half of its 13.3 us at 8
-// sequences on a 2048-token prefix).
-struct ChunkMap {
-    int64_t W;
-    int P;
-    int split;
-    __device__ __forceinline__ int64_t lo(int c) const {
-        if (W < P) {
-            if (split == 0) return min((int64_t)c, W);
-            const int h = max((int)W >> 1, 1);  // pairs that hold windows
-            if (c >= 2 * h) return W;
-            const int a = c & ~1;
-            return (c & 1) == 0 ? a : a + (((a == 2 * h - 2 ? (int)W - a : 2) * split) >> 8);
-        }
-        if (split == 0) return div_nonneg((int64_t)c * W, P);
-        const int h = P >> 1, j = c >> 1;
-        const int64_t a = div_nonneg((int64_t)j * W, h);
-        if ((c & 1) == 0) return a;
-        return a + (((div_nonneg((int64_t)(j + 1) * W, h) - a) * split) >> 8);
-    }
-    // the chunk that owns window p < W
-    __device__ __forceinline__ int owner(int64_t p) const {
-        int j;
-        if (W < P) {
-            if (split == 0) return (int)p;
-            j = min((int)p >> 1, max((int)W >> 1, 1) - 1);
-        } else {
-            if (split == 0) return (int)div_nonneg((p + 1) * P - 1, W);
-            j = (int)div_nonneg((p + 1) * (P >> 1) - 1, W);
-        }
-        return 2 * j + (p >= lo(2 * j + 1) ? 1 : 0);
-    }
 };
 
 typedef int i32x2 __attribute__((ext_vector_type(2)));
