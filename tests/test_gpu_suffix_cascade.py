@@ -517,3 +517,45 @@ def test_fused_above_4_heads_full_precision_p(H, KVH):
     mag = np.einsum("bght,bgtd->bghd", p, np.abs(vv))
     excess = float(((np.abs(got - ref) - 2.0 ** -8 * np.abs(ref)) / mag).max())
     assert excess <= 2.0 ** -19
+
+
+# The stream uses half of its grid's chunks once sequences hold 5 windows of 32 tokens in the
+# mean (up to 5 heads per group): one window below and at that mean, under a table as
+# wide as the lengths and a far wider one, in the stand-alone op and (a serial
+# cascade: prefix work above 2^26) with the cascade's epilogue folding the cut sequences.
+@pytest.mark.parametrize("H,KVH", [(32, 8), (10, 2), (8, 8)])
+@pytest.mark.parametrize("short", [1, 0])
+@pytest.mark.parametrize("cols", [8, 32])
+def test_chunks_in_use_by_mean_length(H, KVH, short, cols):
+    B = 24
+    rng = np.random.default_rng(H + short)
+    wins = rng.integers(1, 10, size=B)
+    wins[0] = 20
+    while wins.sum() != 5 * B - short:
+        b = rng.integers(1, B)
+        wins[b] = max(0, wins[b] + np.sign(5 * B - short - wins.sum()))
+    kvs = np.where(wins > 0, 32 * wins - rng.integers(0, 32, size=B), 0)
+    inp = paged_inputs(B, kvs, H, KVH, seed=H, permute=True, block_cols=cols)
+    out, lse = _suffix(inp)
+    _check_suffix(inp, out, lse, H)
+
+
+@pytest.mark.parametrize("short", [1, 0])
+def test_serial_cascade_chunks_in_use_by_mean_length(short):
+    B, H, KVH, P = 65, 32, 8, 32384
+    suf = np.full(B, 160 - 3)
+    suf[7], suf[11:15] = 160 - 3 + 256 - 32 * short, 77  # 5 B windows (less one)
+    assert ((suf + 31) // 32).sum() == 5 * B - short and B * H * P > 1 << 26
+    q16, k16, v16, bt_pre, bt_suf, suf = _cascade_inputs(B, H, KVH, P, suf, seed=short)
+    bt_suf = np.concatenate([bt_suf, np.zeros((B, 30), np.int32)], axis=1)
+    q, k, v = (torch_bf16(x, DEV) for x in (q16, k16, v16))
+    got, lse = _cascade_run(True, B, P, q, k, v, bt_pre, bt_suf, suf)
+    qf, kf, vf = bits_to_f32(q16), bits_to_f32(k16), bits_to_f32(v16)
+    kp, vp = A.gather_kv(kf, vf, bt_pre[0], P)
+    for b in (0, 6, 7, 8, 12, B - 1):
+        ks, vs = A.gather_kv(kf, vf, bt_suf[b], int(suf[b]))
+        Od, Ld = A.dense(qf[b:b + 1], A.expand_heads(np.concatenate([kp, ks]), H),
+                         A.expand_heads(np.concatenate([vp, vs]), H))
+        err = np.abs(got[b:b + 1] - Od)
+        assert np.all(err <= 2e-3 + 2.0 ** -8 * np.abs(Od)), (b, err.max())
+        assert np.abs(lse.reshape(B, H)[b] - Ld[0]).max() <= 1e-4 * max(1.0, np.abs(Ld[0]).max())

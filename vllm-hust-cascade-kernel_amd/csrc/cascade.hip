@@ -58,7 +58,7 @@ struct CascadeLayout {
     int64_t s1_units;     // fused: stage-1 units
     int64_t s1_splits;
     int64_t s1_bytes;     // stage-1 partials, or the final O1 [R][128] + padded LSE1 [R * 8]
-    int64_t chunks;
+    ck::SuffixChunks chunks;
     int64_t group_batch;  // sequences per suffix launch group
     int64_t sfx_bytes;    // suffix group workspace
     int64_t whole_bytes;  // bf16 O2 [nb][H][128] + fp32 LSE2 [nb * H] of one group
@@ -87,11 +87,12 @@ int cascade_layout(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t h
     L->s1_splits = s1;
     const int64_t final_bytes = rows * (kD + 8) * (int64_t)sizeof(float);
     L->s1_bytes = align_up(s1 > 1 ? s1_ws : final_bytes);
-    L->chunks = L->fused ? ck::suffix_fused_chunks(num_heads, kv_heads)
+    const int64_t fused_chunks = ck::suffix_fused_chunks(num_heads, kv_heads);
+    L->chunks = L->fused ? ck::SuffixChunks{fused_chunks, fused_chunks}
                          : ck::suffix_default_chunks(batch, num_heads, kv_heads, suffix_cap);
     // room for the most chunks of any batch and suffix bound, so that a workspace planned
     // for the largest call also serves the smaller ones
-    const int64_t most = L->fused ? L->chunks : ck::suffix_plan_chunks(num_heads, kv_heads);
+    const int64_t most = L->fused ? fused_chunks : ck::suffix_plan_chunks(num_heads, kv_heads);
     L->sfx_bytes = align_up(ck::suffix_group_ws_bytes(L->group_batch, num_heads, kv_heads, most));
     L->whole_bytes = align_up(L->group_batch * num_heads * (kD * 2 + 4));
     L->total = batch > 0 ? L->s1_bytes + L->sfx_bytes + L->whole_bytes : 0;

@@ -68,7 +68,12 @@ struct ChunkMap {
         return 2 * j + (p >= lo(2 * j + 1) ? 1 : 0);
     }
     // W < P, split > 0: pairs that hold windows
-    CK_HD int few_pairs() const { return (W >> 1) > 1 ? (int)(W >> 1) : 1; }
+    CK_HD int few_pairs() const { return ((int)W >> 1) > 1 ? (int)W >> 1 : 1; }
 };
+
+// Chunks in use of a grid that has room for `most`: `few` once the sequences hold 5
+// windows in the mean. The lengths decide, not the bound that the host knows (a table
+// as wide as the longest context says nothing of them).
+CK_HD int chunks_used(int64_t W, int batch, int most, int few) { return W >= (int64_t)5 * batch ? few : most; }
 
 }  // namespace ck

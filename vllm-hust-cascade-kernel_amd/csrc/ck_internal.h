@@ -39,7 +39,11 @@ int stage1_fused_args(const void *q, const void *k, const void *v, const int32_t
 // chunk count and the workspace one launch group needs.
 int64_t suffix_group_batch(int64_t kv_cap);
 int64_t suffix_sub_groups(int64_t num_heads, int64_t kv_heads);
-int64_t suffix_default_chunks(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap);
+struct SuffixChunks {
+    int64_t most;  // workgroups launched per kv head group; the partials' room
+    int64_t few;   // of those, the chunks in use for long sequences (chunks_used)
+};
+SuffixChunks suffix_default_chunks(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap);
 int64_t suffix_plan_chunks(int64_t num_heads, int64_t kv_heads);
 int64_t suffix_group_ws_bytes(int64_t nb, int64_t num_heads, int64_t kv_heads, int64_t chunks);
 
@@ -66,7 +70,7 @@ int64_t suffix_fused_chunks(int64_t num_heads, int64_t kv_heads);
 // rows and 8 copies of each LSE.
 int suffix_launch_group(const void *q, const void *k, const void *v, const int32_t *block_table, int64_t bt_cols,
                         const int64_t *kv_seqlens, int64_t b0, int64_t nb, int64_t num_heads, int64_t kv_heads,
-                        int64_t num_blocks, int64_t kv_layout, float scale, int64_t kv_cap, int64_t chunks,
+                        int64_t num_blocks, int64_t kv_layout, float scale, int64_t kv_cap, SuffixChunks chunks,
                         void *out, float *lse, void *group_ws, const Stage1Result *cascade, void *final_out,
                         float *final_lse, hipStream_t stream, const s1::Stage1Args *fused = nullptr,
                         int64_t fused_units = 0, bool f32_out = false);

@@ -209,7 +209,9 @@ int make_plan(int64_t batch, int64_t max_q_len, int64_t num_heads, int64_t kv_he
 //   requests (1 to 200) and of heads: at 512, 24 requests of 40 / 8 16.7 / 17.5, 64 of 16 /
 //   4 17.7 / 19.4 (though 200 of 40 / 8 89.1 / 66.7); at 256, 24 of 40 / 8 11.6 / 14.8. A
 //   bound of one 128-token page, where the reference's rounding of P is checked,
-//   stays on the tiles.
+//   stays on the tiles. The bound is the table's width: short requests under a wide
+//   one stream too, and lose where the tiles run unsplit (up to 300 tokens under
+//   32768, 32 / 8 heads: 8 requests 13.4 / 10.9, 32 12.7 / 14.5, 200 51.6 / 29.2).
 // * Above 8 heads per kv head the stream reads K and V once per group of at most 8
 //   (suffix_sub_groups: 11 and 71 heads are prime, groups of one), the tiles once. It
 //   stays ahead while those reads are short next to the start-up: 8 requests of 1024 on

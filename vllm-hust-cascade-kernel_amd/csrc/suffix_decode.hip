@@ -173,7 +173,10 @@ struct SuffixArgs {
     int kv_sub;    // query-head groups per physical kv head (group = kv_sub x G)
     int kv_cap;
     int chunks;  // chunks of the window list per kv head group
-    int split;   // 0: equal chunks; else chunk pairs, the first taking split/256 (ChunkMap)
+    // PAIRS: ChunkMap's split; otherwise the chunks in use for long sequences (chunks_used).
+    // One field for both: another word in the struct moved the fused kernel's argument
+    // loads behind its stage-1 part (64 / 32 heads on 8192 tokens 50.3 -> 51.4 us).
+    int split_few;
     float scale_log2;
 };
 
@@ -267,8 +270,8 @@ __device__ __forceinline__ void write_f32_row(const SuffixArgs &a, int64_t row, 
 // Two bodies on one CU may share one scan: the body given scan_src (the other
 // body's LDS) skips its own, waits until scan_flag is set and reads the other's
 // lengths and window prefix sums; the body given only scan_flag sets it once its
-// scan is complete.
-template <int G, int NW, int D, bool F32, bool EXACTP, class L = SfxLds<G, NW>, class Bar>
+// scan is complete. PAIRS: chunk pairs (the fused kernel), every chunk of the grid.
+template <int G, int NW, int D, bool F32, bool EXACTP, bool PAIRS, class L = SfxLds<G, NW>, class Bar>
 __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS char *smem, int lb, int tid,
                                                    const Bar &bar, CK_LDS int *scan_flag = nullptr,
                                                    const CK_LDS char *scan_src = nullptr) {
@@ -354,7 +357,9 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     }
 
     const int W = __builtin_amdgcn_readfirstlane(cw[a.batch]);  // scalar: ChunkMap branches on it
-    const ChunkMap cm{W, a.chunks, a.split};
+    const int P = PAIRS ? a.chunks : chunks_used(W, a.batch, a.chunks, a.split_few);
+    if (!PAIRS && chunk >= P) return;  // uniform over the workgroup
+    const ChunkMap cm{W, P, PAIRS ? a.split_few : 0};
     const int w0 = (int)cm.lo(chunk);
     const int w1 = (int)cm.lo(chunk + 1);
     if (w0 >= w1) return;  // uniform over the workgroup
@@ -467,7 +472,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
                 if (d4 == 0) a.lse[row] = lse_v;
             }
         } else {
-            const int64_t pidx = (((int64_t)g * a.chunks + chunk) * 2 + (head_part ? 0 : 1)) * G + h;
+            const int64_t pidx = (((int64_t)g * (PAIRS ? a.chunks : P) + chunk) * 2 + (head_part ? 0 : 1)) * G + h;
             // non-temporal: read once, by the fix-up or cascade epilogue kernel
             __builtin_nontemporal_store(on, reinterpret_cast<f32x4 *>(a.part_o + pidx * kD + 4 * d4));
             if (d4 == 0) a.part_lse[pidx] = lse_v;
@@ -824,7 +829,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
 template <int G, bool F32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void suffix_stream_kernel(SuffixArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    suffix_stream_body<G, 4, (G > 4 ? 1 : kTokDepth), F32, F32>(a, (CK_LDS char *)smem_raw, blockIdx.x, threadIdx.x,
+    suffix_stream_body<G, 4, (G > 4 ? 1 : kTokDepth), F32, F32, false>(a, (CK_LDS char *)smem_raw, blockIdx.x, threadIdx.x,
                                                                 WgBarrier{});
 }
 static_assert(SfxLds<5, 4>::kBytes <= 80 * 1024, "two stand-alone workgroups per CU up to 5 heads");
@@ -909,7 +914,7 @@ __global__ __launch_bounds__(kMaxGroup * 32) void suffix_fixup_kernel(const int3
         }
         return;
     }
-    const ChunkMap cm{W, a.chunks, a.split};
+    const ChunkMap cm{W, chunks_used(W, batch, a.chunks, a.split_few), 0};
     const int ca = cm.owner(beg);
     const int cb = cm.owner(end - 1);
     if (ca == cb) return;  // written by the stream kernel
@@ -956,10 +961,10 @@ struct EpilogueArgs {
     int num_heads;
     int kv_heads;  // kv head groups, as in SuffixArgs
     int chunks;
-    int split;
+    int split_few;  // as in SuffixArgs
 };
 
-template <int G>
+template <int G, bool PAIRS>
 __global__ __launch_bounds__(kMaxGroup * 32) void cascade_epilogue_kernel(const int32_t *cw, const float *s1o, const float *s1lse,
                                                                          int64_t rows, int kv_heads, int nb, int num_heads,
                                                                          int b0, int splits, EpilogueArgs e) {
@@ -993,7 +998,8 @@ __global__ __launch_bounds__(kMaxGroup * 32) void cascade_epilogue_kernel(const 
     float l2 = -INFINITY;
     float4 o2 = make_float4(0.f, 0.f, 0.f, 0.f);
     if (end > beg) {
-        const ChunkMap cm{W, e.chunks, e.split};
+        const ChunkMap cm = PAIRS ? ChunkMap{W, e.chunks, e.split_few}
+                                  : ChunkMap{W, chunks_used(W, nb, e.chunks, e.split_few), 0};
         const int ca = cm.owner(beg);
         const int cb = cm.owner(end - 1);
         if (ca == cb) {
@@ -1124,7 +1130,7 @@ __global__ __launch_bounds__(512) void cascade_fused_kernel(s1::Stage1Args s1a, 
         constexpr int kRoleRot = 3;
         const int g = ((int)blockIdx.x + kRoleRot) % sa.kv_heads, j = (int)blockIdx.x / sa.kv_heads;
         // the streaming waves scan the lengths; the stage-1 waves reuse that scan
-        suffix_stream_body<G, 4, kTokDepth, false, (G > 4), FusedSfx<G>>(
+        suffix_stream_body<G, 4, kTokDepth, false, (G > 4), true, FusedSfx<G>>(
             sa, smem + (role ? 0 : kFusedS1Lds), (2 * j + role) * sa.kv_heads + g, threadIdx.x & 255, bar, bars + 4,
             role ? smem + kFusedS1Lds : nullptr);
     }
@@ -1136,9 +1142,9 @@ int64_t ceil_div(int64_t x, int64_t y) { return (x + y - 1) / y; }
 // split of the heads into kv head groups
 int64_t group_parts(int64_t num_heads, int64_t chunks) { return num_heads * chunks * 2; }
 
-template <int G>
+template <int G, bool PAIRS>
 void launch_epilogue(const EpilogueArgs &e, unsigned grid, hipStream_t st) {
-    hipLaunchKernelGGL(cascade_epilogue_kernel<G>, dim3(grid), dim3(32 * G), 0, st, e.cw, e.s1.o, e.s1.lse, e.s1.rows,
+    hipLaunchKernelGGL((cascade_epilogue_kernel<G, PAIRS>), dim3(grid), dim3(32 * G), 0, st, e.cw, e.s1.o, e.s1.lse, e.s1.rows,
                        e.kv_heads, e.nb, e.num_heads, (int)e.b0, e.s1.splits, e);
 }
 
@@ -1149,12 +1155,12 @@ int launch_fused(const s1::Stage1Args &s1a, int64_t n1, const SuffixArgs &a, con
     constexpr int kLds = fused_lds_bytes<G>();
     int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(&cascade_fused_kernel<G>), kLds, lds_set);
     if (rc != CK_OK) return rc;
-    const int64_t n2 = (int64_t)a.kv_heads * (a.chunks / 2);  // chunk pairs (a.split > 0)
+    const int64_t n2 = (int64_t)a.kv_heads * (a.chunks / 2);  // chunk pairs (PAIRS)
     const int64_t grid = n1 > n2 ? n1 : n2;
     hipLaunchKernelGGL(cascade_fused_kernel<G>, dim3((unsigned)grid), dim3(512), kLds, st, s1a, (int)n1, a, (int)n2);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return static_cast<int>(e);
-    launch_epilogue<G>(epi, (unsigned)(a.batch * a.kv_heads), st);
+    launch_epilogue<G, true>(epi, (unsigned)(a.batch * a.kv_heads), st);
     CK_RETURN_LAUNCH();
 }
 
@@ -1170,7 +1176,7 @@ int launch_suffix(const SuffixArgs &a, bool fixup, const EpilogueArgs *epi, hipS
     if (fixup)
         hipLaunchKernelGGL((suffix_fixup_kernel<G, F32>), dim3((unsigned)(a.batch * a.kv_heads)), dim3(32 * G), 0, st,
                            (const int32_t *)a.cw_out, a.kv_heads, a.batch, a);
-    if (epi) launch_epilogue<G>(*epi, (unsigned)(a.batch * a.kv_heads), st);
+    if (epi) launch_epilogue<G, false>(*epi, (unsigned)(a.batch * a.kv_heads), st);
     CK_RETURN_LAUNCH();
 }
 
@@ -1212,22 +1218,23 @@ int64_t suffix_group_batch(int64_t kv_cap) {
 //   (suffix_stream_kernel), and a second generation pays the start-up again
 //   (64 / 8 heads, 64 suffixes of mean 512: 42.5 us with 512 workgroups, 36.3 with
 //   256; 256 suffixes 115 / 109; 4 of mean 64 27.7 / 10.8).
-// * Up to 5 heads, one per CU for long sequences, at most one per chunk (two at 5
-//   heads): half the partials and start-ups (two / one per CU: 40 / 8 heads, 24
-//   requests of 4096 80.8 / 74.3 us, 64 suffixes of mean 512 37.5 / 36.1; 32 / 8
-//   heads, 16 of mean 512 17.2 / 16.4, 64 36.9 / 37.0). Two per CU otherwise: with
-//   many short sequences per chunk the closes bound it (256 of mean 64: 25.4 / 30.7).
+// * Up to 5 heads the grid holds two per CU, and the kernels use half of them once
+//   sequences hold 5 windows in the mean: half the partials and start-ups (512 / 256
+//   chunks over the groups at 6 windows a sequence: 40 / 8 heads, 16 sequences 1.17, 64
+//   1.18, 256 1.11 times the time; at 20 windows 1.05, 1.07, 1.03; 8 requests of 4096 on 8 /
+//   2 heads 1.21). Below, the closes bound it and the second workgroup hides them (64
+//   of 3 windows 0.96, 256 0.83; 4 windows 0.94, 0.90). Where the groups do not divide
+//   256 to 15/16 (71 of one head: 3 chunks on 213 CUs 59.1 us, 7 47.5) they keep all.
 // * A sequence of n windows spans chunks / batch chunks; its fold takes a memory
 //   round trip per 8 (about 0.15 us a chunk) and a chunk's windows about 0.5 us
 //   each: sqrt(cap / 8) chunks per sequence balance the two (8 / 1 heads, 7 requests
 //   of 4096: 26.2 us over 512 chunks, 13.8 over 112, 15.6 over 56).
-int64_t suffix_default_chunks(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap) {
+SuffixChunks suffix_default_chunks(int64_t batch, int64_t num_heads, int64_t kv_heads, int64_t kv_cap) {
     const int64_t groups = kv_heads * suffix_sub_groups(num_heads, kv_heads);
-    const int64_t g = num_heads / groups;
-    const bool one = g > 5 || (kv_cap >= 1024 && batch <= (g > 4 ? 2 : 1) * 256 / groups);
     const int64_t per_seq = std::max<int64_t>(8, (int64_t)std::sqrt((double)kv_cap / 8));
-    const int64_t p = std::min((one ? 256 : 512) / groups, batch * per_seq);
-    return p > 0 ? p : 1;
+    auto upto = [&](int64_t grid) { return std::max<int64_t>(1, std::min(grid / groups, batch * per_seq)); };
+    const int64_t most = upto(num_heads / groups > 5 ? 256 : 512), few = upto(256);
+    return SuffixChunks{most, 256 / groups * groups >= 240 ? few : most};
 }
 
 // The chunk count the plan reports, whatever the batch: two workgroups per CU. A call
@@ -1250,13 +1257,13 @@ int64_t suffix_group_ws_bytes(int64_t nb, int64_t num_heads, int64_t kv_heads, i
 
 int suffix_launch_group(const void *q, const void *k, const void *v, const int32_t *block_table, int64_t bt_cols,
                         const int64_t *kv_seqlens, int64_t b0, int64_t nb, int64_t num_heads, int64_t kv_heads,
-                        int64_t num_blocks, int64_t kv_layout, float scale, int64_t kv_cap, int64_t chunks,
+                        int64_t num_blocks, int64_t kv_layout, float scale, int64_t kv_cap, SuffixChunks chunks,
                         void *out, float *lse, void *group_ws, const Stage1Result *cascade, void *final_out,
                         float *final_lse, hipStream_t stream, const s1::Stage1Args *fused, int64_t fused_units,
                         bool f32_out) {
     const int64_t sub = suffix_sub_groups(num_heads, kv_heads);
     const int64_t G = num_heads / kv_heads / sub;  // query heads per workgroup
-    const int64_t parts = group_parts(num_heads, chunks);
+    const int64_t parts = group_parts(num_heads, chunks.most);
     SuffixArgs a;
     a.q = static_cast<const uint16_t *>(q) + b0 * num_heads * kD;
     a.k = static_cast<const uint16_t *>(k);
@@ -1278,8 +1285,8 @@ int suffix_launch_group(const void *q, const void *k, const void *v, const int32
     a.kv_heads = (int)(kv_heads * sub);
     a.kv_sub = (int)sub;
     a.kv_cap = (int)kv_cap;
-    a.chunks = (int)chunks;
-    a.split = fused && cascade ? fused_split(G) : 0;
+    a.chunks = (int)chunks.most;
+    a.split_few = fused && cascade ? fused_split(G) : (int)chunks.few;
     a.scale_log2 = scale * kLog2e;
     EpilogueArgs e;
     if (cascade) {
@@ -1295,8 +1302,8 @@ int suffix_launch_group(const void *q, const void *k, const void *v, const int32
         e.nb = (int)nb;
         e.num_heads = (int)num_heads;
         e.kv_heads = a.kv_heads;
-        e.chunks = (int)chunks;
-        e.split = a.split;
+        e.chunks = a.chunks;
+        e.split_few = a.split_few;
     }
     if (fused && cascade) {
         switch (G) {
@@ -1369,14 +1376,14 @@ extern "C" int ck_suffix_decode(const void *q, const void *k, const void *v, con
     if (!aligned_to(q, 16) || !aligned_to(k, 16) || !aligned_to(v, 16) || !aligned_to(out, 8) ||
         !aligned_to(lse, 4) || !aligned_to(workspace, 16))
         return CK_E_INVALID_ARG;
-    const int64_t chunks = num_splits > 0 && num_splits != suffix_plan_chunks(num_heads, kv_heads)
-                               ? num_splits
-                               : suffix_default_chunks(batch, num_heads, kv_heads, kv_cap);
-    if (kv_heads * suffix_sub_groups(num_heads, kv_heads) * chunks > 0x7FFFFFFF || chunks > (1 << 20))
+    const SuffixChunks chunks = num_splits > 0 && num_splits != suffix_plan_chunks(num_heads, kv_heads)
+                                    ? SuffixChunks{num_splits, num_splits}
+                                    : suffix_default_chunks(batch, num_heads, kv_heads, kv_cap);
+    if (kv_heads * suffix_sub_groups(num_heads, kv_heads) * chunks.most > 0x7FFFFFFF || chunks.most > (1 << 20))
         return CK_E_INVALID_ARG;
     const int64_t per_launch = suffix_group_batch(kv_cap);
     const int64_t nbmax = batch < per_launch ? batch : per_launch;
-    if (workspace == nullptr || workspace_bytes < suffix_group_ws_bytes(nbmax, num_heads, kv_heads, chunks))
+    if (workspace == nullptr || workspace_bytes < suffix_group_ws_bytes(nbmax, num_heads, kv_heads, chunks.most))
         return CK_E_WORKSPACE;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     for (int64_t b0 = 0; b0 < batch; b0 += per_launch) {
