@@ -49,7 +49,12 @@ int64_t align_up(int64_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
 // The fused kernel (stage-1 units and suffix chunks side by side) pays off while
 // stage-1 is no larger than the suffix side can hide; a prefix whose MFMA work
 // (kv heads x query rows of a kv head x prefix tokens) exceeds this runs the
-// kernels one after another, stage-1 with all its waves.
+// kernels one after another, stage-1 with all its waves. Fused / serial, us, suffixes of
+// mean 512, work 2^25.5, 2^26, 2^26.5, 2^27: 64 / 32 heads 73 / 81, 83 / 89, 102 / 104,
+// 135 / 125; 128 / 64 94 / 106, 99 / 113, 119 / 127, 142 / 139; 64 / 40 75 / 79, 93 / 96, 119
+// / 119, 154 / 142; 32 / 64 64 / 64, 82 / 83, 102 / 99, 129 / 116. Of mean 128 the two
+// meet half a power earlier. Not everywhere: 32 / 40 (160 rows in two 128-row units)
+// 82 / 71 at 2^25.5, 256 / 40 157 / 198 at 2^26.5.
 constexpr int64_t kFusedMaxS1Work = (int64_t)1 << 26;
 constexpr int64_t kFusedUnits = 256;  // stage-1 units of the fused kernel (one per CU)
 

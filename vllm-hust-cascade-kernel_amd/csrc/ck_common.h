@@ -8,6 +8,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "../../include/cascade_kernels.h"
 
@@ -22,6 +23,20 @@ constexpr int kWave = 64;
 constexpr int kNumXcd = 8;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
+
+// Calls f(std::integral_constant<int, I>{}) for I = 0 .. N - 1 (unrolled, I usable
+// as a compile-time index).
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for_from(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for_from<I + 1, N>(f);
+    }
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f) {
+    static_for_from<0, N>(f);
+}
 
 // ---- bf16 <-> fp32 -----------------------------------------------------------
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }

@@ -49,8 +49,6 @@
 //   staged global -> registers -> LDS.
 // * Tiles are ordered M-fastest and XCD-aware so the workgroups sharing a
 //   weight slice run on the same XCD and hit its L2.
-#include <type_traits>
-
 #include "ck_common.h"
 
 namespace ck {
@@ -64,18 +62,6 @@ constexpr int kThreads = 512;
 constexpr int kRowBytes = kBK * 2;                // 128 B per staged row
 constexpr int kTileBytes = (kBM + kBW) * kRowBytes;  // 64 KB per stage
 constexpr int kChunksPerThread = (kBM + kBW) * (kBK / 8) / kThreads;  // 8
-
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for_from(F &&f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for_from<I + 1, N>(f);
-    }
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F &&f) {
-    static_for_from<0, N>(f);
-}
 
 struct GemmArgs {
     const uint16_t *a;

@@ -64,7 +64,6 @@
 //   kernel folds (it also writes O = 0, LSE = -inf for empty suffixes).
 #include <algorithm>
 #include <cmath>
-#include <type_traits>
 
 #include "ck_common.h"
 #include "chunk_map.h"
@@ -76,20 +75,6 @@ static __device__ unsigned int g_wait_giveups;
 
 namespace ck {
 namespace {
-
-// Calls f(std::integral_constant<int, I>{}) for I = 0 .. N - 1 (unrolled, I usable
-// as a compile-time index).
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for_from(F &&f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for_from<I + 1, N>(f);
-    }
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F &&f) {
-    static_for_from<0, N>(f);
-}
 
 constexpr int kD = 128;
 constexpr int kPage = 128;
@@ -106,11 +91,13 @@ constexpr int kRsrcFlags = 0x00020000;  // buffer descriptor word 3 for gfx9 raw
 // above 4 heads (1 measured faster than 2 and 3).
 constexpr int kTokDepth = 2;
 // Share of each fused workgroup's suffix windows that its streaming waves take
-// (in 1/256); the stage-1 waves take the rest after their stage-1 unit. A batch has
-// more stage-1 rows per suffix byte the more heads share a kv head, so the share
-// is larger above 4 heads per group: 64 / 40 heads on 8192 tokens 53.7 us at 208,
-// 52.6 at 224; 47 / 64 on 6037 42.3, 41.5; 100 / 8 on 8000 30.0, 28.4; 110 / 64 on
-// 2000 44.2, 45.0. 64 / 32 on 8192: 51.3, 51.1 (the same within the runs).
+// (in 1/256); the stage-1 waves take the rest after their stage-1 unit. What decides is
+// a unit's tiles against the workgroup's windows, and no fixed share suits all: 208 /
+// 224, us, 64 / 40 heads on 8192 tokens 54.6 / 52.1, 47 / 40 on 6037 39.0 / 36.8, 64 / 48
+// on 8192 56.5 / 54.7, 100 / 64 on 8000 84.7 / 83.4; short prefixes the other way: 200 / 40
+// on 1000 47.7 / 49.3, 256 / 64 on 2048 133.8 / 136.8. Above 4 heads per group 224 gains
+// up to 5% and costs up to 3%; up to 4 heads 208 is ahead where it matters most (64 /
+// 32 on 8192 46.4 / 48.2; 100 / 32 on 8000 58.5 / 56.8, most others within 1%).
 constexpr int fused_split(int64_t group) { return group > 4 ? 224 : 208; }
 static_assert(fused_split(8) >= 128 && fused_split(8) < 256 && fused_split(4) >= 128, "ChunkMap assumes a share in [1/2, 1)");
 
@@ -392,8 +379,8 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     const char *kbase = reinterpret_cast<const char *>(a.k) + (int64_t)gk * a.head_off * 2;
     const char *vbase = reinterpret_cast<const char *>(a.v) + (int64_t)gk * a.head_off * 2;
     const int64_t pgb = a.page_stride * 2;
-    const uint32_t pg32 = (uint32_t)pgb, win32 = win_bytes, tok32 = (uint32_t)tokb;  // token-major addressing
-    // token-major body: lane (mg, mn); its K rows (token 8 wid + mn, 16 bytes at
+    const uint32_t pg32 = (uint32_t)pgb, win32 = win_bytes, tok32 = (uint32_t)tokb;
+    // lane (mg, mn): its K rows (token 8 wid + mn, 16 bytes at
     // 64 s + 16 mg for step s; rows 8-15 read nothing), its V bytes (lane (t, c):
     // token t, bytes 16 c and 128 + 16 c, at koff) in the wave's LDS slot, read
     // back transposed (tile T at + 32 T), and the addend of its scores (-inf: a
@@ -438,7 +425,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         return TokWin{(int64_t)off, page < 0 ? 0 : (int)(tab_tv(ey) * tok32)};
     };
 
-    // token-major: a window's K rows as the 4 A fragments of its score MFMAs
+    // a window's K rows as the 4 A fragments of its score MFMAs
     auto issue_kfrag = [&](const TokWin &w, u32x4 *kf) __attribute__((always_inline)) {
         const __amdgpu_buffer_rsrc_t r =
             __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(kbase + w.off), (short)0, w.range, kRsrcFlags);
@@ -447,7 +434,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
             kf[s4] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(kfoff + 64 * s4), 0, 0));
     };
 
-    // token-major: a window's V rows (lane (t, c): token t, bytes 16 c and 128 + 16 c),
+    // a window's V rows (lane (t, c): token t, bytes 16 c and 128 + 16 c),
     // issued after the values of the window whose ring slot they reuse
     auto issue_v = [&](const TokWin &w, u32x4 &x0, u32x4 &x1) __attribute__((always_inline)) {
         const __amdgpu_buffer_rsrc_t r =
@@ -535,7 +522,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
         }
     };
 
-    // Token-major: the state of a new segment, set at the start and by every close
+    // The state of a new segment, set at the start and by every close
     // (a segment opens at the chunk's first window or right after the previous
     // segment's close).
     auto reset_seg = [&]() __attribute__((always_inline)) {
@@ -584,8 +571,8 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
     };
 
     i32x2 enext = i32x2{-1, 0};  // the table entry of the next window to issue
-    int eypend = 0;  // packed table fields of window n - 1 (token-major)
-    // Token-major values of the pending window: its V rows (lane (t, c) holds 32
+    int eypend = 0;  // packed table fields of window n - 1
+    // Values of the pending window: its V rows (lane (t, c) holds 32
     // bytes of token t) into the wave's LDS slot, back as the V^T fragments of the 8
     // dim tiles, then O^T += V^T P^T over the terms of P. The slot is written and read
     // by this wave only, whose LDS operations run in issue order.
@@ -604,7 +591,7 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
                     __builtin_bit_cast(s16x4, vtf[T]), __builtin_bit_cast(s16x4, uint2{pb[i][0], pb[i][1]}), oacc[T], 0,
                     0, 0);
     };
-    // Token-major window step, pipelined by one window: step n issues the K rows of
+    // Window step, pipelined by one window: step n issues the K rows of
     // window n + D, computes the scores of window n and the values of window n - 1
     // (its P kept from the step before, its V rows still in their ring slot) -- two
     // independent chains in one basic block, so each fills the other's latencies --
@@ -808,21 +795,21 @@ __device__ __forceinline__ void suffix_stream_body(const SuffixArgs &a, CK_LDS c
             }
         });
         drain_tok(np);
-            // the phase's merged results out, by every wave of the role: each merge
-            // is done once every wave is past its last close
-            bar.sync();
-            const int nseg = qslot;  // segments closed in this phase (the same in every wave)
-            for (int i = tid; i < nseg * G * 32; i += kThr) {
-                const int e = i / (G * 32), u = i % (G * 32);
-                const int h = u >> 5, d4 = u & 31;
-                write_result(sb[e], h, d4, *reinterpret_cast<const CK_LDS f32x4 *>(so + (e * G + h) * kD + 4 * d4),
-                             sl[e * G + h]);
-            }
+        // the phase's merged results out, by every wave of the role: each merge
+        // is done once every wave is past its last close
+        bar.sync();
+        const int nseg = qslot;  // segments closed in this phase (the same in every wave)
+        for (int i = tid; i < nseg * G * 32; i += kThr) {
+            const int e = i / (G * 32), u = i % (G * 32);
+            const int h = u >> 5, d4 = u & 31;
+            write_result(sb[e], h, d4, *reinterpret_cast<const CK_LDS f32x4 *>(so + (e * G + h) * kD + 4 * d4),
+                         sl[e * G + h]);
+        }
         p0 = p1;
     }
 }
 
-// The stand-alone stream kernel: the token-major body on the matrix cores (the
+// The stand-alone stream kernel: the stream body (the
 // fused kernel's streaming body) on 4 waves and at most 256 registers; two
 // workgroups fit a CU up to 5 query heads per group (64 KB of LDS each at 4, 74 KB at
 // 5), one above (103 KB at 8 heads).
