@@ -72,8 +72,9 @@ def test_swiglu_short_k_ring(K, I):
     full-width tile's five-part ring keeps the weights two tiles ahead), K = 96 and
     160 run 32-deep stages (3 and 5 tiles). The ring's prologue and last iterations
     repeat the last tile into parts nothing reads again; the result must not see
-    them. M = 40 leaves 216 activation rows of the m-tile past M."""
-    M = 40
+    them. M = 150 (above the decode-sized kernels) leaves 106 activation rows of the
+    m-tile past M."""
+    M = 150
     a16, b16 = _inputs(M, K, I, seed=K)
     d, _ = torch.ops.npu.f3_gateup_epilogue(torch_bf16(a16, DEV), torch_bf16(b16, DEV), None, None, 1)
     rows = None if I <= 128 else np.random.default_rng(K).choice(M, 8, replace=False)
@@ -101,8 +102,8 @@ def test_full_width_tile_two_m_tiles(mode):
 @pytest.mark.parametrize("K", [80, 144, 4112])
 def test_register_staged_kernel_k_not_multiple_of_32(K, M, mode):
     """K % 16 == 0 but K % 32 != 0 (inside the reference's domain, f3_floor.cpp:64-80)
-    takes the register-staged kernel (the DMA ring steps K by 32 and the decode-sized
-    kernel needs K % 256 == 0): SwiGLU (mode 1) and the gate window with C (mode 0)."""
+    takes the register-staged kernel (the DMA ring steps K by 32, the decode-sized
+    kernels by 128 and 256): SwiGLU (mode 1) and the gate window with C (mode 0)."""
     I = 256 if M < 300 else 128
     a16, b16 = _inputs(M, K, I, seed=500 + K + M + mode)
     a, b = bits_to_f32(a16), bits_to_f32(b16)
@@ -166,9 +167,9 @@ def test_swiglu_m4096_sampled_rows():
 @pytest.mark.parametrize("M,K", [(1, 256), (2, 1024), (16, 512), (17, 256), (31, 512), (32, 768), (33, 512),
                                  (8, 320)])
 def test_decode_sized_m(M, K):
-    """M <= 32 with K % 256 == 0 takes a decode-sized kernel (four K quarters per
-    workgroup, partial sums folded in LDS; one 16-row activation block up to
-    M = 16, two above); M = 33 and K = 320 take the DMA ring.
+    """At I = 256 and M <= 32, K = 256 (and K = 512 up to M = 16) takes the kernel with a K
+    quarter per wave (one 16-row activation block up to M = 16, two above), the rest
+    the one with the activations in LDS; K = 320 takes the DMA ring.
     Every path must meet the same bound."""
     I = 256
     a16, b16 = _inputs(M, K, I, seed=100 + M)
@@ -179,7 +180,7 @@ def test_decode_sized_m(M, K):
 @pytest.mark.parametrize("M", [7, 20])
 @pytest.mark.parametrize("mode", [0, 2, 4, 5, 7, 8])
 def test_decode_sized_window_modes(mode, M):
-    """The decode-sized kernel with one 16-row activation block (M <= 16) and two."""
+    """The decode-sized kernels: a K quarter per wave (M = 7), activations in LDS (M = 20)."""
     K, I = 768, 384
     a16, b16 = _inputs(M, K, I, seed=200 + mode)
     a, b = bits_to_f32(a16), bits_to_f32(b16)
@@ -206,12 +207,12 @@ def test_decode_sized_inplace_d_and_same_c_as_dma_path():
     ws2 = torch.empty_like(ws)
     d0, _ = torch.ops.npu.f3_gateup_epilogue(a, b, ws2, ws2[:, :I], 0)
     assert d0.stride(0) == 2 * I and torch.equal(ws2, ws)
-    # the same rows inside a 40-row call (DMA ring): each result is within half a
+    # the same rows inside a 132-row call (DMA ring): each result is within half a
     # bf16 ulp plus the fp32 summation bound of the exact product, so the two differ
     # by at most one ulp plus twice that bound
-    a40 = torch.cat([a, a, a, a[:4]], 0).contiguous()
-    _, ws40 = torch.ops.npu.f3_gateup_epilogue(a40, b, None, None, 2)
-    diff = (ws40[:M].float() - ws.float()).abs().cpu().numpy()
+    a132 = a.repeat(11, 1).contiguous()
+    _, ws132 = torch.ops.npu.f3_gateup_epilogue(a132, b, None, None, 2)
+    diff = (ws132[:M].float() - ws.float()).abs().cpu().numpy()
     ulp = np.maximum(np.abs(bf16_to_np(ws)), 1e-30) * 2.0 ** -7
     af, bf = bits_to_f32(a16).astype(np.float64), bits_to_f32(b16).astype(np.float64)
     acc_bound = (K - 1) * 2.0 ** -24 * (np.abs(af) @ np.abs(bf).T)
@@ -314,11 +315,13 @@ def test_rejections_and_abi():
                                            None) == -1
 
 
-# The decode-sized kernel (M <= 128, K % 128 == 0): 16-row activation blocks 2 / 4 / 6 /
-# 8 and their edges, 1 to 9 steps of 128 K per K group (rings of 3 and 2 that never
+# The decode-sized kernel with the activations in LDS: 16-row activation blocks 2 / 4 / 6
+# / 8 and their edges, 1 to 9 steps of 128 K per K group (rings of 3 and 2 that never
 # fill, wrap and end on every slot), and 4 / 2 / 1 K groups (I <= 4096, <= 8192,
-# above; K must be a multiple of 512 / 256 / 128). M = 129 takes the DMA ring.
+# above; K must be a multiple of 512 / 256 / 128; one group at more than 64 rows
+# only from 160 or 205 workgroups on). M = 129 takes the DMA ring.
 @pytest.mark.parametrize("M,K,I", [
+    (65, 512, 10368), (96, 640, 10368), (97, 896, 13184), (128, 1152, 13184), (16, 896, 8320),
     (1, 128, 128), (32, 512, 256), (33, 512, 128), (64, 1024, 4096), (64, 1536, 128), (65, 512, 256),
     (17, 256, 128), (64, 768, 128), (96, 256, 128), (97, 1280, 256), (128, 2304, 128),
     (33, 1024, 8192), (128, 512, 8192), (32, 256, 8320), (64, 384, 8320), (65, 512, 8320), (96, 640, 8320),

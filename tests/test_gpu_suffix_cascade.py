@@ -169,7 +169,7 @@ CASCADE_CFGS = [
     (10, 6, 2, 512, "geo512"),       # G = 3, 2 and 1 with suffixes: the fused matrix-core body's padding heads
     (4, 4, 2, 384, "with_empty"),
     (9, 8, 8, 256, "geo512"),
-    (8, 14, 2, 512, "geo512"),       # G = 7: the fused kernel's dims-major streaming waves
+    (8, 14, 2, 512, "geo512"),       # G = 7: the fused kernel's 4-segment, one-slot layout
 ]
 CASCADE_IDS = ["config1_b8_h8", "b16_h32_geo", "empty_suffix", "gqa8_long_cut", "empty_prefix", "all_suffix_empty",
                "gqa16_long_cut", "gqa3_geo", "gqa2_with_empty", "mha_geo", "gqa7_geo"]
