@@ -151,7 +151,7 @@ int ck_fa_fp32_stage1_decode(const void *q, const void *k, const void *v, const 
 
 /* ============================================================================
  * Per-sequence paged decode attention over each sequence's own suffix
- * (one query token per sequence, GQA; P at fp32 precision).
+ * (one query token per sequence, GQA; P as two bf16 terms, within 2^-16 of fp32 P).
  *   q            bf16 [batch, num_heads, 128]
  *   k, v         bf16 paged pool in layout kv_layout: CK_KV_NHD
  *                [num_blocks, 128, kv_heads, 128] or CK_KV_BNSD
@@ -161,11 +161,11 @@ int ck_fa_fp32_stage1_decode(const void *q, const void *k, const void *v, const 
  *   lse          fp32 [batch * num_heads] (compact); a sequence with kv length 0
  *                gets out = 0 and lse = -inf (an empty suffix)
  *   kv_cap       upper bound of kv_seqlens(b), <= bt_cols * 128
- *   num_splits   workgroups per kv head group that share the list of 64-token
- *                windows (<= 0 or the plan's count: as many as suit the batch
- *                and kv_cap, at most the plan's); the plan sizes the workspace
- *                for it. A GQA group of
- *                more than 8 query heads per kv head is split into the fewest
+ *   num_splits   workgroups per kv head group that share the list of 32-token
+ *                windows; <= 0 or the plan's own count: as many as suit the
+ *                batch and the lengths, at most the plan's (any other count is
+ *                taken as it is). The plan sizes the workspace for its count. A
+ *                GQA group of more than 8 query heads per kv head is split into the fewest
  *                equal groups of at most 8, each streamed as its own kv head
  *                group (the K/V pages are then read once per group).
  * Same softmax arithmetic as ck_fa_fp32_stage1 (fp32 accumulation).
@@ -197,7 +197,8 @@ int ck_suffix_decode(const void *q, const void *k, const void *v, const int32_t 
  *   lse_out           fp32 [batch * num_heads]: the merged log-sum-exp
  *   prefix_cap / suffix_cap  bounds of the kv lengths, <= bt_cols * 128
  * Arithmetic: stage-1 as ck_fa_fp32_stage1 (bf16 P into the PV product),
- * suffix as ck_suffix_decode (fp32 P), merge as ck_lse_merge with lse_out;
+ * suffix as ck_suffix_decode (in the fused kernel above 4 query heads per kv
+ * head group P holds fp32, as three bf16 terms), merge as ck_lse_merge with lse_out;
  * the stage-1 split partials and cut-suffix partials are folded in fp32
  * without an intermediate bf16 or fp32 output pass.
  * Replaces the composition fa_fp32_stage1 -> FIA v2 -> lse_merge of

@@ -73,9 +73,9 @@ __global__ __launch_bounds__(kWW * 64) void stage1_wide_kernel(Stage1Args a) {
 }
 
 // 128-row m-tiles: the whole-row body on two sets of 4 waves that take the two
-// 64-token tiles of each page. A lone wave per SIMD spends three quarters of a tile
-// waiting on its own chain (LDS reads, row max, exp), so the second set's work fits
-// beside the first's. One set / two: 64 queries of 32 / 8 heads on 8192 tokens 22.3 /
+// 64-token tiles of each page. A lone wave per SIMD waits on its own chain
+// (LDS reads, row max, exp) between its MFMAs, and the second set's work fits beside
+// the first's. One set / two: 64 queries of 32 / 8 heads on 8192 tokens 22.3 /
 // 21.5 us; 200 of 64 / 8 on 1500 36.9 / 33.0; 24 requests of 2 x 40 / 8 on up to 4000
 // 88.4 / 78; 20 of 8 / 1 on 20000 22.6 / 20.6; 64 requests of 2 on 200 21.4 / 20.7.
 __global__ __launch_bounds__(512) void stage1_pair_kernel(Stage1Args a) {

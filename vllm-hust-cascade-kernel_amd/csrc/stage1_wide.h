@@ -69,8 +69,7 @@ constexpr int kTBytes = kTTok * kD * 2;              // 16 KB of K (or V) per ti
 // HALVES = 2 (the 128-row stand-alone kernel): two sets of NW waves share the rows;
 // each step takes one page, set h its 64-token tile h into a ring of its own, in
 // lockstep on the one barrier, and the two softmax states meet in LDS at the end.
-// Two waves per SIMD then hide each other's LDS, DMA and softmax latencies, which
-// are three quarters of a lone wave's time per tile.
+// Two waves per SIMD then hide each other's LDS, DMA and softmax latencies.
 constexpr int kWW = 8;
 constexpr int kWSlots = 4;
 constexpr int kWStage = 2 * kTBytes;  // K + V of one tile (32 KB)

@@ -9,8 +9,8 @@
 // yields O = 0, LSE = -inf, which the merge treats as weight 0.
 //
 // Arithmetic: S = q k^T * scale in fp32, online softmax in the log2 domain,
-// P at fp32 precision (the matrix-core body feeds P as two bf16 terms whose
-// sum is P within 2^-16) and fp32 accumulation, O = acc / l, LSE = ln(l) + max.
+// P as two bf16 terms whose sum is P within 2^-16, or as three that hold fp32 P (the
+// fused cascade above 4 heads per group, stage 1's decode form), fp32 accumulation, O = acc / l, LSE = ln(l) + max.
 //
 // MI355X design: HBM-bound streaming with a persistent, balanced grid and few
 // instructions per byte (at 8 TB/s a CU receives about 15 bytes per cycle; a
