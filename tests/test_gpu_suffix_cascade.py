@@ -559,3 +559,24 @@ def test_serial_cascade_chunks_in_use_by_mean_length(short):
         err = np.abs(got[b:b + 1] - Od)
         assert np.all(err <= 2e-3 + 2.0 ** -8 * np.abs(Od)), (b, err.max())
         assert np.abs(lse.reshape(B, H)[b] - Ld[0]).max() <= 1e-4 * max(1.0, np.abs(Ld[0]).max())
+
+
+# Fewer windows than chunks in the fused kernel: a window per chunk, on the last workgroups.
+# One window, pairs and odd counts, sequences of one and of several windows, empty ones,
+# with and without stage-1 units on the same workgroups.
+@pytest.mark.parametrize("B,H,KVH,P", [(1, 32, 8, 1024), (2, 40, 8, 128), (3, 32, 8, 1024), (3, 8, 1, 2048),
+                                       (5, 64, 8, 5120), (30, 32, 8, 8192)])
+def test_fused_few_windows(B, H, KVH, P, no_wait_giveups):
+    suf = np.array([32, 1, 20, 0, 100] + [33] * 25)[:B].astype(np.int64)
+    q16, k16, v16, bt_pre, bt_suf, suf = _cascade_inputs(B, H, KVH, P, suf, seed=B)
+    q, k, v = (torch_bf16(x, DEV) for x in (q16, k16, v16))
+    got, lse = _cascade_run(True, B, P, q, k, v, bt_pre, bt_suf, suf)
+    qf, kf, vf = bits_to_f32(q16), bits_to_f32(k16), bits_to_f32(v16)
+    kp, vp = A.gather_kv(kf, vf, bt_pre[0], P)
+    for b in range(min(B, 7)):
+        ks, vs = A.gather_kv(kf, vf, bt_suf[b], int(suf[b]))
+        Od, Ld = A.dense(qf[b:b + 1], A.expand_heads(np.concatenate([kp, ks]), H),
+                         A.expand_heads(np.concatenate([vp, vs]), H))
+        err = np.abs(got[b:b + 1] - Od)
+        assert np.all(err <= 2e-3 + 2.0 ** -8 * np.abs(Od)), (b, err.max())
+        assert (np.abs(lse.reshape(B, H)[b] - Ld[0]) / np.maximum(np.abs(Ld[0]), 1.0)).max() <= 1e-4

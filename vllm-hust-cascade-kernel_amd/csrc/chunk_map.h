@@ -28,14 +28,15 @@ CK_HD int64_t div_nonneg(int64_t x, int64_t d) { return (int64_t)((double)x / (d
 // even): chunks 2j and 2j + 1 share the j-th of P / 2 equal ranges, the first
 // taking split / 256 of it, in [1/2, 1) (the fused cascade kernel's two roles on
 // one CU).
-// With fewer windows than chunks the first chunks take one window each (split > 0:
-// the first pairs two, one per chunk; an odd last window joins the last pair, and
-// a single window is the first pair's second chunk's), in closed form without a
-// division. So no chunk between two that hold windows is ever empty, and folding a
-// cut sequence's partials tests nothing (ranges spread over all P chunks left
-// empty ones inside a sequence there, and testing them, two chunk bounds per chunk
-// of dependent double divisions, cost the cascade epilogue half of its 13.3 us at 8
-// sequences on a 2048-token prefix).
+// With fewer windows than chunks each takes a chunk of its own, the first ones (split >
+// 0: the last ones), in closed form without a division. So no chunk between two that hold
+// windows is ever empty, and folding a cut sequence's partials tests nothing (ranges
+// spread over all P chunks left empty ones inside a sequence there, and testing them, two
+// chunk bounds per chunk of dependent double divisions, cost the cascade epilogue half
+// of its 13.3 us at 8 sequences on a 2048-token prefix). The last chunks in the fused
+// kernel, whose stage-1 units are on its first workgroups: a window there waits for a
+// unit (1 sequence of 64 tokens, 32 / 8 heads, on a 1024-token prefix: 15.7 us on the
+// first pairs, 12.1 here; 3 of 32 tokens 16.1 and 12.1).
 struct ChunkMap {
     int64_t W;
     int P;
@@ -43,10 +44,7 @@ struct ChunkMap {
     CK_HD int64_t lo(int c) const {
         if (W < P) {
             if (split == 0) return c < W ? c : W;
-            const int h = few_pairs();
-            if (c >= 2 * h) return W;
-            const int a = c & ~1;
-            return (c & 1) == 0 ? a : a + (((a == 2 * h - 2 ? (int)W - a : 2) * split) >> 8);
+            return c > P - W ? c - (P - W) : 0;
         }
         if (split == 0) return div_nonneg((int64_t)c * W, P);
         const int h = P >> 1, j = c >> 1;
@@ -56,19 +54,11 @@ struct ChunkMap {
     }
     // the chunk that owns window p < W
     CK_HD int owner(int64_t p) const {
-        int j;
-        if (W < P) {
-            if (split == 0) return (int)p;
-            j = (int)p >> 1;
-            if (j > few_pairs() - 1) j = few_pairs() - 1;
-        } else {
-            if (split == 0) return (int)div_nonneg((p + 1) * P - 1, W);
-            j = (int)div_nonneg((p + 1) * (P >> 1) - 1, W);
-        }
+        if (W < P) return (int)(split == 0 ? p : p + P - W);
+        if (split == 0) return (int)div_nonneg((p + 1) * P - 1, W);
+        const int j = (int)div_nonneg((p + 1) * (P >> 1) - 1, W);
         return 2 * j + (p >= lo(2 * j + 1) ? 1 : 0);
     }
-    // W < P, split > 0: pairs that hold windows
-    CK_HD int few_pairs() const { return ((int)W >> 1) > 1 ? (int)W >> 1 : 1; }
 };
 
 // Chunks in use of a grid that has room for `most`: `few` once the sequences hold 5
