@@ -24,7 +24,7 @@
 //   (stage1_wide.h):
 //   - stage1_pair_kernel (m-tile of 128 rows): two sets of 4 waves, one 64-token
 //     tile of each page per set, a 2-slot K/V ring each; (O, m, l) of the sets are
-//     merged in LDS. Splits of a single page run stage1_narrow_kernel: one set and a
+//     merged in LDS. Splits of up to two pages run stage1_narrow_kernel: one set and a
 //     3-slot ring, the body the fused cascade kernel runs as its stage-1 role.
 //   - stage1_wide_kernel (m-tile of 256 rows, when a request has more than 128
 //     rows per kv head and enough kv to fill the chip): 8 waves, two per SIMD;
@@ -83,8 +83,10 @@ __global__ __launch_bounds__(512) void stage1_pair_kernel(Stage1Args a) {
     stage1_wide_body<4, 2, 2>(a, (CK_LDS char *)smem_raw, blockIdx.x, gridDim.x, threadIdx.x, WgBarrier{});
 }
 
-// 128-row m-tiles over splits of one page: one set of 4 waves (two sets take one tile
-// each and then merge, which costs more than the second tile)
+// 128-row m-tiles over splits of one or two pages: one set of 4 waves (two sets take a
+// tile or two each and then merge, which costs about what it saves: one request on 147
+// tokens 9.6 us with one set, 10.4 with two, 64 of 2 on up to 200 21 and 22, 8 of 2 on up
+// to 200 10.9 and 10.2)
 constexpr int kNLds = wide_lds_bytes<3>();
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void stage1_narrow_kernel(Stage1Args a) {
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -318,7 +320,7 @@ int ck::stage1_launch(const void *q, const void *k, const void *v, const int32_t
         rc = ensure_dynamic_lds(reinterpret_cast<const void *>(&stage1_wide_kernel), kWLds, lds_set_w);
         if (rc != CK_OK) return rc;
         hipLaunchKernelGGL(stage1_wide_kernel, dim3((unsigned)grid), dim3(kWW * 64), kWLds, s, a);
-    } else if (p.split_len > kPage) {
+    } else if (p.split_len > 2 * kPage) {
         static std::atomic<uint64_t> lds_set2{0};
         rc = ensure_dynamic_lds(reinterpret_cast<const void *>(&stage1_pair_kernel), kPairLds, lds_set2);
         if (rc != CK_OK) return rc;
