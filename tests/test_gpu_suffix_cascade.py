@@ -519,7 +519,7 @@ def test_fused_above_4_heads_full_precision_p(H, KVH):
     assert excess <= 2.0 ** -19
 
 
-# The stream uses half of its grid's chunks once sequences hold 5 windows of 32 tokens in the
+# The stream uses half of its grid's chunks once sequences hold 12 windows of 32 tokens in the
 # mean (up to 5 heads per group): one window below and at that mean, under a table as
 # wide as the lengths and a far wider one, in the stand-alone op and (a serial
 # cascade: prefix work above 2^26) with the cascade's epilogue folding the cut sequences.
@@ -529,11 +529,11 @@ def test_fused_above_4_heads_full_precision_p(H, KVH):
 def test_chunks_in_use_by_mean_length(H, KVH, short, cols):
     B = 24
     rng = np.random.default_rng(H + short)
-    wins = rng.integers(1, 10, size=B)
-    wins[0] = 20
-    while wins.sum() != 5 * B - short:
+    wins = rng.integers(1, 24, size=B)
+    wins[0] = 32
+    while wins.sum() != 12 * B - short:
         b = rng.integers(1, B)
-        wins[b] = max(0, wins[b] + np.sign(5 * B - short - wins.sum()))
+        wins[b] = min(32, max(0, wins[b] + np.sign(12 * B - short - wins.sum())))
     kvs = np.where(wins > 0, 32 * wins - rng.integers(0, 32, size=B), 0)
     inp = paged_inputs(B, kvs, H, KVH, seed=H, permute=True, block_cols=cols)
     out, lse = _suffix(inp)
@@ -543,9 +543,9 @@ def test_chunks_in_use_by_mean_length(H, KVH, short, cols):
 @pytest.mark.parametrize("short", [1, 0])
 def test_serial_cascade_chunks_in_use_by_mean_length(short):
     B, H, KVH, P = 65, 32, 8, 32384
-    suf = np.full(B, 160 - 3)
-    suf[7], suf[11:15] = 160 - 3 + 256 - 32 * short, 77  # 5 B windows (less one)
-    assert ((suf + 31) // 32).sum() == 5 * B - short and B * H * P > 1 << 26
+    suf = np.full(B, 384 - 3)
+    suf[7], suf[11:15], suf[20] = 381 + 288 - 32 * short, 309, 349  # 12 B windows, or one less
+    assert ((suf + 31) // 32).sum() == 12 * B - short and B * H * P > 1 << 26
     q16, k16, v16, bt_pre, bt_suf, suf = _cascade_inputs(B, H, KVH, P, suf, seed=short)
     bt_suf = np.concatenate([bt_suf, np.zeros((B, 30), np.int32)], axis=1)
     q, k, v = (torch_bf16(x, DEV) for x in (q16, k16, v16))

@@ -61,9 +61,9 @@ struct ChunkMap {
     }
 };
 
-// Chunks in use of a grid that has room for `most`: `few` once the sequences hold 5
+// Chunks in use of a grid that has room for `most`: `few` once the sequences hold 12
 // windows in the mean. The lengths decide, not the bound that the host knows (a table
 // as wide as the longest context says nothing of them).
-CK_HD int chunks_used(int64_t W, int batch, int most, int few) { return W >= (int64_t)5 * batch ? few : most; }
+CK_HD int chunks_used(int64_t W, int batch, int most, int few) { return W >= (int64_t)12 * batch ? few : most; }
 
 }  // namespace ck

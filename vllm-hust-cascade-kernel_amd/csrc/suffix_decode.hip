@@ -1206,12 +1206,13 @@ int64_t suffix_group_batch(int64_t kv_cap) {
 //   (64 / 8 heads, 64 suffixes of mean 512: 42.5 us with 512 workgroups, 36.3 with
 //   256; 256 suffixes 115 / 109; 4 of mean 64 27.7 / 10.8).
 // * Up to 5 heads the grid holds two per CU, and the kernels use half of them once
-//   sequences hold 5 windows in the mean: half the partials and start-ups (512 / 256
-//   chunks over the groups at 6 windows a sequence: 40 / 8 heads, 16 sequences 1.17, 64
-//   1.18, 256 1.11 times the time; at 20 windows 1.05, 1.07, 1.03; 8 requests of 4096 on 8 /
-//   2 heads 1.21). Below, the closes bound it and the second workgroup hides them (64
-//   of 3 windows 0.96, 256 0.83; 4 windows 0.94, 0.90). Where the groups do not divide
-//   256 to 15/16 (71 of one head: 3 chunks on 213 CUs 59.1 us, 7 47.5) they keep all.
+//   sequences hold 12 windows in the mean: half the partials and start-ups (512 / 256
+//   chunks over the groups at 16 windows a sequence: 40 / 8 heads, 16 sequences 1.09, 64
+//   1.03, 256 1.05 times the time; at 20 windows 1.05, 1.07, 1.03; 8 requests of 4096 on 8 /
+//   2 heads 1.21). Below, the closes bound it and the second workgroup hides them (8
+//   windows: 130 of 40 / 8 0.96; 4: 64 0.94, 256 0.90; 2: 256 0.83). A chunk of more than
+//   one phase's 8 segments costs a phase more, and where the groups do not divide 256 to
+//   15/16 CUs idle (71 of one head: 3 chunks on 213 CUs 59.1 us, 7 47.5): all, then.
 // * A sequence of n windows spans chunks / batch chunks; its fold takes a memory
 //   round trip per 8 (about 0.15 us a chunk) and a chunk's windows about 0.5 us
 //   each: sqrt(cap / 8) chunks per sequence balance the two (8 / 1 heads, 7 requests
@@ -1221,7 +1222,7 @@ SuffixChunks suffix_default_chunks(int64_t batch, int64_t num_heads, int64_t kv_
     const int64_t per_seq = std::max<int64_t>(8, (int64_t)std::sqrt((double)kv_cap / 8));
     auto upto = [&](int64_t grid) { return std::max<int64_t>(1, std::min(grid / groups, batch * per_seq)); };
     const int64_t most = upto(num_heads / groups > 5 ? 256 : 512), few = upto(256);
-    return SuffixChunks{most, 256 / groups * groups >= 240 ? few : most};
+    return SuffixChunks{most, 256 / groups * groups >= 240 && batch <= kQSlots * few ? few : most};
 }
 
 // The chunk count the plan reports, whatever the batch: two workgroups per CU. A call
